@@ -26,10 +26,14 @@ typedef struct fsx_hip_args {
     const double *A_re, *A_im, *B_re, *B_im;   /* [3][qnum][(L+1)^2] */
     const double *a;                           /* [6*qnum] */
     const double *cint;                        /* [6][qnum]: constant parts, x2 for mixed pairs */
-    const double *dW;                          /* [nbeta][(L+1)(2L+1)^2] */
+    /* Wigner-d values per beta and l in the operand order of the rotation's 16x16x4
+     * matrix products: [row / 16][m1 / 4][m1 % 4][row % 16], rows l - m and columns
+     * l + m1 of 0 .. 2l, zeros past them */
+    const double *dW;
     const double *dsymb;                       /* (L+1)^3 (2L+1) */
     const double *tw_a, *tw_g;                 /* [nalpha][2], [ngamma][2]: cos, -sin of 2 pi k/N */
     double mult, peak, c1_lo, c1_hi, c2_lo, c2_hi;
+    double pi;                                 /* of the beta grid */
     const int64_t *poses;
     int n;
     double *score, *c1, *c2, *cross;

@@ -21,10 +21,12 @@
  * the contraction kernels use FMA.
  */
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <pthread.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <type_traits>
 
 #include "../fsx_internal.h"
 #include "../fsx_pose.h"
@@ -35,9 +37,7 @@
 #include "../fsx_lbfgsb.h"
 #include "../fsx_lb2.h"
 
-#define FSX_CROSS_THREADS 256
 #define FSX_WAVE 64
-#define FSX_NXCD 8
 /* counters of the fit kernel: evaluations, capped fits, loop iterations summed
  * over wavefronts, of those wavefront-wide ones, the longest wavefront's */
 #define FSX_TALLY_N 5
@@ -45,6 +45,7 @@
 struct cplx { double re, im; };
 struct cplx32 { float re, im; };   /* element of the mixed-precision (FP32) tables */
 typedef double fsx_v4d __attribute__((ext_vector_type(4)));   /* FP64 MFMA 16x16x4 result */
+#include "fsx_cross.h"
 
 /* ---------------------------------------------------------------------- */
 /* device helpers */
@@ -129,141 +130,64 @@ __global__ void k_sbessel_batch(const double *x, int n, int P, double *out)
     out[i] = dev_sbessel((int)(i % P), x[i / P]);
 }
 
-/* Packed translation blocks: per (z, q) the rows (|m|, l) for l >= |m| in
- * order of |m| then l, each holding l1 = |m|..L.  Row (am, l) starts at
- * S(K) - S(K - am) + (l - am)(K - am), S(n) = n(n+1)(2n+1)/6; the block has
- * S(K) entries. */
-__host__ __device__ __forceinline__ int tpk_sq(int n) { return n * (n + 1) * (2 * n + 1) / 6; }
-/* Entry stride (in elements) of the cross-term kernel's staged ligand rows.
- * FP32 tables keep the 3G values of an entry together; when 3G * 8 bytes is
- * a multiple of 32 (G = 4: 96 bytes) two elements of padding make it an odd
- * multiple of 16, so that the entries that one wavefront reads at a U step
- * fall on twice as many LDS bank offsets.  FP64 tables are [G][3][nc]. */
-template <typename E, int G>
-__host__ __device__ constexpr int cross_sb()
-{
-    return sizeof(E) == 8 ? ((3 * G) % 4 == 0 ? 3 * G + 2 : 3 * G) : 3 * G;
-}
-/* LDS bytes of the cross-term kernel's translation block (Tn values of type F),
- * rounded up to 8 so that the pose records after it stay aligned */
-template <typename F>
-__host__ __device__ __forceinline__ size_t cross_tst_bytes(int Tn)
-{
-    return ((size_t)Tn * sizeof(F) + 7) & ~(size_t)7;
-}
-__host__ __device__ __forceinline__ int tpk_row(int am, int l, int K)
-{
-    return tpk_sq(K) - tpk_sq(K - am) + (l - am) * (K - am);
-}
-
 /* T^{|m|}_{l l1}(q z) (fftsaxs.c:182-243), computed from (min(l,l1), max(l,l1))
- * so the mirrored entries are bitwise equal, as in fftsaxs.c:213-238.  One
- * thread per (z, q, packed entry) in the packed layout, per |m| block
- * [l1][l]: element (am, l, l1) at tpk_row(am, am, K) + (l1 - am) * (K - am) +
- * (l - am), the order in which the cross-term kernel's U step reads them
- * (consecutive l, consecutive threads). */
-template <typename E>
-__global__ void k_tmat(decltype(E::re) *T, const double *bes, const double *ds, int znum, int Q, int L)
+ * so the mirrored entries are bitwise equal, as in fftsaxs.c:213-238, in the
+ * operand order of the cross-term kernel's matrix products: per block and tile
+ * of FSX_CROSS_TILE l, steps of 4 l1, FP32 [l1][l], FP64 [l1][l % 4][l / 4] (what a
+ * lane of four 4x4x4 products takes side by side; split: 4 even, then 4 odd
+ * l1), with zeros where l
+ * or l1 exceeds L.  tb: the number of blocks, then per block 2 |m| + split
+ * and its first value, then the table size
+ * Tn.  Only p of the parity of l + l1
+ * contribute (the 3j symbol (l p l1; 0 0 0) vanishes exactly otherwise), so
+ * T = i^(l1 - l) tau with tau real, and the sum runs over those p: stored is
+ * tau = i^(l - l1) T.
+ * One thread forms one table entry for FSX_TMAT_ZQ (z, q): its d-symbols, whose
+ * addresses are scattered over the wavefront, are then read once for all of
+ * them, not once for each. */
+#define FSX_TMAT_ZQ 8
+template <typename F>
+__global__ void __launch_bounds__(256)
+k_tmat(F *T, const double *bes, const double *ds, const int *tb, int nzq, int L, int Tn)
 {
 #pragma clang fp contract(off)
-    const int K = L + 1, N = 2 * L + 1, Tn = tpk_sq(K);
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)znum * Q * Tn) return;
-    const int r = (int)(i % Tn);
-    const long zq = i / Tn;
-    /* |m| block of packed entry r: block am holds (K - am)^2 entries from
-     * tpk_row(am, am, K) */
-    int m = 0;
-    while (m < L && r >= tpk_row(m + 1, m + 1, K)) m++;
-    const int off = r - tpk_row(m, m, K), w = K - m;
-    const int l1 = m + off / w, l = m + off % w;
-    int lo = l < l1 ? l : l1, hi = l < l1 ? l1 : l;
-    const double *b = bes + zq * N;
+    const int K = L + 1, N = 2 * L + 1;
+    const int nbx = (Tn + 255) / 256, by = blockIdx.x / nbx;
+    const int r = (blockIdx.x - by * nbx) * 256 + threadIdx.x;
+    if (r >= Tn) return;
+    int k = 0;
+    while (k + 1 < tb[0] && r >= tb[2 * k + 4]) k++;
+    const int m = tb[2 * k + 1] >> 1, split = tb[2 * k + 1] & 1, Km = K - m;
+    constexpr int TL = FSX_CROSS_TILE;
+    const int nks = cross_steps(Km, split), sv = cross_tstep(split), o = r - tb[2 * k + 2];
+    const int st = o / sv, i = o % sv, ks = st % nks;
+    const int l = m + TL * (st / nks) + (sizeof(F) == 4 ? i & 15 : (i >> 2 & 3) + 4 * (i & 3));
+    const int j = i / TL;   /* l1 of the step: four, or four even and four odd ones */
+    const int l1 = m + (split ? 2 * (4 * ks + (j & 3)) + (j >> 2) : 4 * ks + j);
+    const bool in = l <= L && l1 <= L;
+    const int lo = in ? (l < l1 ? l : l1) : m, hi = in ? (l < l1 ? l1 : l) : m;
     const double *d = ds + ((long)(lo * (lo + 1) + m) * K + hi) * N;
-    double sg = (m % 2) ? -1.0 : 1.0;
-    const double ipr[4] = {1.0, 0.0, -1.0, 0.0}, ipi[4] = {0.0, 1.0, 0.0, -1.0};
-    double re = 0.0, im = 0.0;
-    for (int p = hi - lo; p <= lo + hi; p++) {
-        double v = sg * d[p] * b[p];
-        re += ipr[p % 4] * v;
-        im += ipi[p % 4] * v;
-    }
-    /* only p of the parity of l + l1 contribute (the 3j symbol (l p l1; 0 0 0)
-     * vanishes exactly otherwise), so T = i^(l1 - l) tau with tau real, and
-     * the other part is an exact zero: stored is tau = i^(l - l1) T */
-    const int ph = ((l - l1) % 4 + 4) % 4;
-    const double tau = ph == 0 ? re : ph == 1 ? -im : ph == 2 ? -re : im;
-    T[zq * Tn + r] = (decltype(E::re))tau;
-}
-
-__device__ __forceinline__ double wave_sum(double v)
-{
+    const double sg = (m % 2) ? -1.0 : 1.0;
+    const int zq0 = by * FSX_TMAT_ZQ;
+    double t[FSX_TMAT_ZQ];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, FSX_WAVE);
-    return v;
+    for (int k = 0; k < FSX_TMAT_ZQ; k++) t[k] = 0.0;
+    if (in)
+        for (int p = hi - lo; p <= lo + hi; p += 2) {
+            const double dv = sg * d[p];
+            const bool neg = (p & 2) != 0;
+#pragma unroll
+            for (int k = 0; k < FSX_TMAT_ZQ; k++) {
+                const double v = dv * bes[(size_t)min(zq0 + k, nzq - 1) * N + p];
+                t[k] += neg ? -v : v;
+            }
+        }
+    /* the sum is T's real part for even l - l1, its imaginary part for odd */
+    const int ph = ((l - l1) % 4 + 4) % 4;
+#pragma unroll
+    for (int k = 0; k < FSX_TMAT_ZQ; k++)
+        if (zq0 + k < nzq) T[(size_t)(zq0 + k) * Tn + r] = (F)(ph == 1 || ph == 2 ? -t[k] : t[k]);
 }
-
-/* Cross-lane steps of the 64-lane transpose-reduce, on the two 32-bit halves
- * of a double.  v_permlane32_swap exchanges lanes 32..63 of its first operand
- * with lanes 0..31 of its second, v_permlane16_swap the odd 16-lane rows of
- * the first with the even rows of the second, so that the sum of the two
- * results is, in every lane, its own slot's value plus the partner lane's
- * value of the same slot (lanes below the split keep slot a, lanes above it
- * slot b). */
-__device__ __forceinline__ double tr_swap32(double a, double b)
-{
-    const unsigned long long ua = __builtin_bit_cast(unsigned long long, a);
-    const unsigned long long ub = __builtin_bit_cast(unsigned long long, b);
-    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)ua, (unsigned)ub, false, false);
-    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32),
-                                                     false, false);
-    const double r0 = __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]);
-    const double r1 = __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
-    return r0 + r1;
-}
-__device__ __forceinline__ double tr_swap16(double a, double b)
-{
-    const unsigned long long ua = __builtin_bit_cast(unsigned long long, a);
-    const unsigned long long ub = __builtin_bit_cast(unsigned long long, b);
-    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)ua, (unsigned)ub, false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32),
-                                                     false, false);
-    const double r0 = __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]);
-    const double r1 = __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
-    return r0 + r1;
-}
-__device__ __forceinline__ float tr_swap32(float a, float b)
-{
-    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a),
-                                                    __builtin_bit_cast(unsigned, b), false, false);
-    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
-}
-__device__ __forceinline__ float tr_swap16(float a, float b)
-{
-    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a),
-                                                    __builtin_bit_cast(unsigned, b), false, false);
-    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
-}
-/* a double moved between lanes by a DPP pattern (row_ror:8 = lane xor 8,
- * row_half_mirror = lane 7 - i in each group of 8, quad_perm) */
-template <int CTRL>
-__device__ __forceinline__ double dpp_mov(double v)
-{
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, 0xf, 0xf, false);
-    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, 0xf, 0xf, false);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-template <int CTRL>
-__device__ __forceinline__ float dpp_mov(float v)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
-                                                                 0xf, 0xf, false));
-}
-#define FSX_DPP_ROR8 0x128
-#define FSX_DPP_HMIRROR 0x141
-#define FSX_DPP_XOR1 0xB1
-#define FSX_DPP_XOR2 0x4E
 
 /* x mod n in [0, n) for |x| < 2^24, n >= 1: a float quotient estimate
  * (off by at most one) and one correction. */
@@ -281,8 +205,7 @@ __device__ __forceinline__ int mod_small(int x, int n, float inv_n)
  * k_rotate: out^X_{lm}(beta, gamma, q) = sum_{m1} d^l_{m m1}(beta) src~[q][X][l m1][gamma]
  * with one wavefront per (beta, q, X, entry) and the lanes over gamma, so the
  * Wigner-d value of a term is the same for the whole wavefront and the
- * source loads are contiguous.  Output layout per m-chunk c (entries e in
- * m-major order): out[coff[c] + ((q*nrows + beta*ng + gamma)*3 + X)*csize[c] + e - cstart[c]]. */
+ * source loads are contiguous. */
 __global__ void k_twiddle(cplx *dst, const double *src_re, const double *src_im,
                           const double *twg, int ng, int Q, int L, int conj_src)
 {
@@ -305,26 +228,91 @@ __global__ void k_twiddle(cplx *dst, const double *src_re, const double *src_im,
     dst[i] = v;
 }
 
+/* Where a rotated value goes.  Per m-chunk a row of the table (one q, beta,
+ * gamma) holds
+ *   ligand:   [l1, in steps of 4 per m][re, im][V, D, W], the order in which a
+ *             lane of the translation product reads its operands (a block that
+ *             is summed in both orders of l1 is there twice);
+ *   receptor: [V, D, W][slot][re, im], the slots across the lanes of the
+ *             pairing.  The m = 0 entries l = 2i and 2i + 1 of
+ *             conjugate-symmetric coefficients, whose turned values i^l R_l0
+ *             are real, are the two halves of slot i. */
+struct fsx_tabmap {
+    /* per entry: l, chunk, offset in the row, zero entries to add (ligand), and
+     * the two of a second place (offset -1: none); per chunk: row length */
+    const int *l, *pass, *off, *pad, *off2, *pad2, *rs;
+    const long *coff;                       /* per chunk: first value */
+    int lig, npk;                           /* ligand table; entries packed in halves */
+};
+
+/* one entry's place in the rows of a table: its values of row qrow go to d + qrow
+ * * rs */
+template <typename F>
+struct fsx_tabput {
+    F *d, *d2;          /* first row's place, the second one (NULL: none) */
+    size_t rs;
+    int pad, pad2, lig, half;
+    int ph;             /* power of i that turns the value */
+    __device__ __forceinline__ fsx_tabput(F *out, const fsx_tabmap &M, int e, int X, int lsgn)
+    {
+        const int c = M.pass[e], r = M.rs[c], o2 = M.lig ? M.off2[e] : -1;
+        F *b = out + M.coff[c] + (M.lig ? X : X * (r / 3));
+        rs = r;
+        d = b + M.off[e];
+        d2 = o2 >= 0 ? b + o2 : NULL;
+        pad = M.lig ? M.pad[e] : 0;
+        pad2 = M.lig ? M.pad2[e] : 0;
+        lig = M.lig;
+        half = e < M.npk;
+        ph = (lsgn > 0 ? M.l[e] : -M.l[e]) & 3;
+    }
+    __device__ __forceinline__ void put(size_t qrow, F x, F y) const
+    {
+        const F re = ph == 0 ? x : ph == 1 ? -y : ph == 2 ? -x : y;
+        const F im = ph == 0 ? y : ph == 1 ? x : ph == 2 ? -y : -x;
+        F *p = d + qrow * rs;
+        if (lig) {
+            p[0] = re;
+            p[3] = im;
+            for (int j = 1; j <= pad; j++) p[6 * j] = p[6 * j + 3] = 0;
+            if (d2) {
+                p = d2 + qrow * rs;
+                p[0] = re;
+                p[3] = im;
+                for (int j = 1; j <= pad2; j++) p[6 * j] = p[6 * j + 3] = 0;
+            }
+        } else {
+            /* a whole slot (at an even place) in one store */
+            struct alignas(2 * sizeof(F)) slot { F re, im; };
+            if (half) p[0] = re;
+            else *reinterpret_cast<slot *>(p) = {re, im};
+        }
+    }
+};
+
+/* Wigner-d tables, per beta [l][16 rows][4 m1][64]: row r = l - m (so the rows m
+ * >= 0 come first) and m1 + l in the order of a 16x16x4 product's first operand
+ * (value 16 (m1 % 4) + r % 16), zeros past 2l + 1; dw_base(l): first value of l */
+__host__ __device__ __forceinline__ int dw_steps(int l) { return (2 * l + 4) / 4; }
+__host__ __device__ __forceinline__ int dw_size(int l) { return (2 * l + 16) / 16 * dw_steps(l) * 64; }
+
 /* One block per (q, X, l, chunk of FSX_ROT_BC betas, gamma chunk of gc): the
  * 2l+1 source rows of l, gamma in the chunk, are staged in LDS
  * ([m1][gamma]) together with the blocks d^l_{m m1}(beta) of the chunk's
  * betas; the wavefronts then take (beta, pair of m) items and form
  * out^X_{lm}(beta, gamma) = sum_m1 d^l_{m m1}(beta) src_{l m1}(gamma), lanes
  * over gamma, m1 ascending.  The output goes to a staging table with rows
- * innermost, per chunk c [q][X][entry][row] at coff[c] (lanes store
- * consecutive rows); k_tab_transpose then writes the row-major table the
- * cross-term kernel reads. */
+ * innermost, [q][X][entry][row] (lanes store consecutive rows);
+ * k_tab_transpose then writes the table the cross-term kernel reads. */
 #define FSX_ROT_BC 2
 template <typename E>
 __global__ void __launch_bounds__(256)
-k_rotate(E *out, const cplx *srct, const double *dW, const int *ent, const long *coff,
-         int nbeta, int ng, int Q, int L, int gc, int mlo)
+k_rotate(E *out, const cplx *srct, const double *dW, const int *mstart, int nbeta, int ng,
+         int Q, int L, int gc, int mlo, int ne)
 {
 #pragma clang fp contract(fast)
     extern __shared__ cplx sR[];   /* [2l+1][gc], then FSX_ROT_BC blocks [2l+1][2l+1] of d */
-    const int K = L + 1, K2 = K * K, N = 2 * L + 1;
-    const int *ent_c = ent + 2 * K2, *ent_ec = ent + 3 * K2, *csize = ent + 4 * K2;
-    const int *mstart = ent + 5 * K2;
+    const int K = L + 1, K2 = K * K;
     const int nrows = nbeta * ng;
     const int lane = threadIdx.x % FSX_WAVE, wave = threadIdx.x / FSX_WAVE;
     const int nwave = blockDim.x / FSX_WAVE;
@@ -340,6 +328,11 @@ k_rotate(E *out, const cplx *srct, const double *dW, const int *ent, const long 
     /* output rows m = mb..l (all m, or m >= 0 for the half entry set) */
     const int w = 2 * l + 1, mb = mlo > -l ? mlo : -l, nm = l - mb + 1, ww = nm * w;
     double *sD = reinterpret_cast<double *>(sR + w * gc);
+    int dbase = 0, dsz = 0;
+    for (int k = 0; k <= L; k++) {
+        if (k < l) dbase += dw_size(k);
+        dsz += dw_size(k);
+    }
     const cplx *src = srct + (((long)q * 3 + X) * K2 + l * (l + 1) - l) * ng + g0;
     for (int i = threadIdx.x; i < w * gc; i += blockDim.x) {
         int m1 = i / gc, g = i - m1 * gc;
@@ -347,7 +340,9 @@ k_rotate(E *out, const cplx *srct, const double *dW, const int *ent, const long 
     }
     for (int i = threadIdx.x; i < nbh * ww; i += blockDim.x) {
         const int bb = i / ww, rem = i - bb * ww, mr = rem / w, k = rem - mr * w;
-        sD[i] = dW[(long)(b0 + bb) * K * N * N + ((long)l * N + (L + mb + mr)) * N + (L - l + k)];
+        const int row = l - mb - mr;
+        sD[i] = dW[(size_t)(b0 + bb) * dsz + dbase + (row / 16 * dw_steps(l) + k / 4) * 64 + k % 4 * 16 +
+                   row % 16];
     }
     __syncthreads();
     const int np = (nm + 1) / 2;   /* pairs of m */
@@ -361,9 +356,7 @@ k_rotate(E *out, const cplx *srct, const double *dW, const int *ent, const long 
             /* entry (l, m) in m-major order */
             const int m = mb + (two ? mi + u : mi);
             const int e = mstart[m + L] + (l - (m < 0 ? -m : m));
-            const int c = ent_c[e];
-            const long cs = csize[c];
-            o[u] = out + coff[c] + ((long)(q * 3 + X) * cs + ent_ec[e]) * nrows + (long)b * ng + g0;
+            o[u] = out + ((long)(q * 3 + X) * ne + e) * nrows + (long)b * ng + g0;
         }
         for (int gw = 0; gw < gn; gw += FSX_WAVE) {
             const int g = gw + lane;
@@ -390,13 +383,13 @@ k_rotate(E *out, const cplx *srct, const double *dW, const int *ent, const long 
     }
 }
 
-/* One chunk of a rotated table from the staging layout [q][X][entry][row]
- * to [q][row][X][entry] (cs entries), through a 64-entry x TR-row LDS tile
- * per block: loads run along rows, stores along entries. */
+/* A rotated table from the staging layout [q][X][entry][row] to its final one,
+ * each value turned by i^(lsgn l), through a 64-entry x TR-row LDS tile per
+ * block: loads run along rows, stores along entries. */
 template <typename E, int TR>
 __global__ void __launch_bounds__(256)
-k_tab_transpose(E *out, const E *tmp, int cs, int nrows, int nte, int ntr, int npk,
-                const int *lrot, int lsgn)
+k_tab_transpose(decltype(E::re) *out, const E *tmp, int ne, int nrows, int nte, int ntr,
+                const fsx_tabmap M, int lsgn)
 {
     __shared__ E tile[64][TR + 1];
     int bid = blockIdx.x;
@@ -406,29 +399,19 @@ k_tab_transpose(E *out, const E *tmp, int cs, int nrows, int nte, int ntr, int n
     const int qx = bid / nte;   /* q * 3 + X */
     const int X = qx % 3, q = qx / 3;
     const int e0 = te * 64, r0 = tr * TR;
-    const E *src = tmp + (long)qx * cs * nrows;
+    const E *src = tmp + (long)qx * ne * nrows;
     for (int k = threadIdx.x; k < 64 * TR; k += 256) {
         const int i = k / TR, j = k - (k / TR) * TR;
         const int e = e0 + i, r = r0 + j;
-        if (e < cs && r < nrows) tile[i][j] = src[(long)e * nrows + r];
+        if (e < ne && r < nrows) tile[i][j] = src[(long)e * nrows + r];
     }
     __syncthreads();
     for (int k = threadIdx.x; k < 64 * TR; k += 256) {
         const int j = k >> 6, i = k & 63;
         const int e = e0 + i, r = r0 + j;
-        if (e < cs && r < nrows) {
-            E *d = out + (((long)q * nrows + r) * 3 + X) * cs;
-            E v = tile[i][j];
-            if (lsgn != 0) {   /* times i^(lsgn l), l of the entry */
-                const int ph = (lsgn > 0 ? lrot[e] : -lrot[e]) & 3;
-                const decltype(v.re) a = v.re, b = v.im;
-                v.re = ph == 0 ? a : ph == 1 ? -b : ph == 2 ? -a : b;
-                v.im = ph == 0 ? b : ph == 1 ? a : ph == 2 ? -b : -a;
-            }
-            /* packed m = 0 pairs: i^l R_l0 is real for every l */
-            if (e >= 2 * npk) d[e - npk] = v;
-            else if (e & 1) d[e >> 1].im = v.re;
-            else d[e >> 1].re = v.re;
+        if (e < ne && r < nrows) {
+            const fsx_tabput<decltype(E::re)> P(out, M, e, X, lsgn);
+            P.put((size_t)q * nrows + r, tile[i][j].re, tile[i][j].im);
         }
     }
 }
@@ -442,102 +425,106 @@ k_tab_transpose(E *out, const E *tmp, int cs, int nrows, int nte, int ntr, int n
  * rows m = max(mlo, -l)..l, each block's m rows and 16 columns (8 gamma, real
  * and imaginary parts) a job of one wave.  The results go to an LDS tile of
  * the block's GT rows of the table, all entries; the tile is written out row
- * by row, turned by i^(lsgn l) and with the npk packed m = 0 slot pairs of
- * chunk 0, exactly as k_tab_transpose writes them. */
+ * by row, turned by i^(lsgn l), exactly as k_tab_transpose writes it. */
 template <typename E, int GT>
 __global__ void __launch_bounds__(256)
-k_rotate_mfma(E *out, const cplx *srct, const double *dW, const int *ent, const long *coff,
-              int nbeta, int ng, int Q, int L, int mlo, int ne, int npk, int lsgn)
+k_rotate_mfma(decltype(E::re) *out, const cplx *srct, const double *dW, const int *mstart,
+              const fsx_tabmap M, int nbeta, int ng, int Q, int L, int mlo, int ne, int lsgn)
 {
     extern __shared__ double smem_raw[];
     E *tile = reinterpret_cast<E *>(smem_raw);   /* [GT][ne] */
-    const int K = L + 1, K2 = K * K, N = 2 * L + 1;
-    const int *ent_l = ent, *ent_c = ent + 2 * K2, *ent_ec = ent + 3 * K2, *csize = ent + 4 * K2;
-    const int *mstart = ent + 5 * K2;
+    const int K = L + 1, K2 = K * K;
     const int nrows = nbeta * ng, ngt = (ng + GT - 1) / GT;
-    int r = blockIdx.x;
+    /* the three X of a tile eight blocks apart, on the same XCD: the ligand table
+     * has them side by side, and its L2 joins their parts of a line */
+    int r = blockIdx.x / 24 * 8 + blockIdx.x % 8;
+    const int X = blockIdx.x / 8 % 3;
+    if (r >= Q * nbeta * ngt) return;
     const int gt = r % ngt; r /= ngt;
-    const int b = r % nbeta; r /= nbeta;
-    const int X = r % 3;
-    const int q = r / 3;
+    const int b = r % nbeta;
+    const int q = r / nbeta;
     const int g0 = gt * GT;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int NT = GT / 8;   /* 16-column tiles: 8 gamma x (re, im) each */
-    const double *dWb = dW + (size_t)b * K * N * N;
+    constexpr int CH = 4;        /* steps of 4 m1 whose operands are loaded together */
+    int dsz = 0;
+    for (int l = 0; l <= L; l++) dsz += dw_size(l);
+    const double *dWb = dW + (size_t)b * dsz + lane;
     const cplx *srcq = srct + (size_t)(q * 3 + X) * K2 * ng;
-    /* jobs (l, m-tile, column tile), dealt to the waves in turn */
-    int j = 0;
-    for (int l = 0; l <= L; l++) {
-        const int mb = mlo > -l ? mlo : -l, nm = l - mb + 1, nmt = (nm + 15) / 16;
-        const int njob = nmt * NT;
-        for (int jj = 0; jj < njob; jj++, j++) {
-            if ((j & 3) != w) continue;
-            const int mt = jj / NT, nt = jj - mt * NT;
-            const int i = lane & 15, k = lane >> 4;
-            const int m = mb + mt * 16 + i;
-            const int gl = nt * 8 + (i >> 1), part = i & 1, g = g0 + gl;
-            const bool arow = m <= l, bcol = gl < GT && g < ng;
-            const double *drow = dWb + ((size_t)l * N + (L + (arow ? m : l))) * N + (L - l);
-            const double *scol = reinterpret_cast<const double *>(srcq + (size_t)l * l * ng +
-                                                                  (bcol ? g : g0)) + part;
-            fsx_v4d acc = {0.0, 0.0, 0.0, 0.0};
-            /* the job's operands of up to KS steps loaded together (one
-             * round trip), then its MFMAs; the rest step by step.  KS = 8
-             * (2l + 1 <= 32) for FP64 tables, whose LDS tile bounds the
-             * blocks per CU anyway; 4 for FP32 tables, which keep more
-             * blocks per CU with fewer registers (measured: the FP32 rotate
-             * stage 0.52 against 0.60 ms at L = 15) */
-            constexpr int KS = sizeof(E) == 8 ? 4 : 8;
-            const int nks = (2 * l + 1 + 3) / 4;
-            double av[KS], bv[KS];
+    const int i = lane & 15, k = lane >> 4;
+    /* jobs (l, m-tile, column tile), dealt to the waves in turn, each in chunks
+     * of CH steps; the operands of the next chunk (of this job or the next) are
+     * in flight during the products of the current one.  The loads are
+     * unconditional (past a job's end: values that meet a zero of the other
+     * operand or are not stored), so that the wait before a chunk's products
+     * leaves the next one's loads in flight. */
+    struct { int l, mt, nt, k0, d0; } J = {0, 0, 0, 0, 0};   /* d0: first Wigner-d value of l */
+    auto next_job = [&]() {
+        if (++J.nt < NT) return;
+        J.nt = 0;
+        const int mb = mlo > -J.l ? mlo : -J.l;
+        if (16 * ++J.mt < J.l - mb + 1) return;
+        J.mt = 0;
+        J.d0 += dw_size(J.l);
+        J.l++;
+    };
+    auto next = [&]() {
+        J.k0 += CH;
+        if (J.k0 < dw_steps(J.l)) return;
+        J.k0 = 0;
+        for (int u = 0; u < 4; u++) next_job();
+    };
+    double av[2][CH], bv[2][CH];
+    auto load = [&](double *a, double *bo) {
+        if (J.l > L) return;
+        const int g = min(g0 + J.nt * 8 + (i >> 1), ng - 1), nks = dw_steps(J.l);
+        const double *drow = dWb + J.d0 + J.mt * nks * 64;
+        const double *scol = reinterpret_cast<const double *>(srcq + (size_t)J.l * J.l * ng + g) + (i & 1);
 #pragma unroll
-            for (int st = 0; st < KS; st++) {
-                const int m1i = 4 * st + k;
-                const bool kin = st < nks && m1i <= 2 * l;
-                av[st] = arow && kin ? drow[m1i] : 0.0;
-                bv[st] = bcol && kin ? scol[(size_t)m1i * ng * 2] : 0.0;
-            }
+        for (int st = 0; st < CH; st++) {
+            a[st] = drow[64 * min(J.k0 + st, nks - 1)];
+            bo[st] = scol[(size_t)min(4 * (J.k0 + st) + k, 2 * J.l) * ng * 2];
+        }
+    };
+    for (int u = 0; u < w; u++) next_job();
+    fsx_v4d acc = {0.0, 0.0, 0.0, 0.0};
+    auto run = [&](const double *a, const double *bo, int l, int mt, int nt, int k0) {
+        const int nks = dw_steps(l);
+        if (k0 == 0) acc = (fsx_v4d){0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-            for (int st = 0; st < KS; st++)
-                if (st < nks) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[st], bv[st], acc, 0, 0, 0);
-            for (int kk = 4 * KS; kk < 2 * l + 1; kk += 4) {
-                const int m1i = kk + k;
-                const bool kin = m1i <= 2 * l;
-                const double a1 = arow && kin ? drow[m1i] : 0.0;
-                const double b1 = bcol && kin ? scol[(size_t)m1i * ng * 2] : 0.0;
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc, 0, 0, 0);
-            }
-            const int c = lane & 15;
-            const int gl2 = nt * 8 + (c >> 1), part2 = c & 1;
+        for (int st = 0; st < CH; st++)
+            if (k0 + st < nks) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[st], bo[st], acc, 0, 0, 0);
+        if (k0 + CH < nks) return;
+        const int mb = mlo > -l ? mlo : -l, gl = nt * 8 + (i >> 1), part = i & 1;
 #pragma unroll
-            for (int rr = 0; rr < 4; rr++) {
-                const int m2 = mb + mt * 16 + (lane >> 4) + 4 * rr;
-                if (m2 <= l && gl2 < GT) {
-                    const int e = mstart[m2 + L] + (l - (m2 < 0 ? -m2 : m2));
-                    decltype(E::re) *t = reinterpret_cast<decltype(E::re) *>(&tile[gl2 * ne + e]);
-                    t[part2] = (decltype(E::re))acc[rr];
-                }
+        for (int rr = 0; rr < 4; rr++) {
+            const int m = l - mt * 16 - k - 4 * rr;   /* rows by falling m */
+            if (m >= mb) {
+                const int e = mstart[m + L] + (l - (m < 0 ? -m : m));
+                reinterpret_cast<decltype(E::re) *>(&tile[gl * ne + e])[part] = (decltype(E::re))acc[rr];
             }
         }
+    };
+    load(av[0], bv[0]);
+    while (J.l <= L) {
+        auto P = J;
+        next();
+        load(av[1], bv[1]);
+        run(av[0], bv[0], P.l, P.mt, P.nt, P.k0);
+        if (J.l > L) break;
+        P = J;
+        next();
+        load(av[0], bv[0]);
+        run(av[1], bv[1], P.l, P.mt, P.nt, P.k0);
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < GT * ne; idx += blockDim.x) {
-        const int gl = idx / ne, e = idx - gl * ne, g = g0 + gl;
-        if (g >= ng) continue;
-        E v = tile[idx];
-        if (lsgn != 0) {   /* times i^(lsgn l), l of the entry */
-            const int ph = (lsgn > 0 ? ent_l[e] : -ent_l[e]) & 3;
-            const decltype(v.re) x = v.re, y = v.im;
-            v.re = ph == 0 ? x : ph == 1 ? -y : ph == 2 ? -x : y;
-            v.im = ph == 0 ? y : ph == 1 ? x : ph == 2 ? -y : -x;
-        }
-        const int c = ent_c[e], ec = ent_ec[e], cs = csize[c];
-        E *d = out + coff[c] + ((size_t)((size_t)q * nrows + b * ng + g) * 3 + X) * cs;
-        const int pk = c == 0 ? npk : 0;
-        /* packed m = 0 pairs: i^l R_l0 is real for every l */
-        if (ec >= 2 * pk) d[ec - pk] = v;
-        else if (ec & 1) d[ec >> 1].im = v.re;
-        else d[ec >> 1].re = v.re;
+    /* a thread takes an entry of all rows: its place is looked up once */
+    const int gn = ng - g0 < GT ? ng - g0 : GT;
+    for (int e = threadIdx.x; e < ne; e += blockDim.x) {
+        const fsx_tabput<decltype(E::re)> P(out, M, e, X, lsgn);
+        const size_t row = (size_t)q * nrows + b * ng + g0;
+#pragma unroll 4
+        for (int gl = 0; gl < gn; gl++) P.put(row + gl, tile[gl * ne + e].re, tile[gl * ne + e].im);
     }
 }
 
@@ -548,56 +535,158 @@ __global__ void k_fill_int(int *p, long n, int v)
     if (i < n) p[i] = v;
 }
 
-/* bucket key (z, beta2, gamma2) and the pose's receptor row / alpha index */
+/* The counters of a call in one launch: bucket counts and fills (nc values)
+ * and the record, bucket and unit counters zero, the fit queue at next0, the
+ * fit tallies zero. */
+__global__ void k_init(int *counts, long nc, int *tail, int *next, int next0,
+                       unsigned long long *tally)
+{
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nc) counts[i] = 0;
+    if (i < 3) tail[i] = 0;
+    if (i < FSX_TALLY_N) tally[i] = 0;
+    if (i == 0) *next = next0;
+}
+
+/* The mirror image of a rotated table row.  With d^l_{m,m1}(pi - beta) =
+ * (-1)^(l+m) d^l_{m,-m1}(beta) and coefficients with A_{l,-m} = (-1)^(l+m)
+ * conj(A_lm), the row of (pi - beta, gamma) is, in both tables and after their
+ * turns by i^l and i^-l,
+ *   R_lm(pi - beta, gamma) = (-1)^(l+m) conj(R_lm(beta, gamma + pi)),
+ * so that with an even gamma grid the tables need only beta <= pi / 2: half
+ * the rotations, and half the receptor rows of a q for an XCD's L2 to hold.
+ * A ligand row is mirrored as the translation reads it (cross_body).  A pose
+ * with a mirrored receptor row takes alpha2 negated (Re(w conj(R) U) = Re(conj(w)
+ * R conj(U))), the slots' signs (-1)^(l+m) with its twiddles (row 2 alpha2 + 1),
+ * and the products of the imaginary parts with the other sign. */
+__device__ __forceinline__ void fsx_mirror(int nbeta, int na, int ng, int *b1, int *g1, int *alpha)
+{
+    const int hb = (nbeta - 1) / 2, hg = ng / 2;
+    const bool m1 = *b1 > hb;
+    if (m1) {
+        *b1 = nbeta - 1 - *b1;
+        *g1 = *g1 >= hg ? *g1 - hg : *g1 + hg;
+        if (*alpha > 0) *alpha = na - *alpha;
+    }
+    *alpha = 2 * *alpha + m1;
+}
+
+/* bucket (beta2, z, gamma2) of each pose, its receptor row and twiddle
+ * row */
 __global__ void k_count(const long long *poses, int n, int znum, int nbeta, int na, int ng,
-                        int *keys, int2 *info, int *counts)
+                        int mirror, int *keys, int2 *info, int *counts)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     int row, alpha;
-    const int key = fsx_pose_key(poses[i], znum, nbeta, na, ng, &row, &alpha);
-    if (key >= 0) atomicAdd(&counts[key], 1);
+    int key = fsx_pose_key(poses[i], znum, nbeta, na, ng, &row, &alpha);
+    if (key >= 0) {
+        const int zb = key / ng, z = zb / nbeta;
+        const int b2 = zb - z * nbeta, g2 = key - zb * ng;
+        int b1 = row / ng, g1 = row - b1 * ng;
+        if (mirror) fsx_mirror(nbeta, na, ng, &b1, &g1, &alpha);
+        row = b1 * ng + g1;
+        key = (b2 * znum + z) * ng + g2;
+        atomicAdd(&counts[key], 1);
+    }
     keys[i] = key;
     info[i] = make_int2(row, alpha);
 }
 
-/* exclusive scan of counts[0..nk) into offs[0..nk]; offs[nk+1] = number of
- * non-empty buckets.  One block of 1024. */
-__global__ void k_scan(const int *counts, int nk, int *offs)
+/* First record of every bucket and the cross-term units, one wavefront per
+ * (beta2, z).  Units are cut greedily along gamma2: up to urows rows and
+ * FSX_UPOSES poses; a bucket of more poses takes several.  The wavefronts
+ * reserve their records and units with one atomic each (tail: records,
+ * non-empty buckets, units), so the order of the (beta2, z) groups is only
+ * approximately ascending; every pose's result is the same in any order.
+ * One launch, against a scan by a single block whose time grew with the
+ * number of buckets (828 us at 478,000 buckets). */
+__global__ void __launch_bounds__(256)
+k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int *offs, fsx_unit *units, int *tail)
 {
-    __shared__ int part[1024];
-    __shared__ int nz[1024];
-    int t = threadIdx.x;
-    int chunk = (nk + 1023) / 1024;
-    int b = t * chunk, e = b + chunk < nk ? b + chunk : nk;
-    int s = 0, z = 0;
-    for (int i = b; i < e; i++) {
-        s += counts[i];
-        z += counts[i] != 0;
+    const int zb = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (zb >= nzb) return;
+    const int *c = counts + (size_t)zb * ng, cap = FSX_UPOSES;
+    int total = 0, nz = 0, nu = 0, first = 0;
+    /* pass 0 counts the units, pass 1 writes them */
+    for (int pass = 0; pass < 2; pass++) {
+        int p = 0, un = 0, ur = 0, uc = 0;   /* records so far; open unit's poses and rows; units */
+        fsx_unit u;
+        u.b2 = zb / zn % nb;
+        u.z = zb % zn;
+        u.pad = 0;
+        for (int g0 = 0; g0 < ng; g0 += 64) {
+            const int v = g0 + lane < ng ? c[g0 + lane] : 0;
+            if (pass) {
+                /* exclusive scan over the 64 buckets */
+                int x = v;
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int y = __shfl_up(x, o);
+                    if (lane >= o) x += y;
+                }
+                if (g0 + lane < ng) offs[(size_t)zb * ng + g0 + lane] = total + p + x - v;
+            }
+            unsigned long long mask = __ballot(v > 0);
+            if (!pass) nz += __popcll(mask);
+            while (mask) {
+                const int b = __builtin_ctzll(mask);
+                mask &= mask - 1;
+                int left = __builtin_amdgcn_readlane(v, b);
+                while (left > 0) {
+                    /* close the open unit where the row does not fit in it */
+                    if (un > 0 && (ur == urows || un + left > cap)) {
+                        if (pass && lane == 0) {
+                            u.n = un;
+                            u.nrow = ur;
+                            units[first + uc] = u;
+                        }
+                        uc++;
+                        un = ur = 0;
+                    }
+                    const int k = left < cap - un ? left : cap - un;
+                    if (un == 0) u.p0 = total + p;
+#pragma unroll
+                    for (int r = 0; r < FSX_UROWS; r++)
+                        if (r == ur) {
+                            u.g2[r] = g0 + b;
+                            if (r % 4 == 0) u.cum[r / 4] = 0;
+                            u.cum[r / 4] |= (unsigned)un << r % 4 * 8;
+                        } else if (r > ur) {
+                            u.g2[r] = u.g2[0];
+                        }
+                    ur++;
+                    un += k;
+                    p += k;
+                    left -= k;
+                }
+            }
+        }
+        if (un > 0) {
+            if (pass && lane == 0) {
+                u.n = un;
+                u.nrow = ur;
+                units[first + uc] = u;
+            }
+            uc++;
+        }
+        if (!pass) {
+            int a = 0, b = 0;
+            if (lane == 0 && p > 0) {
+                a = atomicAdd(&tail[0], p);
+                atomicAdd(&tail[1], nz);
+                b = atomicAdd(&tail[2], uc);
+            }
+            total = __builtin_amdgcn_readlane(a, 0);
+            first = __builtin_amdgcn_readlane(b, 0);
+            nu = uc;
+        }
     }
-    part[t] = s;
-    nz[t] = z;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        int v = t >= off ? part[t - off] : 0;
-        int w = t >= off ? nz[t - off] : 0;
-        __syncthreads();
-        part[t] += v;
-        nz[t] += w;
-        __syncthreads();
-    }
-    int run = part[t] - s;
-    for (int i = b; i < e; i++) {
-        offs[i] = run;
-        run += counts[i];
-    }
-    if (t == 1023) {
-        offs[nk] = part[1023];
-        offs[nk + 1] = nz[1023];
-    }
+    (void)nu;
 }
 
-/* sorted pose records: x = input position, y = receptor row, z = alpha index */
+/* sorted pose records: x = input position, y = receptor row, z = alpha index,
+ * w = gamma2 */
 __global__ void k_scatter(const int *keys, const int2 *info, int n, int ng, const int *offs,
                           int *fill, int4 *recs)
 {
@@ -607,543 +696,7 @@ __global__ void k_scatter(const int *keys, const int2 *info, int n, int ng, cons
     if (k < 0) return;
     int p = offs[k] + atomicAdd(&fill[k], 1);
     int2 inf = info[i];
-    /* input position, receptor row, alpha2, gamma2 (key % ng) */
     recs[p] = make_int4(i, inf.x, inf.y, k % ng);
-}
-
-/* ---- per-pose cross terms, one m-chunk per launch --------------------------
- * Work tile = (q, beta2, G consecutive gamma2) with all z inside.  The G
- * ligand row chunks (3 * nc entries each) are staged in LDS once per tile;
- * the packed translation block of each (z, q) is staged once per z (TST;
- * read from global memory when it does not fit) and serves the G rows; each
- * wavefront prefetches the receptor row of its first pose before U is
- * formed.  Per z with requested poses in the tile's G buckets
- * (z, beta2, gamma2), which are adjacent in the bucket order:
- *   U^Y_e = sum_{l1 >= |m|} conj(T^{|m|}_{l l1}(q z)) B^Y_{(l1, m)}
- * (one entry e per thread, for each of the G rows), then per pose (one
- * wavefront, J entries per lane)
- *   2 Re sum_e e^{-i m a2} (R^X_e U^Y_e [+ R^Y_e U^X_e])
- * over the chunk's entries e = (l, m), stored (first chunk) or added into
- * acc[(s*Q + q)*6 + k]. */
-/* Workgroup barrier that orders LDS accesses only: unlike __syncthreads it
- * does not wait for the block's outstanding global stores (the cross-term
- * accumulator writes, which no other thread of the launch reads), so they
- * drain while the block goes on. */
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-#define FSX_CROSS_BLOCK 256
-#define FSX_CROSS_PB 64   /* poses per batch of the cross-term pose loop */
-/* s_waitcnt vmcnt(0) (expcnt and lgkmcnt left at their maxima) */
-#define FSX_WAITCNT_VM0 0x0F70
-/* FP32 tables: at most 128 VGPRs, four blocks of four wavefronts per CU
- * (five blocks of 96 VGPRs were slower: 8.1 against 5.9 ms at L = 15);
- * FP64 tables: the LDS of three blocks fills a CU, no register bound */
-template <int J, int TST, int G, typename E, int PW>
-__device__ __forceinline__ void
-cross_body(double *acc, const E *Rc, const E *Bc, const decltype(E::re) *T, const E *tw2,
-           const int *ent, int cstart, int nc, const int *counts, const int *offs,
-           const int4 *recs, long ntiles, int nrows, int Q, int L, int nbeta, int nx, int ng,
-           int zn, int first, int npk)
-{
-#pragma clang fp contract(fast)
-    typedef decltype(E::re) F;   /* arithmetic type of the contraction */
-    static_assert(G <= 8, "the tile row of a pose is kept in three bits of its record");
-    extern __shared__ double smem_raw[];
-    E *smem = reinterpret_cast<E *>(smem_raw);
-    /* ligand rows: FP32 tables [nc][SB] (the 3G values of one entry together,
-     * read as 16-byte pairs, then cross_sb's padding), FP64 tables [G][3][nc] */
-    constexpr bool BIL = sizeof(E) == 8;
-    E *sB = smem;
-    constexpr int SB = cross_sb<E, G>();   /* sB: [nc][SB] (BIL) or [G][3][nc] */
-    E *sU = smem + SB * nc;   /* [G][3][nc] */
-    F *sT = reinterpret_cast<F *>(sU + 3 * G * nc);   /* T block, [l1][l] per |m| as in T (TST) */
-    const int K = L + 1, K2 = K * K, N = 2 * L + 1, Tn = tpk_sq(K);
-    /* the current batch of up to FSX_CROSS_PB of the tile's poses: their
-     * (receptor row, 8 alpha2 + gamma2 row within the tile), read from LDS
-     * in the pose loop so that a pose
-     * waits for one global round trip (its receptor row), not two, and their
-     * six lane sums (type F), written to acc by the whole block after the
-     * batch, so that no store is in flight in the pose loop */
-    int2 *sP = reinterpret_cast<int2 *>(reinterpret_cast<char *>(sU + 3 * G * nc) +
-                                        (TST ? cross_tst_bytes<F>(Tn) : 0));
-    F *sO = reinterpret_cast<F *>(sP + FSX_CROSS_PB);
-    const int *ent_l = ent, *ent_m = ent + K2, *mstart = ent + 5 * K2;
-    const int tid = threadIdx.x, lane = tid & (FSX_WAVE - 1), wave = tid / FSX_WAVE;
-    const int nwave = FSX_CROSS_BLOCK / FSX_WAVE;
-    /* U items (entries ordered by decreasing row length K - |m|, so that
-     * the lanes of a wavefront run loops of nearly equal length).  The
-     * nsplit longest entries are split into the even and the odd steps of
-     * their l1 range (adjacent entries, whose LDS reads fall on different
-     * banks), run by lanes 2i and 2i + 1 and summed across the pair; every
-     * other entry takes one thread.  nsplit fills the block: with nc + nsplit
-     * items the longest loop is about half the longest row. */
-    const int *uperm = ent + 7 * K2 + 2;
-    int nlen1 = 0;   /* trailing entries of row length 1 (|m| = L): not split */
-    for (int i = nc - 1; i >= 0 && nlen1 < 2; i--) {
-        const int mm = ent_m[cstart + uperm[cstart + i]];
-        if ((mm < 0 ? -mm : mm) != L) break;
-        nlen1++;
-    }
-    const int nsplit = nc < FSX_CROSS_BLOCK ? min(FSX_CROSS_BLOCK - nc, nc - nlen1) : 0;
-    const bool uact = tid < nc + nsplit;
-    const bool usplit = tid < 2 * nsplit;
-    int ue = 0, ul = 0, um = 0, uam = 0, uk0 = 0, uk1 = 0, ukst = 1;
-    if (uact) {
-        ue = uperm[cstart + (usplit ? tid >> 1 : tid - nsplit)];
-        ul = ent_l[cstart + ue];
-        um = ent_m[cstart + ue];
-        uam = um < 0 ? -um : um;
-        uk0 = usplit && (tid & 1) ? 1 : 0;
-        uk1 = L - uam + 1;
-        ukst = usplit ? 2 : 1;
-    }
-    const bool ustore = uact && !(usplit && (tid & 1));
-    const int ub0 = uact ? mstart[um + L] - cstart : 0;
-    /* T (in global memory, and its LDS copy when TST) is stored per |m|
-     * block as [l1][l] (consecutive l, i.e. consecutive threads, at
-     * consecutive addresses): element (am, l, l1) at tpk_row(am, am, K) +
-     * (l1 - am) * (K - am) + (l - am) */
-    const int urow = uact ? tpk_row(uam, uam, K) + (ul - uam) : 0;
-    const int ustep = K - uam;
-    /* pairing slots: with npk > 0 (conjugate-symmetric coefficients, the
-     * chunk of m = 0) the m = 0 entries l = 2i and 2i + 1 share slot i, the
-     * real part of the first (real for even l) and the imaginary part of the
-     * second (imaginary for odd l); their twiddle is 1, so Re(w R U) of the
-     * slot is the sum of the two entries' terms.  Entry e >= 2 npk has slot
-     * e - npk. */
-    const int ns = nc - npk;
-    /* PW poses per wavefront, LP lanes each: lane sl of a pose takes slots
-     * sl, sl + LP, ... (J per lane) */
-    constexpr int LP = FSX_WAVE / PW;
-    const int sl = lane % LP, half = lane / LP;
-    /* bytes per receptor row and per row of U in LDS (three parts of nc
-     * entries each), the lane's slot within a row, and the step to its last
-     * slot (back to slot 0 when that one is past the last slot) */
-    const unsigned rstride = 3u * (unsigned)nc * (unsigned)sizeof(E);
-    const unsigned soff = (unsigned)(sl * sizeof(E));
-    const unsigned dlast = sl + LP * (J - 1) < ns ? (unsigned)(LP * (J - 1) * sizeof(E))
-                                                  : (unsigned)0 - soff;
-    /* byte offset of each slot's twiddle e^(-i m alpha2) within a row of tw2
-     * (rows of 2L + 2 entries, m = -L..L and a zero at 2L + 1, which a slot
-     * past the last one reads) */
-    unsigned emo[J];
-#pragma unroll
-    for (int j = 0; j < J; j++) {
-        int ec = sl + LP * j;
-        const int m = ec < ns ? ent_m[cstart + (ec < npk ? 2 * ec : ec + npk)] : L + 1;
-        emo[j] = (unsigned)(m + L) * (unsigned)sizeof(E);
-    }
-    /* after the lane reduction: one pose: lanes 0, 8, .., 40 hold the six
-     * sums; two poses: lanes 0, 8, 4, 16, 24, 20 of each half (bits 4, 3, 2
-     * of the lane select sum 3 b4 + (b2 ? 2 : b3)) */
-    const int rb4 = (lane >> 4) & 1, rb3 = (lane >> 3) & 1, rb2 = (lane >> 2) & 1;
-    const int slot = PW == 1 ? lane >> 3 : 3 * rb4 + (rb2 ? 2 : rb3);
-    const bool writer = PW == 1 ? (lane & 7) == 0 && slot < 6 : (lane & 3) == 0 && !(rb2 && rb3);
-    const int ngg = (ng + G - 1) / G;   /* gamma2 groups per beta2 */
-    const int nbg = nbeta * ngg;
-    /* Tiles in nx contiguous ranges of the (q, beta2, gamma2 group) order,
-     * one per XCD: workgroups are dispatched to the XCDs round-robin, so
-     * block b runs on XCD b % nx, and the blocks of one XCD walk one range
-     * together.  At any time they then read the receptor rows of about one
-     * q, which that XCD's L2 can hold.  nx = 1: one range, plain grid
-     * stride.  The grid is a multiple of nx. */
-    const long per = (ntiles + nx - 1) / nx;
-    const int xb = blockIdx.x % nx, gb = gridDim.x / nx;
-    for (long j = blockIdx.x / nx; j < per; j += gb) {
-        const long tile = xb * per + j;
-        if (tile >= ntiles) break;
-        const int q = (int)(tile / nbg), bgg = (int)(tile - (long)q * nbg);
-        const int b2 = bgg / ngg, g20 = (bgg - b2 * ngg) * G;
-        const int nr = ng - g20 < G ? ng - g20 : G;   /* rows of this tile */
-        const E *Bq = Bc + (((long)q * nrows + b2 * ng + g20) * 3) * nc;
-        const E *Rq = Rc + (long)q * nrows * 3 * nc;   /* receptor rows of this q */
-        const char *RqB = reinterpret_cast<const char *>(Rq);
-        bool staged = false;
-        /* Each z's bucket header, translation block (TST) and first pose
-         * records are read one z ahead: the next z's header is requested
-         * before the U step, its translation block and records after it,
-         * so that they arrive while this z's U
-         * step and pose loop run instead of stalling the block between z
-         * values.  Header: the tile's buckets are adjacent keys, their poses
-         * adjacent in recs; lane r < nr of every wavefront reads the count
-         * of row r and lane G the first record's offset (vector loads, so
-         * that waiting for them does not wait for the LDS traffic of the U
-         * step), read back by lane broadcast. */
-        auto hload = [&](int zz) {
-            const int key = (zz * nbeta + b2) * ng + g20;
-            int v = 0;
-            if (lane < nr) v = counts[key + lane];
-            else if (lane == G) v = offs[key];
-            return v;
-        };
-        /* first pose of each row of the tile (rows past nr: none) */
-        auto hread = [&](int v, int (&cm)[G + 1], int &st) {
-            cm[0] = 0;
-#pragma unroll
-            for (int r = 0; r < G; r++)
-                cm[r + 1] = cm[r] + (r < nr ? __builtin_amdgcn_readlane(v, r) : 0);
-            st = __builtin_amdgcn_readlane(v, G);
-        };
-        /* a translation block straight into sT (TST): each wavefront copies
-         * 64 consecutive 4-byte words per instruction with global_load_lds,
-         * so the copy runs in the background without registers; it is
-         * waited for (vmcnt) before the barrier that precedes the U step */
-        auto tdma = [&](int zz) {
-            const unsigned *Tz = reinterpret_cast<const unsigned *>(T + ((long)zz * Q + q) * Tn);
-            const int nw = Tn * (int)(sizeof(F) / 4);
-            unsigned *dst = reinterpret_cast<unsigned *>(sT);
-            for (int b = wave * FSX_WAVE; b < nw; b += nwave * FSX_WAVE)
-                if (b + lane < nw)
-                    __builtin_amdgcn_global_load_lds(
-                        Tz + b + lane, (__attribute__((address_space(3))) void *)(dst + b), 4, 0, 0);
-        };
-        int2 rpf = make_int2(0, 0);   /* a first record (tid < FSX_CROSS_PB) */
-        auto rload = [&](int st, int n) {
-            if (n > 0 && tid < FSX_CROSS_PB) {
-                const int4 r4 = recs[st + min(tid, n - 1)];
-                rpf = make_int2(r4.y, (r4.z << 3) | (r4.w - g20));
-            }
-        };
-        int cum[G + 1], start = 0;
-        hread(hload(0), cum, start);
-        int cnt = cum[G];
-        if (TST && cnt > 0) tdma(0);
-        rload(start, cnt);
-        for (int z = 0; z < zn; z++) {
-            const bool zmore = z + 1 < zn;
-            int cum2[G + 1], start2 = 0;
-#pragma unroll
-            for (int r = 0; r <= G; r++) cum2[r] = 0;
-            if (cnt == 0) {
-                /* an empty z: straight on to the next one */
-                if (zmore) {
-                    hread(hload(z + 1), cum2, start2);
-                    const int cnt2 = cum2[G];
-                    if (TST && cnt2 > 0) tdma(z + 1);
-                    rload(start2, cnt2);
-#pragma unroll
-                    for (int r = 0; r <= G; r++) cum[r] = cum2[r];
-                    start = start2;
-                    cnt = cnt2;
-                }
-                continue;
-            }
-            const F *Tq = T + ((long)z * Q + q) * Tn;
-            /* pose loader: receptor row entries, twiddles and row of pose p,
-             * whose record is sP[p - pb].  One register set (a second one for
-             * the next pose's loads, in flight during this pose's pairing,
-             * measured slower: the kernel then holds three blocks per CU
-             * instead of four); the first pose is loaded after the U step
-             * (loading it before kept its registers live through U and cost
-             * FP64 tables a wavefront per SIMD) */
-            E rrc[3][J];
-            F wrc[J], wic[J];
-            int prowc = 0;
-            auto load_pose = [&](int p, int pb, E (&rr)[3][J], F (&wr)[J], F (&wi)[J],
-                                 int &prow) {
-                const int2 rec = sP[p - pb];
-                prow = rec.y & 7;
-                /* no branches, so that the J slots' loads are all in flight
-                 * together: a lane's slot past the last one (only the last
-                 * of the J can be) reads slot 0, and the pairing gives it a
-                 * zero twiddle.  Receptor entries: the part's base (uniform,
-                 * in scalar registers) plus one 32-bit byte offset of the
-                 * row and the lane's slot (the host keeps a q's rows below
-                 * 4 GiB and their count below 2^24), the slot step LP j as
-                 * the load's immediate offset */
-                const unsigned roff = __umul24((unsigned)rec.x, rstride) + soff;
-                const unsigned twr = __umul24((unsigned)rec.y >> 3, (unsigned)((N + 1) * sizeof(E)));
-#pragma unroll
-                for (int j = 0; j < J; j++) {
-                    const E w = *reinterpret_cast<const E *>(
-                        reinterpret_cast<const char *>(tw2) + (twr + emo[j]));
-                    wr[j] = w.re;
-                    wi[j] = w.im;
-#pragma unroll
-                    for (int X = 0; X < 3; X++) {
-                        const char *base = RqB + (size_t)X * nc * sizeof(E);
-                        rr[X][j] = j < J - 1
-                                       ? *reinterpret_cast<const E *>(base + (size_t)roff +
-                                                                      (size_t)(LP * j * sizeof(E)))
-                                       : *reinterpret_cast<const E *>(base + (size_t)(roff + dlast));
-                    }
-                }
-            };
-            /* the translation block copied in the background (TST) has
-             * landed in sT (the barrier before the U step makes it visible
-             * to the other wavefronts) */
-            if (TST) __builtin_amdgcn_s_waitcnt(FSX_WAITCNT_VM0);
-            /* the next z's header, requested after that wait (which would
-             * otherwise wait for it too) and read after the U step */
-            const int hv = zmore ? hload(z + 1) : 0;
-            __builtin_amdgcn_sched_barrier(0);
-
-            /* all FSX_CROSS_PB records of a batch are valid: past the
-             * z's last pose they repeat it, so the pose loop reads them
-             * without a clamp */
-            if (tid < FSX_CROSS_PB) sP[tid] = rpf;
-            /* staging: four loads per thread in flight (an index past the end
-             * reloads element b0, whose store is then skipped), then the stores */
-            if (!staged) {
-                /* global (row r, part Y, entry e) -> LDS e * 3G + 3r + Y (BIL) */
-                const int nb3 = 3 * nc * nr;
-                auto bdst = [&](int b) {
-                    if (!BIL) return b;
-                    const int rY = b / nc;
-                    return (b - rY * nc) * SB + rY;
-                };
-                for (int b0 = tid; b0 < nb3; b0 += 4 * FSX_CROSS_BLOCK) {
-                    const int i1 = b0 + FSX_CROSS_BLOCK, i2 = b0 + 2 * FSX_CROSS_BLOCK;
-                    const int i3 = b0 + 3 * FSX_CROSS_BLOCK;
-                    E t0 = Bq[b0];
-                    E t1 = Bq[i1 < nb3 ? i1 : b0];
-                    E t2 = Bq[i2 < nb3 ? i2 : b0];
-                    E t3 = Bq[i3 < nb3 ? i3 : b0];
-                    sB[bdst(b0)] = t0;
-                    if (i1 < nb3) sB[bdst(i1)] = t1;
-                    if (i2 < nb3) sB[bdst(i2)] = t2;
-                    if (i3 < nb3) sB[bdst(i3)] = t3;
-                }
-                staged = true;
-            }
-            lds_barrier();
-            {
-                /* T = i^(l1 - l) tau with tau real and the ligand rows stored
-                 * as i^(-l1) B, so that i^(-l) conj(T) B = tau (i^(-l1) B): a
-                 * real-by-complex sum */
-                const F *Tr = (TST ? sT : Tq) + urow;
-                const E *bp = sB + ub0 * (BIL ? SB : 1);
-                F ur[G][3], ui[G][3];
-#pragma unroll
-                for (int r = 0; r < G; r++)
-#pragma unroll
-                    for (int Y = 0; Y < 3; Y++) ur[r][Y] = ui[r][Y] = 0;
-                for (int k = uk0; k < uk1; k += ukst) {
-                    /* the step's LDS reads first, then its FMAs */
-                    const F tv = Tr[k * ustep];
-                    E bv[3 * G];
-#pragma unroll
-                    for (int i = 0; i < 3 * G; i++) bv[i] = BIL ? bp[k * SB + i] : bp[i * nc + k];
-#pragma unroll
-                    for (int r = 0; r < G; r++)
-#pragma unroll
-                        for (int Y = 0; Y < 3; Y++) {
-                            ur[r][Y] += tv * bv[r * 3 + Y].re;
-                            ui[r][Y] += tv * bv[r * 3 + Y].im;
-                        }
-                }
-                /* split entries: the even steps (even lane) plus the odd
-                 * steps (its odd neighbour), in that order */
-                if (nsplit > 0) {
-#pragma unroll
-                    for (int r = 0; r < G; r++)
-#pragma unroll
-                        for (int Y = 0; Y < 3; Y++) {
-                            const F orr = dpp_mov<FSX_DPP_XOR1>(ur[r][Y]);
-                            const F oi = dpp_mov<FSX_DPP_XOR1>(ui[r][Y]);
-                            if (usplit) {
-                                ur[r][Y] += orr;
-                                ui[r][Y] += oi;
-                            }
-                        }
-                }
-                /* stored is i^(-l) U (the receptor rows hold i^l R, so the
-                 * pairing's products are unchanged); in a packed m = 0 slot
-                 * both values are real, the second one negated so that
-                 * Re(R U) of the slot adds the two entries' products */
-                if (ustore) {
-                    const int us = ue < 2 * npk ? ue >> 1 : ue - npk;   /* pairing slot */
-#pragma unroll
-                    for (int r = 0; r < G; r++)
-#pragma unroll
-                        for (int Y = 0; Y < 3; Y++) {
-                            E *d = sU + (r * 3 + Y) * nc + us;
-                            if (ue >= 2 * npk) {
-                                d->re = ur[r][Y];
-                                d->im = ui[r][Y];
-                            } else if (ue & 1) {
-                                d->im = -ur[r][Y];
-                            } else {
-                                d->re = ur[r][Y];
-                            }
-                        }
-                }
-            }
-            lds_barrier();
-            /* the next z's header, and its first records and translation
-             * block in flight during this z's pose loop (U has read sT) */
-            int cnt2 = 0;
-            if (zmore) {
-                hread(hv, cum2, start2);
-                cnt2 = cum2[G];
-                rload(start2, cnt2);
-                if (TST && cnt2 > 0) tdma(z + 1);
-            }
-            /* batches of FSX_CROSS_PB poses; the records of the first are
-             * staged with the ligand rows */
-            for (int pb = 0; pb < cnt; pb += FSX_CROSS_PB) {
-            if (pb > 0) {
-                if (tid < FSX_CROSS_PB) {
-                    const int4 r4 = recs[start + min(pb + tid, cnt - 1)];
-                    sP[tid] = make_int2(r4.y, (r4.z << 3) | (r4.w - g20));
-                }
-                lds_barrier();
-            }
-            const int pe = min(cnt, pb + FSX_CROSS_PB);
-            /* pairing of one pose (this lane's half of the wavefront) with
-             * the pose record's receptor row and twiddles in rr, wr, wi */
-            auto pair_pose = [&](const E (&rr)[3][J], const F (&wr)[J], const F (&wi)[J],
-                                 int prow, int p) {
-                const bool act = p < pe;
-                const E *sUp = reinterpret_cast<const E *>(reinterpret_cast<const char *>(sU) +
-                                                           __umul24((unsigned)prow, rstride));
-                F va[6] = {0, 0, 0, 0, 0, 0};
-#pragma unroll
-                for (int j = 0; j < J; j++) {
-                    const bool ok = j < J - 1 || sl + LP * j < ns;
-                    const int ec = ok ? sl + LP * j : 0;
-                    {
-                        E rv = rr[0][j], rd = rr[1][j], rw = rr[2][j];
-                        E uv = sUp[ec], ud = sUp[nc + ec], uw = sUp[2 * nc + ec];
-                        const F w_r = wr[j], w_i = wi[j];   /* zero past the last slot */
-                        /* twiddled receptor factor: w * R^X */
-                        F vr = w_r * rv.re - w_i * rv.im, vi = w_r * rv.im + w_i * rv.re;
-                        F dr = w_r * rd.re - w_i * rd.im, di = w_r * rd.im + w_i * rd.re;
-                        F xr = w_r * rw.re - w_i * rw.im, xi = w_r * rw.im + w_i * rw.re;
-                        /* Re of each product, accumulated term by term (one
-                         * fused multiply-add per term) */
-                        va[0] += vr * uv.re; va[0] -= vi * uv.im;
-                        va[1] += vr * ud.re; va[1] -= vi * ud.im;
-                        va[1] += dr * uv.re; va[1] -= di * uv.im;
-                        va[2] += vr * uw.re; va[2] -= vi * uw.im;
-                        va[2] += xr * uv.re; va[2] -= xi * uv.im;
-                        va[3] += dr * ud.re; va[3] -= di * ud.im;
-                        va[4] += dr * uw.re; va[4] -= di * uw.im;
-                        va[4] += xr * ud.re; va[4] -= xi * ud.im;
-                        va[5] += xr * uw.re; va[5] -= xi * uw.im;
-                    }
-                }
-                /* the cross-lane sums run in the contraction's type */
-                F v[8] = {va[0], va[1], va[2], va[3], va[4], va[5], 0, 0};
-                if (PW == 1) {
-                    /* transpose-reduce over the 64 lanes: after the three
-                     * halving steps lane bits 5,4,3 select the slot, then a
-                     * sum over the 8 lanes of bits 2,1,0; lanes 0, 8, .., 40
-                     * hold slots 0..5 */
-#pragma unroll
-                    for (int i = 0; i < 4; i++) v[i] = tr_swap32(v[i], v[i + 4]);
-#pragma unroll
-                    for (int i = 0; i < 2; i++) v[i] = tr_swap16(v[i], v[i + 2]);
-                    const bool hi = (lane & 8) != 0;
-                    const F send = hi ? v[0] : v[1];
-                    const F keep = hi ? v[1] : v[0];
-                    v[0] = keep + dpp_mov<FSX_DPP_ROR8>(send);
-                    v[0] += dpp_mov<FSX_DPP_HMIRROR>(v[0]);
-                    v[0] += dpp_mov<FSX_DPP_XOR1>(v[0]);
-                    v[0] += dpp_mov<FSX_DPP_XOR2>(v[0]);
-                } else {
-                    /* the same within each 32-lane half (one pose each), on
-                     * the six sums: lane bit 4 (16-row swap) pairs sums i and
-                     * i + 3; bit 3 (row_ror:8) pairs the first two of those
-                     * and adds the third across itself; bit 2
-                     * (row_half_mirror: lane j <-> 7 - j) pairs the two
-                     * results; then a sum over the quad of bits 1,0 */
-#pragma unroll
-                    for (int i = 0; i < 3; i++) v[i] = tr_swap16(v[i], v[i + 3]);
-                    const bool b3 = rb3 != 0, b2 = rb2 != 0;
-                    {
-                        const F send = b3 ? v[0] : v[1];
-                        const F keep = b3 ? v[1] : v[0];
-                        v[0] = keep + dpp_mov<FSX_DPP_ROR8>(send);
-                        v[1] = v[2] + dpp_mov<FSX_DPP_ROR8>(v[2]);
-                    }
-                    const F send = b2 ? v[0] : v[1];
-                    const F keep = b2 ? v[1] : v[0];
-                    v[0] = keep + dpp_mov<FSX_DPP_HMIRROR>(send);
-                    v[0] += dpp_mov<FSX_DPP_XOR1>(v[0]);
-                    v[0] += dpp_mov<FSX_DPP_XOR2>(v[0]);
-                }
-                if (writer && act) sO[(p - pb) * 6 + slot] = v[0];
-            };
-            /* the wavefront's poses of this batch, pp = wave, wave + nwave,
-             * ...: PW consecutive poses per step (a half past the batch's
-             * last pose repeats it and does not write) */
-            for (int pp = wave; pb + PW * pp < pe; pp += nwave) {
-                const int p = pb + PW * pp + half;
-                load_pose(p, pb, rrc, wrc, wic, prowc);
-                /* every load of the pose is issued before the first use */
-                __builtin_amdgcn_sched_barrier(0);
-                pair_pose(rrc, wrc, wic, prowc, p);
-            }
-            /* the batch's sums to acc (pose-major [pose][q][6]), added to
-             * those of the earlier m-chunks */
-            lds_barrier();
-            for (int i = tid; i < (pe - pb) * 6; i += FSX_CROSS_BLOCK) {
-                const int ip = i / 6;
-                double *d = acc + ((long)(start + pb + ip) * Q + q) * 6 + (i - ip * 6);
-                const double x = 2.0 * (double)sO[i];
-                *d = first ? x : *d + x;
-            }
-            }
-            /* no barrier here: until the next z's first barrier a wavefront
-             * only writes the next records (sP), the staged ligand rows (sB,
-             * at a new tile) and the translation block (sT, read by the U
-             * step before its closing barrier), none of which the batch's
-             * writing of sO reads; the next pose loop writes sO only after
-             * that barrier */
-#pragma unroll
-            for (int r = 0; r <= G; r++) cum[r] = cum2[r];
-            start = start2;
-            cnt = cnt2;
-        }
-    }
-}
-
-template <int J, int TST, int G, typename E, int PW>
-__global__ void __launch_bounds__(FSX_CROSS_BLOCK, sizeof(E) == 8 ? 4 : 1)
-k_cross(double *acc, const E *Rc, const E *Bc, const decltype(E::re) *T, const E *tw2,
-        const int *ent, int cstart, int nc, const int *counts, const int *offs,
-        const int4 *recs, long ntiles, int nrows, int Q, int L, int nbeta, int nx, int ng,
-        int zn, int first, int npk)
-{
-    cross_body<J, TST, G, E, PW>(acc, Rc, Bc, T, tw2, ent, cstart, nc, counts, offs, recs, ntiles,
-                                 nrows, Q, L, nbeta, nx, ng, zn, first, npk);
-}
-
-/* One m-chunk of several complexes in one persistent launch (the batched
- * form): every block takes its share of the tiles of job 0, then of job 1,
- * and so on, so that a block that runs out of one complex's tiles goes on
- * to the next complex instead of idling until the launch drains.  The jobs
- * of one launch share the template parameters; each complex appears at most
- * once (its m-chunks are launched in order, one launch per chunk index). */
-struct fsx_cross_job {
-    double *acc;
-    const void *Rc, *Bc, *T, *tw2;
-    const int *ent, *counts, *offs;
-    const int4 *recs;
-    long ntiles;
-    int cstart, nc, nrows, Q, L, nbeta, nx, ng, zn, first, npk;
-};
-
-template <int J, int TST, int G, typename E, int PW>
-__global__ void __launch_bounds__(FSX_CROSS_BLOCK, sizeof(E) == 8 ? 4 : 1)
-k_cross_jobs(const fsx_cross_job *jobs, int njobs)
-{
-    typedef decltype(E::re) F;
-    for (int k = 0; k < njobs; k++) {
-        const fsx_cross_job &jb = jobs[k];
-        cross_body<J, TST, G, E, PW>(jb.acc, (const E *)jb.Rc, (const E *)jb.Bc, (const F *)jb.T,
-                                     (const E *)jb.tw2, jb.ent, jb.cstart, jb.nc, jb.counts,
-                                     jb.offs, jb.recs, jb.ntiles, jb.nrows, jb.Q, jb.L, jb.nbeta,
-                                     jb.nx, jb.ng, jb.zn, jb.first, jb.npk);
-        /* the next job lays out the LDS for its own chunk size */
-        __syncthreads();
-    }
 }
 
 /* ---- per-pose fit, lockstep over a pose queue ------------------------------
@@ -2256,7 +1809,7 @@ static __device__ __align__(256) unsigned char scratch[FSX_NOALLOC_SCRATCH_BYTES
 static void *g_scratch = NULL;
 enum {
     B_BES, B_T, B_RT, B_BT, B_A, B_B, B_DW, B_DS, B_TWA, B_TWG, B_Q, B_Z, B_AM, B_CINT,
-    B_POSES, B_KEYS, B_COUNTS, B_OFFS, B_FILL, B_RECS, B_INFO, B_ACC, B_SCORE, B_C1, B_C2,
+    B_POSES, B_KEYS, B_COUNTS, B_OFFS, B_UNITS, B_RECS, B_INFO, B_ACC, B_SCORE, B_C1, B_C2,
     B_CROSSOUT, B_ENT, B_COFF, B_NEXT, B_TALLY, B_SRCT, B_TW2, B_FITCT, B_FITOUT, B_BX, B_BOUT, B_AXYZ,
     B_AFF, B_AWS, B_AQ, B_ARE, B_AIM, B_RTMP, B_FITSC, B_ACCF, B_IN, B_NBUF
 };
@@ -2354,253 +1907,76 @@ static inline unsigned nblk(long n, int t) { return (unsigned)((n + t - 1) / t);
         if (r_ != FSX_OK) return r_;   \
     } while (0)
 
-/* launches of the element-type dependent stages (FP64 or FP32 tables);
- * g: the buffers of the plan being launched (indices P_*) */
-enum { G_DW = 7, G_ENT = 23, G_COFF = 25 };
+/* kernel of a cross-term launch for chunks of ns slots */
 template <typename E>
-static void launch_rotate(hipStream_t s, void *out, void *tmp, const cplx *srct, long nrot,
-                          size_t lds, int nb, int ng, int Q, int L, int gc, int C,
-                          const int *csz, const int *cst, const long *coff, int mlo, int npk0,
-                          int lrot, void *const *g)
+static const void *cross_kernel(int jn, int jobs)
 {
-    hipLaunchKernelGGL(k_rotate<E>, dim3((unsigned)nrot), dim3(256), lds, s, (E *)tmp, srct,
-                       (const double *)g[G_DW], (const int *)g[G_ENT],
-                       (const long *)g[G_COFF], nb, ng, Q, L, gc, mlo);
-    /* 64-row tiles of FP32 tables, 32-row tiles of FP64 tables (33 KB of LDS) */
-    const int TR = sizeof(E) == 8 ? 64 : 32;
-    const int nrows = nb * ng;
-    for (int c = 0; c < C; c++) {
-        if (csz[c] == 0) continue;
-        const int nte = (csz[c] + 63) / 64, ntr = (nrows + TR - 1) / TR;
-        const long nblkT = (long)Q * 3 * nte * ntr;
-        if (sizeof(E) == 8)
-            hipLaunchKernelGGL((k_tab_transpose<E, 64>), dim3((unsigned)nblkT), dim3(256), 0, s,
-                               (E *)out + coff[c], (const E *)tmp + coff[c], csz[c], nrows, nte, ntr,
-                               c == 0 ? npk0 : 0, (const int *)g[G_ENT] + cst[c], lrot);
-        else
-            hipLaunchKernelGGL((k_tab_transpose<E, 32>), dim3((unsigned)nblkT), dim3(256), 0, s,
-                               (E *)out + coff[c], (const E *)tmp + coff[c], csz[c], nrows, nte, ntr,
-                               c == 0 ? npk0 : 0, (const int *)g[G_ENT] + cst[c], lrot);
-    }
+    if (jobs)
+        return jn <= 1 ? (const void *)k_cross_jobs<1, E> : jn <= 2 ? (const void *)k_cross_jobs<2, E>
+             : jn <= 3 ? (const void *)k_cross_jobs<3, E> : (const void *)k_cross_jobs<4, E>;
+    return jn <= 1 ? (const void *)k_cross<1, E> : jn <= 2 ? (const void *)k_cross<2, E>
+         : jn <= 3 ? (const void *)k_cross<3, E> : (const void *)k_cross<4, E>;
 }
-
-/* plan buffer indices the cross-term launch reads (kept equal to the P_*
- * enumeration below) */
-enum { G_T = 1, G_RT = 2, G_BT = 3, G_COUNTS = 17, G_OFFS = 18, G_RECS = 20, G_ACC = 21,
-       G_TW2 = 24 };
-template <typename E, int G>
-static void launch_cross_g(hipStream_t s, int C, const int *csz, const int *cst,
-                           const long *coff, int Tn, long grid, int nrows, int Q, int L,
-                           int nb, int npk0, int ng, int zn, void *const *g)
+static const void *cross_kernel_of(int mixed, int jn, int jobs)
 {
-    const int tst = (long)Tn * (long)(sizeof(E) / 2) <= 40 * 1024;
-    const long ntiles = (long)Q * nb * ((ng + G - 1) / G);
-    for (int c = 0; c < C; c++) {
-        if (csz[c] == 0) continue;
-        const int npk = c == 0 ? npk0 : 0;
-        const int ns = csz[c] - npk;   /* pairing slots */
-        /* FP32 tables: two poses per wavefront (32 lanes each) when the
-         * slots fit four per lane (FSX_CROSS_PW=1: one pose per wavefront) */
-        const int pw = sizeof(E) == 8 && ns <= 4 * (FSX_WAVE / 2) &&
-                       env_int("FSX_CROSS_PW", 2, 1, 2) == 2 ? 2 : 1;
-        int jn = (ns + FSX_WAVE / pw - 1) / (FSX_WAVE / pw);
-        void (*kern)(double *, const E *, const E *, const decltype(E::re) *, const E *, const int *,
-                     int, int, const int *, const int *, const int4 *, long, int, int, int,
-                     int, int, int, int, int, int);
-        if (pw == 2)
-            kern = tst ? (jn <= 1 ? k_cross<1, 1, G, E, 2> : jn <= 2 ? k_cross<2, 1, G, E, 2>
-                          : jn <= 3 ? k_cross<3, 1, G, E, 2> : k_cross<4, 1, G, E, 2>)
-                       : (jn <= 1 ? k_cross<1, 0, G, E, 2> : jn <= 2 ? k_cross<2, 0, G, E, 2>
-                          : jn <= 3 ? k_cross<3, 0, G, E, 2> : k_cross<4, 0, G, E, 2>);
-        else if (tst)
-            kern = jn <= 1 ? k_cross<1, 1, G, E, 1> : jn <= 2 ? k_cross<2, 1, G, E, 1>
-                 : jn <= 3 ? k_cross<3, 1, G, E, 1> : k_cross<4, 1, G, E, 1>;
-        else
-            kern = jn <= 1 ? k_cross<1, 0, G, E, 1> : jn <= 2 ? k_cross<2, 0, G, E, 1>
-                 : jn <= 3 ? k_cross<3, 0, G, E, 1> : k_cross<4, 0, G, E, 1>;
-        size_t lds = sizeof(E) * (size_t)(cross_sb<E, G>() + 3 * G) * csz[c] +
-                     (tst ? cross_tst_bytes<decltype(E::re)>(Tn) : 0) +
-                     (sizeof(decltype(E::re)) * 6 + sizeof(int2)) * FSX_CROSS_PB;
-        /* persistent-style grid: the blocks that fit the chip at once
-         * (FSX_CROSS_BLOCKS_PER_CU overrides the per-CU count) */
-        long gsz = grid;
-        if (gsz <= 0) {
-            int per = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, FSX_CROSS_BLOCK, lds)
-                    != hipSuccess || per < 1)
-                per = 2;
-            gsz = (long)g_ncu * per;
-        }
-        if (gsz > ntiles) gsz = ntiles;
-        /* XCD-contiguous tile ranges when the grid divides evenly
-         * (FSX_CROSS_XCD=0 turns them off) */
-        int nx = env_int("FSX_CROSS_XCD", 1, 0, 1) ? g_nxcd : 1;
-        if (nx > 1 && (gsz % nx != 0 || ntiles < 4L * gsz)) nx = 1;
-        hipLaunchKernelGGL(kern, dim3((unsigned)gsz), dim3(FSX_CROSS_BLOCK), lds, s,
-                           (double *)g[G_ACC], (const E *)g[G_RT] + coff[c],
-                           (const E *)g[G_BT] + coff[c], (const decltype(E::re) *)g[G_T],
-                           (const E *)g[G_TW2], (const int *)g[G_ENT], cst[c], csz[c],
-                           (const int *)g[G_COUNTS], (const int *)g[G_OFFS],
-                           (const int4 *)g[G_RECS], ntiles, nrows, Q, L, nb, nx, ng, zn,
-                           c == 0, npk);
+    return mixed ? cross_kernel<cplx32>(jn, jobs) : cross_kernel<cplx>(jn, jobs);
+}
+static int cross_jn(int ns) { return ns <= FSX_WAVE ? 1 : (ns + FSX_WAVE - 1) / FSX_WAVE; }
+static size_t cross_lds_of(int mixed, int ns, int urows)
+{
+    return mixed ? cross_lds<float>(ns, urows) : cross_lds<double>(ns, urows);
+}
+/* blocks of a cross-term launch: those resident at once, up to five per CU
+ * (FSX_CROSS_BLOCKS_PER_CU overrides the per-CU count).  More only take each
+ * other's cache lines: FP32 tables, 300,000 poses at L = 25, 98, 76, 66.2, 65.6 and
+ * 73.7 ms with 2 to 6 blocks; 210,000 at L = 15 5.63, 4.64, 4.40, 4.46 and 4.64. */
+static long cross_grid(const void *kern, size_t lds)
+{
+    int per = env_int("FSX_CROSS_BLOCKS_PER_CU", 0, 0, 16);
+    if (per == 0) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, FSX_CROSS_BLOCK, lds) != hipSuccess ||
+            per < 1)
+            per = 1;
+        per = per > 5 ? 5 : per;
     }
+    return (long)g_ncu * per;
+}
+/* ranges of the (q, unit) order: one per XCD when the grid divides evenly
+ * (FSX_CROSS_XCD=0 turns them off) */
+static int cross_nx(long grid)
+{
+    return env_int("FSX_CROSS_XCD", 1, 0, 1) && grid % g_nxcd == 0 ? g_nxcd : 1;
 }
 
 /* The persistent form of the cross-term stage (fsx_score_batch): each
  * complex's m-chunks become jobs, grouped into launches of k_cross_jobs by
- * chunk index and kernel shape, with the shape choices of launch_cross_g. */
+ * chunk index and kernel shape. */
 struct fsx_cross_group {
-    int mixed, G, tst, jn, pw, chunk;   /* the kernel shape and the m-chunk index */
-    size_t lds;                         /* the largest job's LDS */
+    int mixed, jn, chunk;       /* the kernel and the m-chunk index */
+    size_t lds;                 /* the largest job's LDS */
     int njobs, cap;
-    long grid;                          /* blocks of the launch */
+    long grid;                  /* blocks of the launch */
     fsx_cross_job *jobs;
 };
-
-template <typename E, int G>
-static const void *cross_jobs_kernel(int tst, int jn, int pw)
-{
-    if (pw == 2)
-        return tst ? (jn <= 1 ? (const void *)k_cross_jobs<1, 1, G, E, 2>
-                      : jn <= 2 ? (const void *)k_cross_jobs<2, 1, G, E, 2>
-                      : jn <= 3 ? (const void *)k_cross_jobs<3, 1, G, E, 2>
-                                : (const void *)k_cross_jobs<4, 1, G, E, 2>)
-                   : (jn <= 1 ? (const void *)k_cross_jobs<1, 0, G, E, 2>
-                      : jn <= 2 ? (const void *)k_cross_jobs<2, 0, G, E, 2>
-                      : jn <= 3 ? (const void *)k_cross_jobs<3, 0, G, E, 2>
-                                : (const void *)k_cross_jobs<4, 0, G, E, 2>);
-    return tst ? (jn <= 1 ? (const void *)k_cross_jobs<1, 1, G, E, 1>
-                  : jn <= 2 ? (const void *)k_cross_jobs<2, 1, G, E, 1>
-                  : jn <= 3 ? (const void *)k_cross_jobs<3, 1, G, E, 1>
-                            : (const void *)k_cross_jobs<4, 1, G, E, 1>)
-               : (jn <= 1 ? (const void *)k_cross_jobs<1, 0, G, E, 1>
-                  : jn <= 2 ? (const void *)k_cross_jobs<2, 0, G, E, 1>
-                  : jn <= 3 ? (const void *)k_cross_jobs<3, 0, G, E, 1>
-                            : (const void *)k_cross_jobs<4, 0, G, E, 1>);
-}
-
-static const void *cross_group_kernel(const fsx_cross_group *g)
-{
-    if (g->mixed) {
-        if (g->G >= 4) return cross_jobs_kernel<cplx32, 4>(g->tst, g->jn, g->pw);
-        if (g->G >= 2) return cross_jobs_kernel<cplx32, 2>(g->tst, g->jn, g->pw);
-        return cross_jobs_kernel<cplx32, 1>(g->tst, g->jn, g->pw);
-    }
-    if (g->G >= 4) return cross_jobs_kernel<cplx, 4>(g->tst, g->jn, g->pw);
-    if (g->G >= 2) return cross_jobs_kernel<cplx, 2>(g->tst, g->jn, g->pw);
-    return cross_jobs_kernel<cplx, 1>(g->tst, g->jn, g->pw);
-}
-
-/* the jobs of one complex's chunks appended to their groups (groups grown
- * as needed); nx is set at launch */
-template <typename E, int G>
-static int cross_collect_g(fsx_cross_group **gr, int *ngr, int C, const int *csz, const int *cst,
-                           const long *coff, int Tn, int nrows, int Q, int L, int nb, int npk0,
-                           int ng, int zn, void *const *g)
-{
-    typedef decltype(E::re) F;
-    const int tst = (long)Tn * (long)(sizeof(E) / 2) <= 40 * 1024;
-    const long ntiles = (long)Q * nb * ((ng + G - 1) / G);
-    for (int c = 0; c < C; c++) {
-        if (csz[c] == 0) continue;
-        const int npk = c == 0 ? npk0 : 0;
-        const int ns = csz[c] - npk;
-        const int pw = sizeof(E) == 8 && ns <= 4 * (FSX_WAVE / 2) &&
-                       env_int("FSX_CROSS_PW", 2, 1, 2) == 2 ? 2 : 1;
-        const int jn = (ns + FSX_WAVE / pw - 1) / (FSX_WAVE / pw);
-        const size_t lds = sizeof(E) * (size_t)(cross_sb<E, G>() + 3 * G) * csz[c] +
-                           (tst ? cross_tst_bytes<F>(Tn) : 0) +
-                           (sizeof(F) * 6 + sizeof(int2)) * FSX_CROSS_PB;
-        const int mixed = sizeof(E) == 8, jq = jn <= 1 ? 1 : jn <= 2 ? 2 : jn <= 3 ? 3 : 4;
-        fsx_cross_group *t = NULL;
-        for (int i = 0; i < *ngr; i++) {
-            fsx_cross_group *u = &(*gr)[i];
-            if (u->mixed == mixed && u->G == G && u->tst == tst && u->jn == jq && u->pw == pw &&
-                u->chunk == c)
-                t = u;
-        }
-        if (!t) {
-            fsx_cross_group *ng2 = (fsx_cross_group *)realloc(*gr, sizeof(fsx_cross_group) * (*ngr + 1));
-            if (!ng2) return FSX_ERR_NOMEM;
-            *gr = ng2;
-            t = &(*gr)[(*ngr)++];
-            memset(t, 0, sizeof(*t));
-            t->mixed = mixed; t->G = G; t->tst = tst; t->jn = jq; t->pw = pw; t->chunk = c;
-        }
-        if (t->njobs == t->cap) {
-            const int cap = t->cap ? 2 * t->cap : 8;
-            fsx_cross_job *nj = (fsx_cross_job *)realloc(t->jobs, sizeof(fsx_cross_job) * cap);
-            if (!nj) return FSX_ERR_NOMEM;
-            t->jobs = nj;
-            t->cap = cap;
-        }
-        if (lds > t->lds) t->lds = lds;
-        fsx_cross_job *jb = &t->jobs[t->njobs++];
-        jb->acc = (double *)g[G_ACC];
-        jb->Rc = (const E *)g[G_RT] + coff[c];
-        jb->Bc = (const E *)g[G_BT] + coff[c];
-        jb->T = g[G_T];
-        jb->tw2 = g[G_TW2];
-        jb->ent = (const int *)g[G_ENT];
-        jb->counts = (const int *)g[G_COUNTS];
-        jb->offs = (const int *)g[G_OFFS];
-        jb->recs = (const int4 *)g[G_RECS];
-        jb->ntiles = ntiles;
-        jb->cstart = cst[c]; jb->nc = csz[c]; jb->nrows = nrows; jb->Q = Q; jb->L = L;
-        jb->nbeta = nb; jb->nx = 1; jb->ng = ng; jb->zn = zn; jb->first = c == 0; jb->npk = npk;
-    }
-    return FSX_OK;
-}
-
-/* G = gamma2 rows per tile: tile_rows when set (the batch tuner's choice),
- * else FSX_CROSS_ROWS, else 4 for FP32 tables (the translation block and the
- * pose loop shared by more rows) and 2 for FP64 tables (LDS-bound) */
-template <typename E>
-static void launch_cross(hipStream_t s, int C, const int *csz, const int *cst, const long *coff,
-                         int Tn, long grid, int nrows, int Q, int L, int nb, int npk0, int ng,
-                         int zn, void *const *g, int tile_rows)
-{
-    const int G = tile_rows > 0 ? tile_rows : env_int("FSX_CROSS_ROWS", sizeof(E) == 8 ? 4 : 2, 1, 4);
-    if (G >= 4) launch_cross_g<E, 4>(s, C, csz, cst, coff, Tn, grid, nrows, Q, L, nb, npk0, ng, zn, g);
-    else if (G >= 2) launch_cross_g<E, 2>(s, C, csz, cst, coff, Tn, grid, nrows, Q, L, nb, npk0, ng, zn, g);
-    else launch_cross_g<E, 1>(s, C, csz, cst, coff, Tn, grid, nrows, Q, L, nb, npk0, ng, zn, g);
-}
 
 /* Entry tables of the m-major coefficient order used by the rotated tables
  * and the cross-term kernel: e runs over m = mlo..L, then l = |m|..L (mlo =
  * -L for the full set, 0 for the half set of conjugate-symmetric inputs).
  * The entries are cut into C chunks of whole m values with about ne/C
- * entries each.  ent layout (ints): [0,K2) l, [K2,2K2) m, [2K2,3K2) chunk,
- * [3K2,4K2) index within the chunk, [4K2, 4K2+C) chunk sizes,
- * [5K2, 5K2+2L+1) first entry of each m, [6K2, 6K2+C) chunk starts. */
-static int entry_tables(int L, int C, int mlo, int *ent)
+ * entries each; chunk[m - mlo] is the chunk of m. */
+static int entry_chunks(int L, int C, int mlo, int *chunk)
 {
-    const int K = L + 1, K2 = K * K;
-    const int ne = mlo == 0 ? K * (K + 1) / 2 : K2;
-    int *el = ent, *em = ent + K2, *ec = ent + 2 * K2, *ei = ent + 3 * K2;
-    int *csz = ent + 4 * K2, *mst = ent + 5 * K2, *cst = ent + 6 * K2;
+    const int K = L + 1, ne = mlo == 0 ? K * (K + 1) / 2 : K * K;
     int e = 0, c = 0, cfirst = 0;
-    for (int m = -L; m <= L; m++) mst[m + L] = 0;
     for (int m = mlo; m <= L; m++) {
-        int am = m < 0 ? -m : m;
         /* close the chunk once it holds its share of the entries */
         if (e > cfirst && c < C - 1 && (long)e * C >= (long)(c + 1) * ne) {
-            csz[c] = e - cfirst;
-            cst[c] = cfirst;
             c++;
             cfirst = e;
         }
-        mst[m + L] = e;
-        for (int l = am; l <= L; l++, e++) {
-            el[e] = l;
-            em[e] = m;
-            ec[e] = c;
-            ei[e] = e - cfirst;
-        }
+        chunk[m - mlo] = c;
+        e += K - (m < 0 ? -m : m);
     }
-    csz[c] = e - cfirst;
-    cst[c] = cfirst;
-    for (int k = c + 1; k < C; k++) { csz[k] = 0; cst[k] = e; }
     return ne;
 }
 
@@ -2645,13 +2021,13 @@ static int spf_conj_symmetric(const double *re, const double *im, int Q, int L)
  * statistics once the stream has drained. */
 enum {
     P_BES, P_T, P_RT, P_BT, P_RTMP, P_A, P_B, P_DW, P_DS, P_TWA, P_TWG, P_Q, P_Z, P_AM, P_CINT,
-    P_KEYS, P_INFO, P_COUNTS, P_OFFS, P_FILL, P_RECS, P_ACC, P_FITSC, P_ENT, P_TW2, P_COFF,
+    P_KEYS, P_INFO, P_COUNTS, P_OFFS, P_UNITS, P_RECS, P_ACC, P_FITSC, P_ENT, P_TW2, P_COFF,
     P_NEXT, P_TALLY, P_SRCT, P_POSES, P_SCORE, P_C1, P_C2, P_CROSSOUT, P_ACCF, P_IN, P_NBUF
 };
 /* the process-wide slot of each plan buffer (single calls) */
 static const int k_plan_slot[P_NBUF] = {
     B_BES, B_T, B_RT, B_BT, B_RTMP, B_A, B_B, B_DW, B_DS, B_TWA, B_TWG, B_Q, B_Z, B_AM, B_CINT,
-    B_KEYS, B_INFO, B_COUNTS, B_OFFS, B_FILL, B_RECS, B_ACC, B_FITSC, B_ENT, B_TW2, B_COFF,
+    B_KEYS, B_INFO, B_COUNTS, B_OFFS, B_UNITS, B_RECS, B_ACC, B_FITSC, B_ENT, B_TW2, B_COFF,
     B_NEXT, B_TALLY, B_SRCT, B_POSES, B_SCORE, B_C1, B_C2, B_CROSSOUT, B_ACCF, B_IN};
 /* The inputs and host tables of a call, packed into one device buffer
  * (P_IN, each at a 256-byte aligned offset) and uploaded by one copy from
@@ -2672,10 +2048,13 @@ typedef void (*fit_kernel_t)(const double *, const int4 *, const int *, int, con
 struct fsx_plan {
     fsx_hip_args A;
     int L, K, K2, N, Q, n, nb, na, ng, zn, nrows, mixed, half, mlo, npk, C, Tn, ne, dev_out;
+    int urows;           /* gamma2 rows per cross-term unit */
+    int mirror, nbr;     /* tables of beta <= pi / 2 only (fsx_mirror); their betas */
     long nkeys;
     size_t dsz, spf, es, nent;
-    int *ent;     /* host tables (malloc) */
-    long *coff;
+    int *ent;     /* host tables (malloc); ent: FSX_E_* parts */
+    long *coff;   /* first table value of each chunk: receptor [C], ligand [C] */
+    int *pm;      /* first tile, tiles, first entry, entries of each chunk [C][4] */
     double *tw2;
     size_t sz[P_NBUF];   /* bytes of each device buffer (0: not used) */
     size_t inoff[P_NBUF];   /* offset of a packed input within P_IN */
@@ -2696,17 +2075,152 @@ struct fsx_plan {
                             rotation-then-transpose kernels */
 };
 
+/* parts of the entry table (ints), from K2 = (L + 1)^2, K = L + 1, N = 2 L + 1:
+ * per entry l, m, chunk, row offset in the receptor table, row offset and
+ * padding of its places in the ligand table; first entry of each m; the blocks
+ * of the translation table (k_tmat); per chunk the row lengths of the two
+ * tables; the translation's tiles */
+#define FSX_E_L(p) 0
+#define FSX_E_M(p) ((p)->K2)
+#define FSX_E_PASS(p) (2 * (p)->K2)
+#define FSX_E_OFFR(p) (3 * (p)->K2)
+#define FSX_E_OFFB(p) (4 * (p)->K2)
+#define FSX_E_PADB(p) (5 * (p)->K2)
+#define FSX_E_OFFB2(p) (6 * (p)->K2)
+#define FSX_E_PADB2(p) (7 * (p)->K2)
+#define FSX_E_MST(p) (8 * (p)->K2)
+#define FSX_E_TB(p) (FSX_E_MST(p) + (p)->N)
+#define FSX_E_RSR(p) (FSX_E_TB(p) + 4 * (p)->K + 3)
+#define FSX_E_RSB(p) (FSX_E_RSR(p) + (p)->N)
+#define FSX_E_TILES(p) ((FSX_E_RSB(p) + (p)->N + 7) / 8 * 8)
+#define FSX_E_SIZE(p) ((size_t)FSX_E_TILES(p) + 8 * 6 * (size_t)(p)->N)   /* up to 3 tiles in 2 orders per m */
+
 static void plan_free_host(fsx_plan *p)
 {
     free(p->ent);
     free(p->coff);
+    free(p->pm);
     free(p->tw2);
+    p->pm = NULL;
     p->ent = NULL;
     p->coff = NULL;
     p->tw2 = NULL;
 }
 
-/* tile_rows, slot_cap: the cross-term tile shape (gamma2 rows per tile,
+/* Entry tables, translation tiles and table offsets of the chunks (chunk[m -
+ * mlo]) */
+static void plan_entries(fsx_plan *p, const int *chunk)
+{
+    const int L = p->L, K = p->K, TL = FSX_CROSS_TILE;
+    int *t = p->ent, *tb = t + FSX_E_TB(p), e = 0, c, nt = 0, tn = 0;
+    fsx_tile *tiles = (fsx_tile *)(t + FSX_E_TILES(p));
+    for (int m = -L; m <= L; m++) t[FSX_E_MST(p) + m + L] = 0;
+    tb[0] = 0;
+    /* block of |m| in the given order of l1: its first value in the table */
+    auto tblock = [&](int am, int split) {
+        for (int k = 0; k < tb[0]; k++)
+            if (tb[2 * k + 1] == 2 * am + split) return tb[2 * k + 2];
+        const int k = tb[0]++, Km = K - am;
+        tb[2 * k + 1] = 2 * am + split;
+        tb[2 * k + 2] = tn;
+        tn += cross_steps(Km, split) * ((Km + TL - 1) / TL) * cross_tstep(split);
+        tb[2 * k + 3] = 0;
+        tb[2 * k + 4] = tn;
+        return tb[2 * k + 2];
+    };
+    for (c = 0; c < p->C; c++) {
+        const int npk = c == 0 ? p->npk : 0, e0 = e;
+        int nc = 0, m0 = L + 1, m1 = -L - 1;
+        for (int m = p->mlo; m <= L; m++)
+            if (chunk[m - p->mlo] == c) {
+                nc += K - (m < 0 ? -m : m);
+                m0 = m < m0 ? m : m0;
+                m1 = m;
+            }
+        /* FP64: the entries whose l1 are summed by parity, then added: the
+         * first nsplit of the chunk by increasing |m| (as many as made up 256
+         * lanes of one entry, or half an entry, each; single terms are not
+         * split) */
+        int nsplit = 0;
+        if (!p->mixed && nc < 256) {
+            int one = 0;
+            for (int m = m0; m <= m1; m++) one += m == L || m == -L;
+            nsplit = 256 - nc < nc - one ? 256 - nc : nc - one;
+        }
+        p->pm[4 * c] = nt;
+        p->pm[4 * c + 2] = e0;
+        p->pm[4 * c + 3] = nc;
+        int b = 0;
+        for (int m = m0; m <= m1; m++) {
+            const int am = m < 0 ? -m : m, Km = K - am;
+            /* entries before this m by increasing |m| (m = -|m| before |m|) */
+            int before = 0;
+            for (int k = m0; k <= m1; k++) {
+                const int ak = k < 0 ? -k : k;
+                if (ak < am || (ak == am && k < m)) before += K - ak;
+            }
+            int nsp = nsplit - before;
+            nsp = nsp < 0 ? 0 : nsp > Km ? Km : nsp;
+            t[FSX_E_MST(p) + m + L] = e;
+            for (int i = 0; i < Km; i++) {
+                const int ec = e + i - e0;
+                t[FSX_E_L(p) + e + i] = am + i;
+                t[FSX_E_M(p) + e + i] = m;
+                t[FSX_E_PASS(p) + e + i] = c;
+                t[FSX_E_OFFR(p) + e + i] = ec < 2 * npk ? ec : 2 * (ec - npk);
+                t[FSX_E_OFFB2(p) + e + i] = -1;
+                t[FSX_E_PADB2(p) + e + i] = 0;
+            }
+            /* split order (the first nsp l), natural order (the others) */
+            for (int split = 1, place = 0; split >= 0; split--) {
+                const int lo = split ? 0 : nsp, hi = split ? nsp : Km;
+                if (lo >= hi) continue;
+                const int nks = cross_steps(Km, split), to = tblock(am, split);
+                int *off = t + (place ? FSX_E_OFFB2(p) : FSX_E_OFFB(p)) + e;
+                int *pad = t + (place ? FSX_E_PADB2(p) : FSX_E_PADB(p)) + e;
+                for (int i = 0; i < Km; i++) {
+                    /* split: the even ones' steps, then the odd ones' */
+                    const int pos = !split ? i : i % 2 ? 4 * nks + i / 2 : i / 2;
+                    const int end = !split || i % 2 == 0 ? 4 * nks : 8 * nks;
+                    const int last = split ? i + 2 >= Km : i + 1 == Km;
+                    off[i] = b + 6 * pos;
+                    pad[i] = last ? end - 1 - pos : 0;
+                }
+                for (int t0 = 0; t0 < Km; t0 += TL) {
+                    const int l = lo > t0 ? lo - t0 : 0, h = hi - t0 < TL ? hi - t0 : TL;
+                    if (l >= h) continue;
+                    fsx_tile *x = &tiles[nt++];
+                    x->bo = b;
+                    x->to = to + t0 / TL * nks * cross_tstep(split);
+                    x->e = e - e0 + t0;
+                    x->nks = nks;
+                    x->odd = split ? 24 * nks : 0;
+                    x->lo = l;
+                    x->hi = h;
+                    x->packed = m == 0 && npk > 0;
+                }
+                b += 24 * nks << split;
+                place++;
+            }
+            e += Km;
+        }
+        p->pm[4 * c + 1] = nt - p->pm[4 * c];
+        t[FSX_E_RSR(p) + c] = 6 * (nc - npk);
+        t[FSX_E_RSB(p) + c] = b;
+    }
+    p->Tn = tn;
+    long cr = 0, cb = 0;
+    for (c = 0; c < p->C; c++) {
+        p->coff[c] = cr;
+        p->coff[p->C + c] = cb;
+        cr += (long)p->Q * p->nrows * t[FSX_E_RSR(p) + c];
+        cb += (long)p->Q * p->nrows * t[FSX_E_RSB(p) + c];
+    }
+    p->sz[P_RT] = (size_t)cr * (p->es / 2);
+    p->sz[P_BT] = (size_t)(cb + FSX_TAB_PAD) * (p->es / 2);
+}
+
+/* tile_rows, slot_cap: the cross-term tile shape (pairs of gamma2 rows per unit,
  * pairing slots per m-chunk); 0 takes the defaults (environment knobs, then
  * the form's defaults) */
 static int plan_init(fsx_plan *p, const fsx_hip_args *A, int tile_rows, int slot_cap)
@@ -2722,7 +2236,8 @@ static int plan_init(fsx_plan *p, const fsx_hip_args *A, int tile_rows, int slot
     p->nkeys = (long)zn * nb * ng;
     if (p->nkeys > 0x3fffffffL || (long)p->nrows * Q > 0x7fffffffL) return FSX_ERR_ARG;
     if ((long)L * na >= (1L << 24) || (long)L * ng >= (1L << 24)) return FSX_ERR_ARG;
-    p->dsz = (size_t)K * N * N;
+    p->dsz = 0;
+    for (int l = 0; l <= L; l++) p->dsz += dw_size(l);
     p->spf = (size_t)3 * Q * K2;
     p->mixed = (A->flags & FSX_MIXED_FP32) != 0;
     p->dev_out = (A->flags & FSX_DEVICE_OUTPUT) != 0;
@@ -2735,64 +2250,76 @@ static int plan_init(fsx_plan *p, const fsx_hip_args *A, int tile_rows, int slot
      * pairing slots two by two (FSX_CROSS_PACK=0 keeps one slot each) */
     p->npk = p->half && env_int("FSX_CROSS_PACK", 1, 0, 1) ? K / 2 : 0;
     p->es = p->mixed ? sizeof(cplx32) : sizeof(cplx);   /* table element size */
+    /* half the betas by the mirror image of rows: FP32 tables, whose rounding
+     * is far above the 1e-11 by which a truncated pi makes the grid's mirror
+     * image miss the grid (the FP64 form keeps every beta) */
+    p->mirror = p->mixed && p->half && ng % 2 == 0 && na < (1 << 22) &&
+                fabs(A->pi - 3.14159265358979323846) < 1e-10 && env_int("FSX_MIRROR", 1, 0, 1);
+    p->nbr = p->mirror ? (nb + 1) / 2 : nb;
     /* m-chunks: one launch per chunk of entries, starting from one chunk
      * (FSX_CROSS_CHUNKS: the smallest count to try); more below while a chunk
      * is too large */
     int C = env_int("FSX_CROSS_CHUNKS", 1, 1, N);
-    p->Tn = tpk_sq(K);
-    p->nent = 8 * (size_t)K2 + 2;
+    p->nent = FSX_E_SIZE(p);
     p->ent = (int *)malloc(sizeof(int) * p->nent);
-    p->coff = (long *)malloc(sizeof(long) * (N + 1));
-    p->tw2 = (double *)calloc(2 * (size_t)na * (N + 1), sizeof(double));
-    if (!p->ent || !p->coff || !p->tw2) {
+    p->coff = (long *)malloc(sizeof(long) * 2 * (N + 1));
+    p->pm = (int *)malloc(sizeof(int) * 4 * (N + 1));
+    const int twk = p->mirror ? 2 : 1;   /* x and (l + m) mod 2 of a mirrored form's rows */
+    p->tw2 = (double *)calloc(2 * (size_t)na * (N + 1) * twk * twk, sizeof(double));
+    int *chunk = (int *)malloc(sizeof(int) * N);
+    if (!p->ent || !p->coff || !p->pm || !p->tw2 || !chunk) {
+        free(chunk);
         plan_free_host(p);
         return FSX_ERR_NOMEM;
     }
-    int *ent = p->ent;
-    /* more chunks until the largest fits: at most 4 entries per lane, and
-     * for FP32 tables at most 128 pairing slots (the two-poses-per-wavefront
-     * pairing); FSX_CROSS_CHUNK overrides the slot limit */
+    /* more chunks until the largest fits: at most 256 entries, and for FP32
+     * tables at most 128 pairing slots (the order of the FP32 sums across
+     * chunks); FSX_CROSS_CHUNK overrides the slot limit */
     const int cmax = slot_cap > 0 ? slot_cap
                                   : env_int("FSX_CROSS_CHUNK", p->mixed ? 2 * FSX_WAVE : 4 * FSX_WAVE,
                                             64, 4 * FSX_WAVE);
     int ncmax, nsmax, ne;
     for (;;) {
-        ne = entry_tables(L, C, p->mlo, ent);
+        ne = entry_chunks(L, C, p->mlo, chunk);
         ncmax = nsmax = 0;
         for (int c = 0; c < C; c++) {
-            const int nc = ent[4 * K2 + c], ns = nc - (c == 0 ? p->npk : 0);
+            int nc = 0;
+            for (int m = p->mlo; m <= L; m++)
+                if (chunk[m - p->mlo] == c) nc += K - (m < 0 ? -m : m);
+            const int ns = nc - (c == 0 ? p->npk : 0);
             if (nc > ncmax) ncmax = nc;
             if (ns > nsmax) nsmax = ns;
         }
         if ((ncmax <= 4 * FSX_WAVE && nsmax <= cmax) || C == N) break;
         C++;
     }
-    if (ncmax > 4 * FSX_WAVE) {
-        plan_free_host(p);
-        return FSX_ERR_ARG;
-    }
     /* the cross-term kernel addresses a q's receptor rows and a row of the
-     * twiddle table by 32-bit byte offsets from 24-bit products */
-    if ((size_t)p->nrows * 3 * ncmax * p->es >= ((size_t)1 << 32) || p->nrows >= (1 << 24) ||
-        na >= (1 << 24) || (size_t)na * (2 * L + 2) * p->es >= ((size_t)1 << 32)) {
+     * twiddle table by 32-bit byte offsets */
+    if (ncmax > 4 * FSX_WAVE || (size_t)p->nrows * 3 * ncmax * p->es >= ((size_t)1 << 32) ||
+        p->nrows >= (1 << 24) || na >= (1 << 24) ||
+        (size_t)na * (2 * L + 2) * p->es >= ((size_t)1 << 32)) {
+        free(chunk);
         plan_free_host(p);
         return FSX_ERR_ARG;
     }
+    p->nrows = p->nbr * ng;
     p->C = C;
     p->ne = ne;
-    /* U-phase thread -> entry of each chunk: entries by increasing |m|
-     * (decreasing row length K - |m|), in entry order within one |m| */
-    {
-        int *uperm = ent + 7 * K2 + 2;
-        const int *em = ent + K2, *csz = ent + 4 * K2, *cst = ent + 6 * K2;
+    plan_entries(p, chunk);
+    free(chunk);
+    p->urows = 2 * (tile_rows > 0 ? tile_rows : env_int("FSX_CROSS_ROWS", 0, 0, 4));
+    if (p->urows == 0) {
+        /* as many rows as three blocks' LDS leaves room for: a unit's fixed cost
+         * is shared by more poses, but a CU needs three blocks to cover the
+         * receptor rows' latency (FP64, L = 15, 210,000 poses: 9.5 ms with 6
+         * rows, 12.6 ms with 8 and two blocks, 12.6 ms with 4) */
+        int nsm = 0;
         for (int c = 0; c < C; c++) {
-            int t = 0;
-            for (int am = 0; am <= L; am++)
-                for (int i = 0; i < csz[c]; i++) {
-                    const int m = em[cst[c] + i];
-                    if ((m < 0 ? -m : m) == am) uperm[cst[c] + t++] = i;
-                }
+            const int ns = p->ent[FSX_E_RSR(p) + c] / 6;
+            if (ns > nsm) nsm = ns;
         }
+        p->urows = FSX_UROWS;
+        while (p->urows > 2 && 3 * ((cross_lds_of(p->mixed, nsm, p->urows) + 2047) / 2048) > 80) p->urows -= 2;
     }
     /* twiddle e^{-i m a2 2pi/na} per (a2, m): the same table entries the
      * reference's exact transform uses, gathered by (m a2) mod na */
@@ -2803,28 +2330,33 @@ static int plan_init(fsx_plan *p, const fsx_hip_args *A, int tile_rows, int slot
             /* half set: the m > 0 terms stand for m and -m (an exact
              * factor 2) */
             const double f = p->half && m > 0 ? 2.0 : 1.0;
-            p->tw2[2 * ((long)a2 * (N + 1) + m + L)] = f * A->tw_a[2 * k];
-            p->tw2[2 * ((long)a2 * (N + 1) + m + L) + 1] = f * A->tw_a[2 * k + 1];
+            for (int v = 0; v < twk * twk; v++) {
+                /* v = 2 x + ((l + m) mod 2), fsx_mirror */
+                const double sg = v == 3 ? -f : f;
+                double *w = p->tw2 + 2 * (((long)a2 * twk + v / 2) * twk * (N + 1) +
+                                          (long)(m + L) * twk + v % 2);
+                w[0] = sg * A->tw_a[2 * k];
+                w[1] = sg * A->tw_a[2 * k + 1];
+            }
         }
     /* the mixed form reads them as FP32 pairs, in place */
     if (p->mixed) {
         float *f32 = (float *)p->tw2;
-        for (long i = 0; i < 2L * na * (N + 1); i++) f32[i] = (float)p->tw2[i];
+        for (long i = 0; i < 2L * na * (N + 1) * twk * twk; i++) f32[i] = (float)p->tw2[i];
     }
-    const int *csz = ent + 4 * K2;
-    p->coff[0] = 0;
-    for (int c = 0; c < C; c++) p->coff[c + 1] = p->coff[c] + (long)Q * p->nrows * 3 * csz[c];
     /* buffer sizes */
     const size_t es = p->es, spfe = (size_t)3 * Q * ne;   /* rotated-table entries per row */
     size_t *z = p->sz;
     z[P_BES] = sizeof(double) * zn * Q * N;
-    z[P_T] = es * zn * Q * (size_t)p->Tn;
-    z[P_RT] = z[P_BT] = z[P_RTMP] = es * (size_t)p->nrows * spfe;
-    /* the MFMA rotation when a tile of 16 (else 8) rows of the table fits
-     * 64 KB of LDS (FSX_ROT_MFMA=0: the rotation-then-transpose kernels) */
+    z[P_T] = es / 2 * (zn * Q * (size_t)p->Tn + FSX_TAB_PAD);
+    z[P_RTMP] = es * (size_t)p->nrows * spfe;
+    /* the MFMA rotation, 16 rows of the table to a tile where that takes up to
+     * 32 KB of LDS (at 35 and 45 KB, FP64 L = 15 and FP32 L = 25, 0.72 and 6.3 ms
+     * against 0.66 and 5.0 with 8 rows and twice the blocks; at 17 KB the same),
+     * 8 rows up to 64 KB (FSX_ROT_MFMA=0: the rotation-then-transpose kernels) */
     p->rot_gt = 0;
     if (env_int("FSX_ROT_MFMA", 1, 0, 1)) {
-        if ((size_t)16 * ne * es <= 64 * 1024) p->rot_gt = 16;
+        if ((size_t)16 * ne * es <= 32 * 1024) p->rot_gt = 16;
         else if ((size_t)8 * ne * es <= 64 * 1024) p->rot_gt = 8;
     }
     if (p->rot_gt) z[P_RTMP] = 0;
@@ -2838,14 +2370,16 @@ static int plan_init(fsx_plan *p, const fsx_hip_args *A, int tile_rows, int slot
     z[P_AM] = z[P_CINT] = sizeof(double) * 6 * Q;
     z[P_KEYS] = sizeof(int) * n;
     z[P_INFO] = sizeof(int2) * n;
-    z[P_COUNTS] = z[P_FILL] = sizeof(int) * p->nkeys;
-    z[P_OFFS] = sizeof(int) * (p->nkeys + 2);
+    z[P_COUNTS] = sizeof(int) * 2 * p->nkeys;   /* counts, then fills */
+    z[P_OFFS] = sizeof(int) * (p->nkeys + 3);   /* then records, buckets, units */
+    z[P_UNITS] = sizeof(fsx_unit) * (size_t)n;
     z[P_RECS] = sizeof(int4) * n;
     z[P_ACC] = sizeof(double) * 6 * Q * (size_t)n;
     z[P_FITSC] = sizeof(double) * (size_t)(n > 0 ? n : 1);
     z[P_ENT] = sizeof(int) * p->nent;
-    z[P_TW2] = sizeof(double) * 2 * (size_t)na * (N + 1);   /* rows of 2L + 2 entries */
-    z[P_COFF] = sizeof(long) * (C + 1);
+    /* rows of 2L + 2 entries (FP32 tables: the packed FP32 values) */
+    z[P_TW2] = 2 * (size_t)na * (N + 1) * twk * twk * (p->mixed ? sizeof(float) : sizeof(double));
+    z[P_COFF] = sizeof(long) * 2 * p->C;
     z[P_NEXT] = sizeof(int);
     z[P_TALLY] = FSX_TALLY_N * sizeof(unsigned long long);
     z[P_SRCT] = sizeof(cplx) * (size_t)Q * 3 * K2 * ng;
@@ -3022,7 +2556,7 @@ static int plan_upload(fsx_plan *p, hipStream_t s, int up_dw, int up_ds)
     put(P_CINT, 0, A->cint, sizeof(double) * 6 * Q);
     put(P_ENT, 0, p->ent, sizeof(int) * p->nent);
     put(P_TW2, 0, p->tw2, p->sz[P_TW2]);
-    put(P_COFF, 0, p->coff, sizeof(long) * (p->C + 1));
+    put(P_COFF, 0, p->coff, p->sz[P_COFF]);
     HIPR(hipMemcpyAsync(p->d[P_IN], h, p->sz[P_IN], hipMemcpyHostToDevice, s));
     if (up_dw) HIPR(hipMemcpyAsync(p->d[P_DW], A->dW, p->sz[P_DW], hipMemcpyHostToDevice, s));
     if (up_ds)
@@ -3052,29 +2586,60 @@ static int plan_upload(fsx_plan *p, hipStream_t s, int up_dw, int up_ds)
 #define FSX_ST_FIT 8       /* the fit */
 #define FSX_ST_ALL 15
 
+/* chunk c of the plan as a cross-term job of a launch of grid blocks */
+static fsx_cross_job cross_job(const fsx_plan *p, int c, long grid)
+{
+    void *const *g = p->d;
+    fsx_cross_job jb;
+    memset(&jb, 0, sizeof(jb));
+    const size_t fs = p->es / 2;
+    jb.acc = (double *)g[P_ACC];
+    jb.R = (const char *)g[P_RT] + fs * p->coff[c];
+    jb.B = (const char *)g[P_BT] + fs * p->coff[p->C + c];
+    jb.T = g[P_T];
+    jb.tw2 = g[P_TW2];
+    jb.tiles = (const fsx_tile *)((const int *)g[P_ENT] + FSX_E_TILES(p)) + p->pm[4 * c];
+    jb.ntiles = p->pm[4 * c + 1];
+    jb.el = (const int *)g[P_ENT] + FSX_E_L(p);
+    jb.em = (const int *)g[P_ENT] + FSX_E_M(p);
+    jb.units = (const fsx_unit *)g[P_UNITS];
+    jb.tail = (const int *)g[P_OFFS] + p->nkeys;
+    jb.recs = (const int4 *)g[P_RECS];
+    jb.Q = p->Q; jb.L = p->L; jb.nrows = p->nrows; jb.ng = p->ng; jb.zn = p->zn; jb.Tn = p->Tn;
+    jb.cstart = p->pm[4 * c + 2];
+    jb.nc = p->pm[4 * c + 3];
+    jb.npk = c == 0 ? p->npk : 0;
+    jb.rsB = p->ent[FSX_E_RSB(p) + c];
+    jb.first = c == 0;
+    jb.nx = cross_nx(grid);
+    jb.urows = p->urows;
+    jb.mirror = p->mirror;
+    jb.nbeta = p->nb;
+    return jb;
+}
+
 static int plan_enqueue(fsx_plan *p, hipStream_t s, hipEvent_t *ev, int stages = FSX_ST_ALL)
 {
     const fsx_hip_args *A = &p->A;
     const int L = p->L, K = p->K, K2 = p->K2, N = p->N, Q = p->Q, n = p->n;
-    const int nb = p->nb, na = p->na, ng = p->ng, zn = p->zn, nrows = p->nrows, C = p->C;
+    const int nb = p->nbr, ng = p->ng, zn = p->zn, nrows = p->nrows;
     const long nkeys = p->nkeys;
-    const int *csz = p->ent + 4 * K2, *cst = p->ent + 6 * K2;
-    const long *coff = p->coff;
     void **g = p->d;
-    int *counts = (int *)g[P_COUNTS], *offs = (int *)g[P_OFFS], *fill = (int *)g[P_FILL];
-    (void)na;
+    int *counts = (int *)g[P_COUNTS], *offs = (int *)g[P_OFFS], *tail = offs + nkeys;
+    const int *ent = (const int *)g[P_ENT];
     if (stages & FSX_ST_PREP) {
     /* translation tables */
     const long nbes = (long)zn * Q * N;
     hipLaunchKernelGGL(k_bessel, dim3(nblk(nbes, 256)), dim3(256), 0, s, (double *)g[P_BES],
                        (const double *)g[P_Z], (const double *)g[P_Q], zn, Q, N);
-    const long nt = (long)zn * Q * tpk_sq(K);
+    const int nzq = zn * Q;
+    const dim3 gt(nblk(p->Tn, 256) * nblk(nzq, FSX_TMAT_ZQ));
     if (p->mixed)
-        hipLaunchKernelGGL(k_tmat<cplx32>, dim3(nblk(nt, 256)), dim3(256), 0, s, (float *)g[P_T],
-                           (const double *)g[P_BES], (const double *)g[P_DS], zn, Q, L);
+        hipLaunchKernelGGL(k_tmat<float>, gt, dim3(256), 0, s, (float *)g[P_T], (const double *)g[P_BES],
+                           (const double *)g[P_DS], ent + FSX_E_TB(p), nzq, L, p->Tn);
     else
-        hipLaunchKernelGGL(k_tmat<cplx>, dim3(nblk(nt, 256)), dim3(256), 0, s, (double *)g[P_T],
-                           (const double *)g[P_BES], (const double *)g[P_DS], zn, Q, L);
+        hipLaunchKernelGGL(k_tmat<double>, gt, dim3(256), 0, s, (double *)g[P_T], (const double *)g[P_BES],
+                           (const double *)g[P_DS], ent + FSX_E_TB(p), nzq, L, p->Tn);
     HIPR(hipGetLastError());
     if (ev) HIPR(hipEventRecord(ev[1], s));
     /* rotated receptor and ligand coefficients, m-chunked */
@@ -3093,68 +2658,86 @@ static int plan_enqueue(fsx_plan *p, hipStream_t s, hipEvent_t *ev, int stages =
             void *out = side == 0 ? g[P_RT] : g[P_BT];
             hipLaunchKernelGGL(k_twiddle, dim3(nblk(ntw, 256)), dim3(256), 0, s, srct, src,
                                src + spf, (const double *)g[P_TWG], ng, Q, L, side);
-            const int npk = side == 0 ? p->npk : 0, lrot = side == 0 ? 1 : -1;
+            const int lrot = side == 0 ? 1 : -1;
+            fsx_tabmap M;
+            M.l = ent + FSX_E_L(p);
+            M.pass = ent + FSX_E_PASS(p);
+            M.off = ent + (side == 0 ? FSX_E_OFFR(p) : FSX_E_OFFB(p));
+            M.pad = ent + FSX_E_PADB(p);
+            M.off2 = ent + FSX_E_OFFB2(p);
+            M.pad2 = ent + FSX_E_PADB2(p);
+            M.rs = ent + (side == 0 ? FSX_E_RSR(p) : FSX_E_RSB(p));
+            M.coff = (const long *)g[P_COFF] + (side == 0 ? 0 : p->C);
+            M.lig = side;
+            M.npk = 2 * p->npk;
+            const int *mst = ent + FSX_E_MST(p);
+            const double *dw = (const double *)g[P_DW];
             if (p->rot_gt) {
                 const int gt = p->rot_gt;
-                const long nbr = (long)Q * 3 * nb * ((ng + gt - 1) / gt);
+                const dim3 nbr((unsigned)(((long)Q * nb * ((ng + gt - 1) / gt) + 7) / 8 * 24));
                 const size_t lds = (size_t)gt * p->ne * p->es;
-                const double *dw = (const double *)g[P_DW];
-                const int *en = (const int *)g[P_ENT];
-                const long *co = (const long *)g[P_COFF];
-                if (p->mixed && gt == 16)
-                    hipLaunchKernelGGL((k_rotate_mfma<cplx32, 16>), dim3((unsigned)nbr), dim3(256), lds, s,
-                                       (cplx32 *)out, (const cplx *)srct, dw, en, co, nb, ng, Q, L,
-                                       p->mlo, p->ne, npk, lrot);
-                else if (p->mixed)
-                    hipLaunchKernelGGL((k_rotate_mfma<cplx32, 8>), dim3((unsigned)nbr), dim3(256), lds, s,
-                                       (cplx32 *)out, (const cplx *)srct, dw, en, co, nb, ng, Q, L,
-                                       p->mlo, p->ne, npk, lrot);
-                else if (gt == 16)
-                    hipLaunchKernelGGL((k_rotate_mfma<cplx, 16>), dim3((unsigned)nbr), dim3(256), lds, s,
-                                       (cplx *)out, (const cplx *)srct, dw, en, co, nb, ng, Q, L,
-                                       p->mlo, p->ne, npk, lrot);
-                else
-                    hipLaunchKernelGGL((k_rotate_mfma<cplx, 8>), dim3((unsigned)nbr), dim3(256), lds, s,
-                                       (cplx *)out, (const cplx *)srct, dw, en, co, nb, ng, Q, L,
-                                       p->mlo, p->ne, npk, lrot);
+#define FSX_ROT(E, F, GT)                                                                      \
+    hipLaunchKernelGGL((k_rotate_mfma<E, GT>), nbr, dim3(256), lds, s, (F *)out,               \
+                       (const cplx *)srct, dw, mst, M, nb, ng, Q, L, p->mlo, p->ne, lrot)
+                if (p->mixed && gt == 16) FSX_ROT(cplx32, float, 16);
+                else if (p->mixed) FSX_ROT(cplx32, float, 8);
+                else if (gt == 16) FSX_ROT(cplx, double, 16);
+                else FSX_ROT(cplx, double, 8);
+#undef FSX_ROT
                 continue;
             }
-            if (p->mixed)
-                launch_rotate<cplx32>(s, out, g[P_RTMP], srct, nrot, lds_rot, nb, ng, Q, L, gc, C,
-                                      csz, cst, coff, p->mlo, npk, lrot, g);
-            else
-                launch_rotate<cplx>(s, out, g[P_RTMP], srct, nrot, lds_rot, nb, ng, Q, L, gc, C,
-                                    csz, cst, coff, p->mlo, npk, lrot, g);
+            /* 64-row tiles of FP32 tables, 32-row tiles of FP64 tables (33 KB of LDS) */
+            const int nte = (p->ne + 63) / 64;
+            if (p->mixed) {
+                hipLaunchKernelGGL(k_rotate<cplx32>, dim3((unsigned)nrot), dim3(256), lds_rot, s,
+                                   (cplx32 *)g[P_RTMP], (const cplx *)srct, dw, mst, nb, ng, Q, L, gc,
+                                   p->mlo, p->ne);
+                const int ntr = (nrows + 63) / 64;
+                hipLaunchKernelGGL((k_tab_transpose<cplx32, 64>), dim3((unsigned)((long)Q * 3 * nte * ntr)),
+                                   dim3(256), 0, s, (float *)out, (const cplx32 *)g[P_RTMP], p->ne, nrows,
+                                   nte, ntr, M, lrot);
+            } else {
+                hipLaunchKernelGGL(k_rotate<cplx>, dim3((unsigned)nrot), dim3(256), lds_rot, s,
+                                   (cplx *)g[P_RTMP], (const cplx *)srct, dw, mst, nb, ng, Q, L, gc,
+                                   p->mlo, p->ne);
+                const int ntr = (nrows + 31) / 32;
+                hipLaunchKernelGGL((k_tab_transpose<cplx, 32>), dim3((unsigned)((long)Q * 3 * nte * ntr)),
+                                   dim3(256), 0, s, (double *)out, (const cplx *)g[P_RTMP], p->ne, nrows,
+                                   nte, ntr, M, lrot);
+            }
         }
     }
     HIPR(hipGetLastError());
     if (ev) HIPR(hipEventRecord(ev[2], s));
-    /* bucket poses by (z, beta2, gamma2) */
-    hipLaunchKernelGGL(k_fill_int, dim3(nblk(nkeys, 256)), dim3(256), 0, s, counts, nkeys, 0);
-    hipLaunchKernelGGL(k_fill_int, dim3(nblk(nkeys, 256)), dim3(256), 0, s, fill, nkeys, 0);
-    hipLaunchKernelGGL(k_count, dim3(nblk(n, 256)), dim3(256), 0, s, p->dposes, n, zn, nb, p->na,
-                       ng, (int *)g[P_KEYS], (int2 *)g[P_INFO], counts);
-    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, (const int *)counts, (int)nkeys, offs);
+    /* poses sorted by (beta2, z, gamma2), and the cross-term units */
+    hipLaunchKernelGGL(k_init, dim3(nblk(2 * nkeys, 256)), dim3(256), 0, s, counts, 2 * nkeys, tail,
+                       (int *)g[P_NEXT], (int)p->fit_next0, (unsigned long long *)g[P_TALLY]);
+    hipLaunchKernelGGL(k_count, dim3(nblk(n, 256)), dim3(256), 0, s, p->dposes, n, zn, p->nb, p->na,
+                       ng, p->mirror, (int *)g[P_KEYS], (int2 *)g[P_INFO], counts);
+    hipLaunchKernelGGL(k_units, dim3(nblk((long)p->nb * zn, 4)), dim3(256), 0, s, (const int *)counts,
+                       p->nb * zn, p->nb, zn, ng, p->urows, offs, (fsx_unit *)g[P_UNITS], tail);
     hipLaunchKernelGGL(k_scatter, dim3(nblk(n, 256)), dim3(256), 0, s, (const int *)g[P_KEYS],
-                       (const int2 *)g[P_INFO], n, ng, (const int *)offs, fill, (int4 *)g[P_RECS]);
+                       (const int2 *)g[P_INFO], n, ng, (const int *)offs, counts + nkeys,
+                       (int4 *)g[P_RECS]);
     HIPR(hipGetLastError());
     if (ev) HIPR(hipEventRecord(ev[3], s));
     }
     /* per-pose cross terms, one launch per m-chunk, accumulated in order */
     if (stages & FSX_ST_CROSS) {
-    const long grid = (long)g_ncu * env_int("FSX_CROSS_BLOCKS_PER_CU", 0, 0, 16);
-    if (p->mixed)
-        launch_cross<cplx32>(s, C, csz, cst, coff, p->Tn, grid, nrows, Q, L, nb, p->npk, ng, zn, g,
-                             p->tile_rows);
-    else
-        launch_cross<cplx>(s, C, csz, cst, coff, p->Tn, grid, nrows, Q, L, nb, p->npk, ng, zn, g,
-                           p->tile_rows);
-    HIPR(hipGetLastError());
+    for (int c = 0; c < p->C; c++) {
+        const int ns = p->ent[FSX_E_RSR(p) + c] / 6;
+        const void *kern = cross_kernel_of(p->mixed, cross_jn(ns), 0);
+        const size_t lds = cross_lds_of(p->mixed, ns, p->urows);
+        /* no more blocks than (q, unit) items can be */
+        long grid = cross_grid(kern, lds);
+        if (grid > (long)n * Q) grid = ((long)n * Q + g_nxcd - 1) / g_nxcd * g_nxcd;
+        fsx_cross_job jb = cross_job(p, c, grid);
+        void *args[1] = {&jb};
+        HIPR(hipLaunchKernel(kern, dim3((unsigned)grid), dim3(FSX_CROSS_BLOCK), args, lds, s));
+    }
     if (ev) HIPR(hipEventRecord(ev[4], s));
     }
     if (stages & FSX_ST_FITPREP) {
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, s, (int *)g[P_NEXT], 1L, (int)p->fit_next0);
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, s, (int *)g[P_TALLY], 2L * FSX_TALLY_N, 0);
     /* rescaled profiles in place of the pose parts (bounded by n slots;
      * the kernels read the number of valid slots on the device) */
     hipLaunchKernelGGL(k_fit_scale, dim3(nblk(n, 256)), dim3(256), 0, s, (const double *)g[P_ACC],
@@ -3213,7 +2796,7 @@ static int plan_download(fsx_plan *p, hipStream_t s, int *tail, unsigned long lo
 static void plan_stats(const fsx_plan *p, fsx_stats *st, const float *ms, const int *tail,
                        const unsigned long long *tally)
 {
-    const int K = p->K, K2 = p->K2, Q = p->Q, ne = p->ne, npk = p->npk, C = p->C;
+    const int K = p->K, Q = p->Q, ne = p->ne, npk = p->npk, C = p->C;
     const int nvalid = tail[0];
     const long items = (long)Q * tail[1];
     if (ms) {
@@ -3237,7 +2820,10 @@ static void plan_stats(const fsx_plan *p, fsx_stats *st, const float *ms, const 
      * terms per item) and 54 per (pose, q, pairing slot); the npk packed
      * slots carry two m = 0 entries whose other halves are zero */
     double tpair = 0.0;
-    for (int e = 0; e < ne; e++) tpair += K - (p->ent[K2 + e] < 0 ? -p->ent[K2 + e] : p->ent[K2 + e]);
+    for (int m = p->mlo; m <= p->L; m++) {
+        const double Km = K - (m < 0 ? -m : m);
+        tpair += Km * Km;
+    }
     const double nslot = (double)(ne - npk);
     st->cross_flops = (double)items * 3.0 * 8.0 * tpair + (double)nvalid * Q * nslot * 54.0;
     /* algorithmic bytes: per pose and q one receptor row (3 parts, one
@@ -3247,11 +2833,6 @@ static void plan_stats(const fsx_plan *p, fsx_stats *st, const float *ms, const 
                     + (double)items * 3.0 * ne * (double)p->es;
     st->cross_entries = ne;
 }
-
-static_assert(G_T == P_T && G_RT == P_RT && G_BT == P_BT && G_DW == P_DW && G_COUNTS == P_COUNTS &&
-                  G_OFFS == P_OFFS && G_RECS == P_RECS && G_ACC == P_ACC && G_ENT == P_ENT &&
-                  G_TW2 == P_TW2 && G_COFF == P_COFF,
-              "plan buffer indices of the launch helpers");
 
 /* single calls: the process-wide buffer slots */
 static int get_slot(int i, size_t bytes, void *ctx, void **out)
@@ -3343,10 +2924,10 @@ static fsx_bset g_bstr[FSX_BSTREAMS];
 static inline int per_stream_buffer(int i, int persist)
 {
     switch (i) {
-    case P_T: case P_RT: case P_BT: case P_COUNTS: case P_RECS: case P_ACC: case P_NEXT:
+    case P_T: case P_RT: case P_BT: case P_UNITS: case P_RECS: case P_ACC: case P_NEXT:
     case P_ACCF:
         return !persist;
-    case P_BES: case P_RTMP: case P_KEYS: case P_INFO: case P_FILL: case P_FITSC: case P_SRCT:
+    case P_BES: case P_RTMP: case P_KEYS: case P_INFO: case P_COUNTS: case P_FITSC: case P_SRCT:
         return 1;
     default:
         return 0;
@@ -3366,7 +2947,7 @@ static size_t g_gkey_len = 0;
 
 /* the launch parameters a captured graph depends on, per complex */
 struct fsx_gkey {
-    int L, nb, na, ng, Q, zn, n, flags, half, npk, C, tile_rows, aq_lds;
+    int L, nb, na, ng, Q, zn, n, flags, half, npk, C, urows, mirror, tile_rows, aq_lds;
     long lanes;
     double mult, peak, c1_lo, c1_hi, c2_lo, c2_hi;
     void *d[P_NBUF];
@@ -3551,21 +3132,38 @@ static int tune_one(const fsx_hip_args *A)
 }
 
 
-/* the cross-term jobs of plan p appended to the groups (the tile rows of
- * launch_cross) */
+/* the cross-term chunks of plan p appended to the groups (grown as needed);
+ * nx is set at launch */
 static int plan_cross_collect(const fsx_plan *p, fsx_cross_group **gr, int *ngr)
 {
-    const int G = p->tile_rows > 0 ? p->tile_rows
-                                   : env_int("FSX_CROSS_ROWS", p->mixed ? 4 : 2, 1, 4);
-    const int *csz = p->ent + 4 * p->K2, *cst = p->ent + 6 * p->K2;
-    void *const *g = p->d;
-#define FSX_COLLECT(E, GG)                                                                   \
-    cross_collect_g<E, GG>(gr, ngr, p->C, csz, cst, p->coff, p->Tn, p->nrows, p->Q, p->L,    \
-                           p->nb, p->npk, p->ng, p->zn, g)
-    if (p->mixed) return G >= 4 ? FSX_COLLECT(cplx32, 4) : G >= 2 ? FSX_COLLECT(cplx32, 2)
-                                                                : FSX_COLLECT(cplx32, 1);
-    return G >= 4 ? FSX_COLLECT(cplx, 4) : G >= 2 ? FSX_COLLECT(cplx, 2) : FSX_COLLECT(cplx, 1);
-#undef FSX_COLLECT
+    for (int c = 0; c < p->C; c++) {
+        const int ns = p->ent[FSX_E_RSR(p) + c] / 6;
+        const size_t lds = cross_lds_of(p->mixed, ns, p->urows);
+        const int jn = cross_jn(ns);
+        fsx_cross_group *t = NULL;
+        for (int i = 0; i < *ngr; i++) {
+            fsx_cross_group *u = &(*gr)[i];
+            if (u->mixed == p->mixed && u->jn == jn && u->chunk == c) t = u;
+        }
+        if (!t) {
+            fsx_cross_group *ng2 = (fsx_cross_group *)realloc(*gr, sizeof(fsx_cross_group) * (*ngr + 1));
+            if (!ng2) return FSX_ERR_NOMEM;
+            *gr = ng2;
+            t = &(*gr)[(*ngr)++];
+            memset(t, 0, sizeof(*t));
+            t->mixed = p->mixed; t->jn = jn; t->chunk = c;
+        }
+        if (t->njobs == t->cap) {
+            const int cap = t->cap ? 2 * t->cap : 8;
+            fsx_cross_job *nj = (fsx_cross_job *)realloc(t->jobs, sizeof(fsx_cross_job) * cap);
+            if (!nj) return FSX_ERR_NOMEM;
+            t->jobs = nj;
+            t->cap = cap;
+        }
+        if (lds > t->lds) t->lds = lds;
+        t->jobs[t->njobs++] = cross_job(p, c, 1);
+    }
+    return FSX_OK;
 }
 
 static int grow_dev(void **buf, size_t *cap, size_t bytes)
@@ -3680,21 +3278,9 @@ static int run_batch_locked(int nprob, const fsx_hip_args *args, fsx_stats *st)
             }
         size_t ntot = 0;
         for (int i = 0; i < ncg; i++) ntot += cg[i].njobs;
-        const long bpc_env = env_int("FSX_CROSS_BLOCKS_PER_CU", 0, 0, 16);
-        const int xcd = env_int("FSX_CROSS_XCD", 1, 0, 1);
         for (int i = 0; rc == FSX_OK && i < ncg; i++) {
-            int per = (int)bpc_env;
-            if (per == 0 && (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                                 &per, cross_group_kernel(&cg[i]), FSX_CROSS_BLOCK, cg[i].lds) !=
-                                 hipSuccess ||
-                             per < 1))
-                per = 2;
-            const long gsz = (long)g_ncu * per;
-            for (int j = 0; j < cg[i].njobs; j++) {
-                fsx_cross_job *jb = &cg[i].jobs[j];
-                jb->nx = xcd && g_nxcd > 1 && gsz % g_nxcd == 0 && jb->ntiles >= 4L * gsz ? g_nxcd : 1;
-            }
-            cg[i].grid = gsz;
+            cg[i].grid = cross_grid(cross_kernel_of(cg[i].mixed, cg[i].jn, 1), cg[i].lds);
+            for (int j = 0; j < cg[i].njobs; j++) cg[i].jobs[j].nx = cross_nx(cg[i].grid);
         }
         if (rc == FSX_OK) rc = grow_dev((void **)&g_cjob_dev, &g_cjob_cap,
                                         sizeof(fsx_cross_job) * (ntot > 0 ? ntot : 1));
@@ -3756,6 +3342,7 @@ static int run_batch_locked(int nprob, const fsx_hip_args *args, fsx_stats *st)
         const fsx_plan *p = &pl[k];
         ky->L = p->L; ky->nb = p->nb; ky->na = p->na; ky->ng = p->ng; ky->Q = p->Q; ky->zn = p->zn;
         ky->n = p->n; ky->flags = (int)A->flags; ky->half = p->half; ky->npk = p->npk; ky->C = p->C;
+        ky->urows = p->urows; ky->mirror = p->mirror;
         ky->tile_rows = p->tile_rows; ky->aq_lds = p->aq_lds; ky->lanes = p->lanes;
         ky->mult = A->mult; ky->peak = A->peak; ky->c1_lo = A->c1_lo; ky->c1_hi = A->c1_hi;
         ky->c2_lo = A->c2_lo; ky->c2_hi = A->c2_hi;
@@ -3808,8 +3395,9 @@ static int run_batch_locked(int nprob, const fsx_hip_args *args, fsx_stats *st)
                     const fsx_cross_job *jobs = g_cjob_dev + o;
                     int nj = cg[i].njobs;
                     void *kargs[2] = {(void *)&jobs, (void *)&nj};
-                    if (hipLaunchKernel(cross_group_kernel(&cg[i]), dim3((unsigned)cg[i].grid),
-                                        dim3(FSX_CROSS_BLOCK), kargs, cg[i].lds, g_stream) !=
+                    if (hipLaunchKernel(cross_kernel_of(cg[i].mixed, cg[i].jn, 1),
+                                        dim3((unsigned)cg[i].grid), dim3(FSX_CROSS_BLOCK), kargs,
+                                        cg[i].lds, g_stream) !=
                         hipSuccess)
                         rc = FSX_ERR_HIP;
                 }

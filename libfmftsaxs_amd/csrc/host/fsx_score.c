@@ -108,11 +108,32 @@ static const double *dw_table(int L, int nbeta, double pi, unsigned long long *k
     }
     if (hit < 0) {
         const size_t dsz = (size_t)(L + 1) * (2 * L + 1) * (2 * L + 1);
-        double *dW = (double *)malloc(sizeof(double) * dsz * nbeta);
-        if (!dW) return NULL;
+        size_t psz = 0;
+        for (int l = 0; l <= L; l++) psz += (size_t)((2 * l + 16) / 16) * ((2 * l + 4) / 4) * 64;
+        double *d = (double *)malloc(sizeof(double) * dsz);
+        double *dW = (double *)calloc(psz * nbeta, sizeof(double));
+        if (!d || !dW) {
+            free(d);
+            free(dW);
+            return NULL;
+        }
         /* fftsaxs.c:632-636, 706-708: beta_i = 0 + i * (pi - 0)/(nbeta - 1) */
         const double bstep = (pi - 0.0) / (nbeta - 1);
-        for (int b = 0; b < nbeta; b++) fsx_wigner_d(L, 0.0 + b * bstep, dW + b * dsz);
+        const int N = 2 * L + 1;
+        double *o = dW;
+        for (int b = 0; b < nbeta; b++) {
+            fsx_wigner_d(L, 0.0 + b * bstep, d);
+            /* in the order of the rotation's matrix products (fsx_internal.h) */
+            for (int l = 0; l <= L; l++) {
+                const int nks = (2 * l + 4) / 4, nmt = (2 * l + 16) / 16;
+                for (int r = 0; r <= 2 * l; r++)
+                    for (int k = 0; k <= 2 * l; k++)
+                        o[(r / 16 * nks + k / 4) * 64 + k % 4 * 16 + r % 16] =
+                            d[((size_t)l * N + (L + l - r)) * N + (L - l + k)];
+                o += (size_t)nmt * nks * 64;
+            }
+        }
+        free(d);
         hit = lru;
         free(g_dw[hit].dW);
         g_dw[hit].dW = dW;
@@ -182,7 +203,7 @@ static int prepare(const fsx_problem *pb, const int64_t *poses, int n, double *s
     a->a = pb->a; a->cint = h->cint; a->dW = dW; a->dsymb = ds; a->tw_a = h->twa; a->tw_g = h->twg;
     a->dw_key = dw_key;
     a->ds_key = (unsigned long long)L + 1;   /* the d-symbol table of L never changes */
-    a->mult = pb->mult; a->peak = pb->peak;
+    a->mult = pb->mult; a->peak = pb->peak; a->pi = pb->pi;
     a->c1_lo = pb->c1_lo; a->c1_hi = pb->c1_hi; a->c2_lo = pb->c2_lo; a->c2_hi = pb->c2_hi;
     a->poses = poses; a->n = n; a->score = score; a->c1 = c1; a->c2 = c2; a->cross = cross;
     a->flags = flags;
