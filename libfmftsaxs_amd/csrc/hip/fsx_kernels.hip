@@ -1142,7 +1142,7 @@ __global__ void __launch_bounds__(256)
 k_fit(const double *acc, const int4 *recs, const int *nvalid_p, int Q, const double *qvals,
       const double *a, double mult, double c1_lo, double c1_hi, double c2_lo, double c2_hi,
       double *score, double *c1o, double *c2o, int *next, unsigned long long *tally,
-      int wide_max)
+      int wide_max, int fpw)
 {
 #pragma clang fp contract(off)
     /* LDS: the K blocks [FSX_LB_KN][256], the wide evaluation's sums
@@ -1153,7 +1153,9 @@ k_fit(const double *acc, const int4 *recs, const int *nvalid_p, int Q, const dou
     extern __shared__ double sKf[];
     double *sW = sKf + FSX_LB_KN * FSX_LB_KSTRIDE + (threadIdx.x >> 6) * FSX_WIDE_SUMS * 64;
     const int nvalid = *nvalid_p;
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
+    /* each wavefront starts with fpw fits in its first lanes */
+    const int lane0 = threadIdx.x & 63;
+    int s = lane0 < fpw ? (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6) * fpw + lane0 : nvalid;
     fsx_fitpar fp;
     if (AQ_LDS) {
         double *sA = sKf + FSX_LB_KN * FSX_LB_KSTRIDE + 4 * FSX_WIDE_SUMS * 64;
@@ -1241,7 +1243,7 @@ k_fit(const double *acc, const int4 *recs, const int *nvalid_p, int Q, const dou
  * loop over q): four wavefronts per SIMD, against one for the
  * compact form's state (on the 210,000-pose L = 15 workload 1.50 ms,
  * against 1.60 ms at three wavefronts in 168 registers without spills).
- * With four lanes per fit (Q up to 64) a wavefront runs 16 fits, so the
+ * With four lanes per fit (many fits, Q up to 64) a wavefront runs 16 fits, so the
  * solver's divergent code is shared by many fits while the evaluation of
  * each is split four ways (at three wavefronts per SIMD: 1.64 ms, against
  * 1.83 ms with two lanes and 1.87 ms with eight).  The moments, q and the
@@ -2043,7 +2045,7 @@ static inline bool plan_packed(int i)
 
 typedef void (*fit_kernel_t)(const double *, const int4 *, const int *, int, const double *,
                              const double *, double, double, double, double, double, double *,
-                             double *, double *, int *, unsigned long long *, int);
+                             double *, double *, int *, unsigned long long *, int, int);
 
 struct fsx_plan {
     fsx_hip_args A;
@@ -2069,6 +2071,7 @@ struct fsx_plan {
     int fit_wide;        /* lanes with a fit at or below which a fit wavefront
                             evaluates them together (L-BFGS-B fits); lanes per
                             fit (Newton fits) */
+    int fit_fpw;         /* fits a wavefront starts with (L-BFGS-B fits) */
     long fit_next0;      /* first queue entry not taken at launch */
     int tile_rows;       /* gamma2 rows per cross-term tile (0: the form's default) */
     int rot_gt;          /* gamma per block of the MFMA rotation (16 or 8), 0: the
@@ -2401,10 +2404,14 @@ static int plan_init(fsx_plan *p, const fsx_hip_args *A, int tile_rows, int slot
      * not fit the block's LDS) the compact-form L-BFGS-B lane per fit, both
      * evaluated in one pass over q; the FP64 form: the reference's
      * L-BFGS-B, lane per fit.  Lanes per fit of the group fit: about
-     * FSX_FG_QLANE q per lane, at least two (FSX_FIT_GROUP_LANES
-     * overrides), doubled until the block's LDS fits */
+     * FSX_FG_QLANE q per lane, at least two, twice that where the lanes
+     * resident at once still take all fits (2,000 fits of 31 q 0.37 ms with 4
+     * lanes, 0.21 with 8, 0.26 with 16; 20,000 of 51 q 0.27, 0.23, 0.28;
+     * 210,000 0.60, 0.68, 0.94) (FSX_FIT_GROUP_LANES overrides), doubled until
+     * the block's LDS fits */
     int fpl = 2;
     while (fpl < FSX_WAVE && fpl * FSX_FG_QLANE < Q) fpl *= 2;
+    if (fpl < FSX_WAVE && 2L * fpl * n <= 256L * FSX_FG_WAVES * g_ncu) fpl *= 2;
     fpl = env_int("FSX_FIT_GROUP_LANES", fpl, 1, FSX_WAVE);
     while (fpl & (fpl - 1)) fpl &= fpl - 1;   /* a power of two */
     while (fpl < FSX_WAVE && fitg_lds(Q, fpl) > FSX_FIT_LDS) fpl *= 2;
@@ -2435,8 +2442,14 @@ static int plan_init(fsx_plan *p, const fsx_hip_args *A, int tile_rows, int slot
     p->lanes = (long)g_ncu * 256 * fit_bpc;
     const int fit_blocks = env_int("FSX_FIT_BLOCKS", 0, 0, 1 << 20);
     if (fit_blocks > 0) p->lanes = 256L * fit_blocks;
-    if (p->lanes > n) p->lanes = ((long)n + 255) / 256 * 256;
-    p->fit_next0 = p->lanes;
+    /* fewer fits than lanes are spread evenly over the wavefronts, for the wide
+     * evaluation to take them from the start and the steps' divergent code to
+     * run for few (52 fits 0.44 to 0.18 ms, 2,000 fits 0.67 to 0.31) */
+    const long nw = p->lanes / FSX_WAVE;
+    p->fit_fpw = n < p->lanes && p->fit_wide > 0 ? (int)((n + nw - 1) / nw) : FSX_WAVE;
+    if (p->fit_fpw < 1) p->fit_fpw = 1;
+    if (p->lanes > n) p->lanes = ((long)(n + p->fit_fpw - 1) / p->fit_fpw * FSX_WAVE + 255) / 256 * 256;
+    p->fit_next0 = p->lanes / FSX_WAVE * p->fit_fpw;
     return FSX_OK;
 }
 
@@ -2764,7 +2777,7 @@ static int plan_enqueue(fsx_plan *p, hipStream_t s, hipEvent_t *ev, int stages =
                            (const int *)(offs + nkeys), Q, (const double *)g[P_Q],
                            (const double *)g[P_AM], A->mult, A->c1_lo, A->c1_hi, A->c2_lo,
                            A->c2_hi, p->dscore, p->dc1, p->dc2, (int *)g[P_NEXT],
-                           (unsigned long long *)g[P_TALLY], p->fit_wide);
+                           (unsigned long long *)g[P_TALLY], p->fit_wide, p->fit_fpw);
     HIPR(hipGetLastError());
     if (ev) HIPR(hipEventRecord(ev[6], s));
     }
