@@ -1463,160 +1463,265 @@ k_fit_batch(const double *ct, int n, const double *qvals, int Q, const double *a
  *   k_atom_geom   r, f^X and conj(Y_lm) (m >= 0) per atom, the reference's
  *                 angles (cart2sph), norms and Legendre recurrence
  *                 (borrowed.c:19-65), contraction off
- *   k_atom_bes    J[l][atom][q] = j_l(q r) by the reference's series, q padded
- *                 to a multiple of 16 with zeros
- *   k_atom_mfma   per (chunk of 1024 atoms, l, 16 q): the sums over the chunk's
+ *   k_atom_bes    J[l][q][atom] = j_l(q r) by the reference's series
+ *   k_atom_mfma   per (chunk of 1024 atoms, l, up to 4 column and 3 q tiles of
+ *                 16): the sums over the chunk's
  *                 atoms as FP64 MFMA products of the (q x atoms) Bessel tile and
  *                 the (atoms x (X, m, re/im)) tile f^X conj(Y_lm); four waves
  *                 take 256 atoms each and are summed in LDS in a fixed order;
  *                 one partial per chunk
  * then k_atom_finish sums the chunks in order and applies 4 pi i^l. */
 #define FSX_AT_CHUNK 1024   /* atoms per k_atom_mfma block (4 waves x 256) */
-#define FSX_AT_MAXT 16      /* column tiles: 3 * 2 (L + 1) <= 16 * 16 for L <= 41 */
+#define FSX_AT_MAXT 16      /* most column tiles of an l: 3 * 2 (L + 1) <= 16 * 16 for L <= 41 */
 
-__global__ void k_atom_geom(const double *xyz, const double *vac, const double *dum,
-                            const double *sa, double h2o_ff, int na, int L, double pi_ref,
-                            double *r_out, double *f_out, double *Y)
+/* A thread per (atom, m), the m of an atom side by side so that the entries of
+ * an l go out together (a thread per atom filled 39 CUs with 10,000 atoms: 176 us
+ * at L = 25, 52 now). */
+__global__ void __launch_bounds__(256)
+k_atom_geom(const double *xyz, const double *vac, const double *dum, const double *sa, double h2o_ff,
+            int na, int L, double pi_ref, double *r_out, double *f_out, double *Y)
 {
 #pragma clang fp contract(off)
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= na) return;
     const int N = L + 1, Kh = N * (N + 1) / 2;
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int a = (int)(i / N), m = (int)(i - (long)a * N);
+    if (a >= na) return;
     /* cart2sph (pdb2spf.c:9-22) */
-    const double x = xyz[3 * a], y = xyz[3 * a + 1], z = xyz[3 * a + 2];
+    const double x = xyz[3 * (size_t)a], y = xyz[3 * (size_t)a + 1], z = xyz[3 * (size_t)a + 2];
     const double rr = sqrt(x * x + y * y + z * z);
     const double th = acos(z / rr);
     double fi;
     if (y > 0.0) fi = acos(x / sqrt(x * x + y * y));
     else fi = -acos(x / sqrt(x * x + y * y)) + 2.0 * pi_ref;
-    r_out[a] = rr;
-    f_out[a] = vac[a];
-    f_out[na + a] = dum[a];
-    f_out[2 * na + a] = sa ? h2o_ff * sa[a] : 0.0;
+    if (m == 0) {
+        r_out[a] = rr;
+        f_out[a] = vac[a];
+        f_out[na + a] = dum[a];
+        f_out[2 * na + a] = sa ? h2o_ff * sa[a] : 0.0;
+    }
     /* associated Legendre values (borrowed.c:40-65), written as conj(Y_lm)
      * = yn(l, m) P_l^m (cos m phi, sin(-m phi)) as soon as each is formed;
      * yn(l, m) = sqrt((2l + 1) / (4 pi) / prod_{k=1..m} (l - k + 1)(l + k))
      * (borrowed.c:19-38) */
     double *Ya = Y + (size_t)a * Kh * 2;
     const double xc = cos(th), yc = sqrt(1. - xc * xc);
-    auto put = [&](int l, int m, double P) {
+    const double cm = cos(fi * m), sm = sin(-fi * m);
+    /* the diagonal, then upwards in l */
+    double pmm = 1.0;
+    for (int k = 1; k <= m; k++) pmm = -1. * (2. * k - 1.) * yc * pmm;
+    double q2 = 0.0, q1 = 0.0;
+    for (int l = 0; l < N; l++) {
+        if (l < m) continue;
+        const double p = l == m ? pmm
+                       : l == m + 1 ? (2. * m + 1.) * xc * q1
+                                    : (2. * l - 1.) / (l - m) * xc * q1 - (l + m - 1.) / (l - m) * q2;
+        q2 = q1;
+        q1 = p;
         double f = 1.;
         const double base = (2 * l + 1.) / (4. * pi_ref);
         for (int k = 1; k <= m; k++) f *= (l - k + 1) * (l + k);
-        const double h = sqrt(base / f) * P;
+        const double h = sqrt(base / f) * p;
         const int e = l * (l + 1) / 2 + m;
-        Ya[2 * e] = h * cos(fi * m);
-        Ya[2 * e + 1] = h * sin(-fi * m);
-    };
-    /* m = 0 column */
-    double p2 = 1, p1 = xc;
-    put(0, 0, 1.0);
-    if (N > 1) put(1, 0, xc);
-    for (int l = 2; l < N; ++l) {
-        const double p = (2. * l - 1.) / l * xc * p1 - (l - 1.) / l * p2;
-        put(l, 0, p);
-        p2 = p1;
-        p1 = p;
+        Ya[2 * e] = h * cm;
+        Ya[2 * e + 1] = h * sm;
     }
-    /* m >= 1: the diagonal from the previous one, then upwards in l */
-    double pmm = 1.0;
-    for (int m = 1; m < N - 1; ++m) {
-        pmm = -1. * (2. * m - 1.) * yc * pmm;
-        put(m, m, pmm);
-        double q2 = pmm, q1 = (2. * m + 1.) * xc * pmm;
-        put(m + 1, m, q1);
-        for (int l = m + 2; l < N; ++l) {
-            const double p = (2. * l - 1.) / (l - m) * xc * q1 - (l + m - 1.) / (l - m) * q2;
-            put(l, m, p);
-            q2 = q1;
-            q1 = p;
+}
+
+/* The series of dev_sbessel for the threads of a block that share l, bit for bit
+ * and without its divisions: begin() tabulates the denominators d = 2k (2k + 2l +
+ * 1) and their rounded reciprocals y for k <= FSX_SB_TAB and 1 / (2l + 1)!!.
+ * - The quotient n / d: q = n y, and twice q += (n - d q) y with fused
+ *   multiply-adds.  The first leaves q within one unit in the last place, and
+ *   from such a q and a correctly rounded y the second gives the correctly
+ *   rounded quotient (Markstein 1990), 5 operations for the division's dozen.
+ *   A residual that underflows belongs to a ratio far below the sum's last bit.
+ * - The test |term / sum| > 1e-5: by products with margins a million times the
+ *   rounding error; the division decides only in between.
+ * Bound by the FP64 instructions of the terms (about 15 for each, up to 40 terms)
+ * and of x^l: 10,000 atoms, L = 25, 81 q 737 us with the divisions and q across the
+ * lanes, 350 now (60 G values/s). */
+#define FSX_SB_TAB 64
+struct sbessel_block {
+    double d[FSX_SB_TAB + 1], y[FSX_SB_TAB + 1], t0;
+    __device__ __forceinline__ void begin(int l)
+    {
+#pragma clang fp contract(off)
+        const int k = threadIdx.x;
+        const double tl1 = 2.0 * (double)l + 1.0;
+        if (k >= 1 && k <= FSX_SB_TAB) {
+            d[k] = 2.0 * (double)k * (2.0 * (double)k + tl1);
+            y[k] = 1.0 / d[k];
         }
+        if (k == 0) {
+            double f = 1.0;
+            for (int i = 1; i <= (int)tl1; i += 2) f *= (double)i;
+            t0 = 1.0 / f;
+        }
+        __syncthreads();
     }
-    if (N > 1) put(N - 1, N - 1, -1. * (2. * (N - 1.) - 1.) * yc * pmm);
-}
+    __device__ __forceinline__ double value(int l, double x) const
+    {
+#pragma clang fp contract(off)
+        if (!(x > 0.0)) return l == 0 ? 1.0 : 0.0;
+        const double tl1 = 2.0 * (double)l + 1.0, n = (-1.0) * x * x;
+        double term = t0, sum = t0;
+        for (int k = 1;; k++) {
+            const double at = fabs(term), as = fabs(sum);
+            if (!(at > fma(as, 0.00001 * (1.0 + 1e-9), 1e-290))) {
+                if (as > 1e-270 && at < as * (0.00001 * (1.0 - 1e-9))) break;
+                if (!(fabs(term / sum) > 0.00001)) break;
+            }
+            double ratio;
+            if (k <= FSX_SB_TAB) {
+                ratio = n * y[k];
+                ratio = fma(fma(-d[k], ratio, n), y[k], ratio);
+                ratio = fma(fma(-d[k], ratio, n), y[k], ratio);
+            } else {
+                ratio = n / (2.0 * (double)k * (2.0 * (double)k + tl1));
+            }
+            term *= ratio;
+            sum += term;
+        }
+        return sum * pow_int_cr(x, l);
+    }
+};
 
-/* J[l][a][q] = j_l(q r_a) for q < Q, 0 for Q <= q < Qp */
-__global__ void k_atom_bes(double *J, const double *r, const double *qvals, int na, int Q, int Qp,
-                           int K)
+/* J[l][q][a] = j_l(q r_a); nbl blocks per l.  A wavefront takes atoms of one q,
+ * whose series have about the same length (with q across the lanes all of them
+ * waited for the largest q: 532 against 350 us at 10,000 atoms, L = 25, 81 q). */
+__global__ void __launch_bounds__(256)
+k_atom_bes(double *J, const double *r, const double *qvals, int na, int Q, unsigned nbl)
 {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)K * na * Qp) return;
-    const int q = (int)(i % Qp);
-    const long la = i / Qp;
-    const int a = (int)(la % na), l = (int)(la / na);
-    J[i] = q < Q ? dev_sbessel(l, qvals[q] * r[a]) : 0.0;
+    __shared__ sbessel_block S;
+    const int l = (int)(blockIdx.x / nbl);
+    S.begin(l);
+    const long i = (long)(blockIdx.x % nbl) * blockDim.x + threadIdx.x, n = (long)na * Q;
+    if (i >= n) return;
+    const int q = (int)(i / na), a = (int)(i - (long)q * na);
+    J[l * n + i] = S.value(l, qvals[q] * r[a]);
 }
 
-/* One block of four waves per (chunk, l, 16-q tile).  Rows are q, columns
+/* One block of four waves per (chunk, l, up to FSX_AT_CT column tiles, up to
+ * FSX_AT_QT q tiles), tiles of 16.  Rows are q, columns
  * c = X * 2(l+1) + 2m + part (part 0: real, 1: imaginary) of f^X conj(Y_lm).
  * FP64 MFMA 16x16x4 operand layout on gfx950: lane i feeds A[i % 16][i / 16]
  * and B[i / 16][i % 16]; result register j of lane i is D[i / 16 + 4j][i % 16].
+ * A step's QT + 2 CT loads feed QT CT products, with the next step's in flight
+ * (with one q tile and every column tile in a block, f and Y were read for each
+ * q tile and waited for at each step: 539 us for 10,000 atoms, L = 25, 81 q,
+ * against 133 to 157; the products alone take 96 at their measured rate).
  * Writes the chunk's partial sums P[chunk][X][Qp][Kh][2]. */
-__global__ void __launch_bounds__(256)
-k_atom_mfma(const double *J, const double *f, const double *Y, double *P, int na, int Qp, int L,
+#define FSX_AT_QT 3
+#define FSX_AT_CT 4
+__host__ __device__ static inline int at_colgroups(int l)
+{
+    return (6 * (l + 1) + 16 * FSX_AT_CT - 1) / (16 * FSX_AT_CT);
+}
+__global__ void __launch_bounds__(256, 2)
+k_atom_mfma(const double *J, const double *f, const double *Y, double *P, int na, int Q, int Qp, int L,
             int chunk0)
 {
     __shared__ fsx_v4d red[3][64];
     const int K = L + 1, Kh = K * (K + 1) / 2, nqt = Qp / 16;
-    int bid = blockIdx.x;
-    const int qt = bid % nqt;
-    bid /= nqt;
-    const int l = bid % K;
-    const int ch = bid / K;
+    const int nqg = (nqt + FSX_AT_QT - 1) / FSX_AT_QT;
+    int bid = blockIdx.x, ncg = 0;
+    for (int l = 0; l <= L; l++) ncg += at_colgroups(l);
+    const int qt0 = bid % nqg * FSX_AT_QT;
+    bid /= nqg;
+    const int ch = bid / ncg;
+    /* the orders with the most columns first */
+    int cg = bid - ch * ncg, l = L;
+    while (cg >= at_colgroups(l)) cg -= at_colgroups(l--);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int ncol = 3 * 2 * (l + 1), nct = (ncol + 15) / 16;
-    /* this lane's column of each tile: X, entry offset and part */
-    int cx[FSX_AT_MAXT], coff[FSX_AT_MAXT];
+    const int ncol = 3 * 2 * (l + 1);
+    const int nq = min(FSX_AT_QT, nqt - qt0);
+    const int nc = min(FSX_AT_CT, (ncol + 15) / 16 - cg * FSX_AT_CT);
+    /* this lane's column of each tile: X (-1: none), entry offset and part */
+    int cx[FSX_AT_CT], coff[FSX_AT_CT];
 #pragma unroll
-    for (int t = 0; t < FSX_AT_MAXT; t++) {
-        const int c = t * 16 + (lane & 15);
+    for (int t = 0; t < FSX_AT_CT; t++) {
+        const int c = (cg * FSX_AT_CT + t) * 16 + (lane & 15);
         const int X = c / (2 * (l + 1)), rem = c - X * 2 * (l + 1);
         cx[t] = c < ncol ? X : -1;
         coff[t] = c < ncol ? l * (l + 1) / 2 * 2 + rem : 0;   /* (entry, part) as a double index */
     }
-    fsx_v4d acc[FSX_AT_MAXT];
+    fsx_v4d acc[FSX_AT_QT][FSX_AT_CT];
 #pragma unroll
-    for (int t = 0; t < FSX_AT_MAXT; t++) acc[t] = (fsx_v4d){0.0, 0.0, 0.0, 0.0};
+    for (int u = 0; u < FSX_AT_QT; u++)
+#pragma unroll
+        for (int t = 0; t < FSX_AT_CT; t++) acc[u][t] = (fsx_v4d){0.0, 0.0, 0.0, 0.0};
     const int abeg = ch * FSX_AT_CHUNK + w * (FSX_AT_CHUNK / 4);
     const int aend = min(abeg + FSX_AT_CHUNK / 4, na);
-    const double *Jl = J + (size_t)l * na * Qp + qt * 16 + (lane & 15);
-    for (int a0 = abeg; a0 < aend; a0 += 4) {
-        const int a = a0 + (lane >> 4);
-        const bool ok = a < aend;
-        const double av = ok ? Jl[(size_t)a * Qp] : 0.0;
-        const double *Ya = Y + (size_t)(ok ? a : 0) * Kh * 2;
+    /* rows past the last q repeat it; nothing reads their sums */
+    const double *Jl[FSX_AT_QT];
 #pragma unroll
-        for (int t = 0; t < FSX_AT_MAXT; t++) {
-            if (t < nct) {
-                const double bv = ok && cx[t] >= 0 ? f[(size_t)cx[t] * na + a] * Ya[coff[t]] : 0.0;
-                acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[t], 0, 0, 0);
+    for (int u = 0; u < FSX_AT_QT; u++)
+        Jl[u] = J + ((size_t)l * Q + min((qt0 + u) * 16 + (lane & 15), Q - 1)) * na;
+    struct ops {
+        double j[FSX_AT_QT], f[FSX_AT_CT], y[FSX_AT_CT];
+    } A, B;
+    /* unconditional, so that a wait for one step leaves the next one's loads in
+     * flight; what is read in place of no atom, tile or column is not used */
+    auto load = [&](ops &o, int a0) {
+        const int a = min(a0 + (lane >> 4), na - 1);
+        const double *Ya = Y + (size_t)a * Kh * 2;
+#pragma unroll
+        for (int u = 0; u < FSX_AT_QT; u++) o.j[u] = Jl[u][a];
+#pragma unroll
+        for (int t = 0; t < FSX_AT_CT; t++) {
+            o.f[t] = f[(size_t)max(cx[t], 0) * na + a];
+            o.y[t] = Ya[coff[t]];
+        }
+    };
+    auto run = [&](const ops &o, int a0) {
+        const bool ok = a0 + (lane >> 4) < aend;
+        double bv[FSX_AT_CT];
+#pragma unroll
+        for (int t = 0; t < FSX_AT_CT; t++) bv[t] = ok && cx[t] >= 0 ? o.f[t] * o.y[t] : 0.0;
+#pragma unroll
+        for (int u = 0; u < FSX_AT_QT; u++)
+            if (u < nq) {
+                const double av = ok ? o.j[u] : 0.0;
+#pragma unroll
+                for (int t = 0; t < FSX_AT_CT; t++)
+                    if (t < nc) acc[u][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv[t], acc[u][t], 0, 0, 0);
             }
+    };
+    if (abeg < aend) {
+        load(A, abeg);
+        for (int a0 = abeg;; a0 += 8) {
+            load(B, a0 + 4);
+            run(A, a0);
+            if (a0 + 4 >= aend) break;
+            load(A, a0 + 8);
+            run(B, a0 + 4);
+            if (a0 + 8 >= aend) break;
         }
     }
     /* wave 0 + wave 1 + wave 2 + wave 3, in that order, per tile */
-    const int q0 = qt * 16;
     double *Pc = P + (size_t)(chunk0 + ch) * 3 * Qp * Kh * 2;
 #pragma unroll
-    for (int t = 0; t < FSX_AT_MAXT; t++) {
-        if (t < nct) {
-            if (w > 0) red[w - 1][lane] = acc[t];
+    for (int u = 0; u < FSX_AT_QT; u++)
+#pragma unroll
+        for (int t = 0; t < FSX_AT_CT; t++) {
+            if (u >= nq || t >= nc) continue;
+            if (w > 0) red[w - 1][lane] = acc[u][t];
             __syncthreads();
             if (w == 0) {
-                fsx_v4d v = acc[t];
+                fsx_v4d v = acc[u][t];
                 v += red[0][lane];
                 v += red[1][lane];
                 v += red[2][lane];
                 if (cx[t] >= 0) {
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
-                        const int q = q0 + (lane >> 4) + 4 * j;
+                        const int q = (qt0 + u) * 16 + (lane >> 4) + 4 * j;
                         Pc[((size_t)cx[t] * Qp + q) * Kh * 2 + coff[t]] = v[j];
                     }
                 }
             }
             __syncthreads();
         }
-    }
 }
 
 /* ---- the atom expansion in split BF16 on MFMA (the mixed form) ----------
@@ -1645,13 +1750,16 @@ __device__ __forceinline__ void split3(double x, __bf16 &h, __bf16 &m, __bf16 &l
 __global__ void k_atom_bes_split(__bf16 *Js, const double *r, const double *qvals, int na, int nap,
                                  int Q, int Qp, int K)
 {
+    /* nap is a multiple of the block size, so a block has one (l, q) */
+    __shared__ sbessel_block S;
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long tot = (long)K * Qp * nap;
-    if (i >= tot) return;
     const int a = (int)(i % nap);
     const long lq = i / nap;
     const int q = (int)(lq % Qp), l = (int)(lq / Qp);
-    const double v = q < Q && a < na ? dev_sbessel(l, qvals[q] * r[a]) : 0.0;
+    S.begin(l);
+    if (i >= tot) return;
+    const double v = q < Q && a < na ? S.value(l, qvals[q] * r[a]) : 0.0;
     __bf16 h, m, lo;
     split3(v, h, m, lo);
     Js[i] = h;
@@ -3567,14 +3675,18 @@ static int atoms_run(hipStream_t s, char *ws, size_t ws_bytes, int natoms, const
     double *f = J + (size_t)K * npass * Qp, *r = f + 3 * (size_t)npass, *Y = r + npass;
     for (long a0 = 0; a0 < natoms; a0 += npass) {
         const int na = (int)(natoms - a0 < npass ? natoms - a0 : npass);
-        hipLaunchKernelGGL(k_atom_geom, dim3(nblk(na, 256)), dim3(256), 0, s, xyz + 3 * a0,
+        hipLaunchKernelGGL(k_atom_geom, dim3(nblk((long)na * K, 256)), dim3(256), 0, s, xyz + 3 * a0,
                            vac + a0, dum + a0, sa ? sa + a0 : (const double *)NULL, h2o_ff, na, L,
                            FSX_PI_REFERENCE, r, f, Y);
-        hipLaunchKernelGGL(k_atom_bes, dim3(nblk((long)K * na * Qp, 256)), dim3(256), 0, s, J,
-                           (const double *)r, qv, na, Q, Qp, K);
+        const unsigned nbl = nblk((long)na * Q, 256);
+        hipLaunchKernelGGL(k_atom_bes, dim3(nbl * K), dim3(256), 0, s, J, (const double *)r, qv, na, Q,
+                           nbl);
         const int nchp = (na + FSX_AT_CHUNK - 1) / FSX_AT_CHUNK;
-        hipLaunchKernelGGL(k_atom_mfma, dim3((unsigned)(nchp * K * (Qp / 16))), dim3(256), 0, s,
-                           (const double *)J, (const double *)f, (const double *)Y, P, na, Qp, L,
+        int ncg = 0;
+        for (int l = 0; l <= L; l++) ncg += at_colgroups(l);
+        const int nqg = (Qp / 16 + FSX_AT_QT - 1) / FSX_AT_QT;
+        hipLaunchKernelGGL(k_atom_mfma, dim3((unsigned)(nchp * ncg * nqg)), dim3(256), 0, s,
+                           (const double *)J, (const double *)f, (const double *)Y, P, na, Q, Qp, L,
                            (int)(a0 / FSX_AT_CHUNK));
     }
     hipLaunchKernelGGL(k_atom_finish, dim3(nblk(3L * Q * Kh, 256)), dim3(256), 0, s,
@@ -3605,7 +3717,7 @@ static int atoms_run_bf16(hipStream_t s, char *ws, size_t ws_bytes, int natoms,
     double *Y = r + natoms;
     __bf16 *Js = reinterpret_cast<__bf16 *>(Y + (size_t)natoms * Kh * 2);
     __bf16 *Bs = Js + 3 * (size_t)K * Qp * nap;
-    hipLaunchKernelGGL(k_atom_geom, dim3(nblk(natoms, 256)), dim3(256), 0, s, xyz, vac, dum, sa,
+    hipLaunchKernelGGL(k_atom_geom, dim3(nblk((long)natoms * K, 256)), dim3(256), 0, s, xyz, vac, dum, sa,
                        h2o_ff, natoms, L, FSX_PI_REFERENCE, r, f, Y);
     hipLaunchKernelGGL(k_atom_bes_split, dim3(nblk((long)K * Qp * nap, 256)), dim3(256), 0, s, Js,
                        (const double *)r, qv, natoms, nap, Q, Qp, K);
