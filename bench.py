@@ -83,7 +83,7 @@ def run_batch(args):
     log-uniform over 1e4..1e6; 51 q on [0, 0.5], z 25..60 A, 10 degree betas,
     64-point alpha/gamma grids; water shell from Shrake-Rupley SASA), scored
     by one fsx_score_batch call per step.  The first call of each form tunes
-    the cross-term tile rows per expansion-order bucket and captures the
+    the cross-term rows per unit, per expansion-order bucket and captures the
     batch into a HIP graph; the timed steps replay it."""
     import torch
     import libfmftsaxs_amd as F

@@ -9,8 +9,8 @@
  *                 ligand    B^Y_lm(b2,g2,q) = sum_m2 e^{-i m2 g2} d^l_{m m2}(b2) conj(B^Y_{l m2})
  *                 (the beta/gamma factors of compute_sum1/compute_sum2 and of the
  *                 3-D DFT, fftsaxs.c:251-333, 416-524, 680, folded per pose axis)
- *   k_count/k_scan/k_scatter   bucket poses by (z, beta2, gamma2)
- *   k_cross       per bucket and q: U^Y_lm = sum_l1 conj(T_{|m| l l1}) B^Y_{l1 m} in LDS,
+ *   k_count/k_units/k_scatter  bucket poses by (beta2, z, gamma2), units of buckets
+ *   k_cross       per unit and q (fsx_cross.h): U^Y_lm = sum_l1 conj(T_{|m| l l1}) B^Y_{l1 m} in LDS,
  *                 then per pose 2 Re sum_lm e^{-i m a2} (R^X U^Y [+ R^Y U^X]) for the six
  *                 cross terms VV,VD,VW,DD,DW,WW (fill_var, fftsaxs.c:87-108)
  *   k_fit         constant terms + peak rescale + bounded L-BFGS-B chi^2 fit per pose
@@ -529,12 +529,6 @@ k_rotate_mfma(decltype(E::re) *out, const cplx *srct, const double *dW, const in
 }
 
 /* ---- pose bucketing --------------------------------------------------- */
-__global__ void k_fill_int(int *p, long n, int v)
-{
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
 /* The counters of a call in one launch: bucket counts and fills (nc values)
  * and the record, bucket and unit counters zero, the fit queue at next0, the
  * fit tallies zero. */
@@ -595,56 +589,73 @@ __global__ void k_count(const long long *poses, int n, int znum, int nbeta, int 
 
 /* First record of every bucket and the cross-term units, one wavefront per
  * (beta2, z).  Units are cut greedily along gamma2: up to urows rows and
- * FSX_UPOSES poses; a bucket of more poses takes several.  The wavefronts
- * reserve their records and units with one atomic each (tail: records,
- * non-empty buckets, units), so the order of the (beta2, z) groups is only
- * approximately ascending; every pose's result is the same in any order.
- * One launch, against a scan by a single block whose time grew with the
- * number of buckets (828 us at 478,000 buckets). */
+ * FSX_UPOSES poses; a bucket of more poses takes several.  PASS 0 counts every
+ * group's records and units (grp), PASS 1 adds those of the groups before and
+ * writes; tail: records, non-empty buckets, units.  The units are in the order of
+ * the groups: with ranges reserved by atomics, in the order the wavefronts came,
+ * an XCD's blocks worked on all beta2 at a time and its L2 lost the ligand rows (cross
+ * terms FP64 L = 15, 210,000 poses 9.76 against 9.27 ms; L = 25, 200,000 poses 156
+ * against 146, FP32 300,000 poses 65.5 against 61.7).
+ * Against a scan by a single block, whose time grew with the number of buckets (828 us
+ * at 478,000). */
+template <int PASS>
 __global__ void __launch_bounds__(256)
-k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int *offs, fsx_unit *units, int *tail)
+k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int *offs, fsx_unit *units,
+        int *tail, int2 *grp)
 {
     const int zb = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (zb >= nzb) return;
     const int *c = counts + (size_t)zb * ng, cap = FSX_UPOSES;
-    int total = 0, nz = 0, nu = 0, first = 0;
-    /* pass 0 counts the units, pass 1 writes them */
-    for (int pass = 0; pass < 2; pass++) {
-        int p = 0, un = 0, ur = 0, uc = 0;   /* records so far; open unit's poses and rows; units */
-        fsx_unit u;
-        u.b2 = zb / zn % nb;
-        u.z = zb % zn;
-        u.pad = 0;
-        for (int g0 = 0; g0 < ng; g0 += 64) {
-            const int v = g0 + lane < ng ? c[g0 + lane] : 0;
-            if (pass) {
-                /* exclusive scan over the 64 buckets */
-                int x = v;
+    int total = 0, first = 0;
+    if (PASS) {
+        for (int k = lane; k < zb; k += 64) {
+            total += grp[k].x;
+            first += grp[k].y;
+        }
 #pragma unroll
-                for (int o = 1; o < 64; o <<= 1) {
-                    const int y = __shfl_up(x, o);
-                    if (lane >= o) x += y;
-                }
-                if (g0 + lane < ng) offs[(size_t)zb * ng + g0 + lane] = total + p + x - v;
+        for (int o = 1; o < 64; o <<= 1) {
+            total += __shfl_xor(total, o);
+            first += __shfl_xor(first, o);
+        }
+        total = __builtin_amdgcn_readfirstlane(total);
+        first = __builtin_amdgcn_readfirstlane(first);
+    }
+    int p = 0, nz = 0, un = 0, ur = 0, uc = 0;   /* records so far, buckets; open unit's poses and rows; units */
+    fsx_unit u;
+    u.b2 = zb / zn % nb;
+    u.z = zb % zn;
+    u.pad = 0;
+    for (int g0 = 0; g0 < ng; g0 += 64) {
+        const int v = g0 + lane < ng ? c[g0 + lane] : 0;
+        if (PASS) {
+            /* exclusive scan over the 64 buckets */
+            int x = v;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(x, o);
+                if (lane >= o) x += y;
             }
-            unsigned long long mask = __ballot(v > 0);
-            if (!pass) nz += __popcll(mask);
-            while (mask) {
-                const int b = __builtin_ctzll(mask);
-                mask &= mask - 1;
-                int left = __builtin_amdgcn_readlane(v, b);
-                while (left > 0) {
-                    /* close the open unit where the row does not fit in it */
-                    if (un > 0 && (ur == urows || un + left > cap)) {
-                        if (pass && lane == 0) {
-                            u.n = un;
-                            u.nrow = ur;
-                            units[first + uc] = u;
-                        }
-                        uc++;
-                        un = ur = 0;
+            if (g0 + lane < ng) offs[(size_t)zb * ng + g0 + lane] = total + p + x - v;
+        }
+        unsigned long long mask = __ballot(v > 0);
+        nz += __popcll(mask);
+        while (mask) {
+            const int b = __builtin_ctzll(mask);
+            mask &= mask - 1;
+            int left = __builtin_amdgcn_readlane(v, b);
+            while (left > 0) {
+                /* close the open unit where the row does not fit in it */
+                if (un > 0 && (ur == urows || un + left > cap)) {
+                    if (PASS && lane == 0) {
+                        u.n = un;
+                        u.nrow = ur;
+                        units[first + uc] = u;
                     }
-                    const int k = left < cap - un ? left : cap - un;
+                    uc++;
+                    un = ur = 0;
+                }
+                const int k = left < cap - un ? left : cap - un;
+                if (PASS) {
                     if (un == 0) u.p0 = total + p;
 #pragma unroll
                     for (int r = 0; r < FSX_UROWS; r++)
@@ -655,34 +666,30 @@ k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int *offs
                         } else if (r > ur) {
                             u.g2[r] = u.g2[0];
                         }
-                    ur++;
-                    un += k;
-                    p += k;
-                    left -= k;
                 }
+                ur++;
+                un += k;
+                p += k;
+                left -= k;
             }
-        }
-        if (un > 0) {
-            if (pass && lane == 0) {
-                u.n = un;
-                u.nrow = ur;
-                units[first + uc] = u;
-            }
-            uc++;
-        }
-        if (!pass) {
-            int a = 0, b = 0;
-            if (lane == 0 && p > 0) {
-                a = atomicAdd(&tail[0], p);
-                atomicAdd(&tail[1], nz);
-                b = atomicAdd(&tail[2], uc);
-            }
-            total = __builtin_amdgcn_readlane(a, 0);
-            first = __builtin_amdgcn_readlane(b, 0);
-            nu = uc;
         }
     }
-    (void)nu;
+    if (un > 0) {
+        if (PASS && lane == 0) {
+            u.n = un;
+            u.nrow = ur;
+            units[first + uc] = u;
+        }
+        uc++;
+    }
+    if (!PASS && lane == 0) {
+        grp[zb] = make_int2(p, uc);
+        if (p > 0) {
+            atomicAdd(&tail[0], p);
+            atomicAdd(&tail[1], nz);
+            atomicAdd(&tail[2], uc);
+        }
+    }
 }
 
 /* sorted pose records: x = input position, y = receptor row, z = alpha index,
@@ -2178,10 +2185,10 @@ struct fsx_plan {
     int grp;             /* the lane-group fit k_fitg (mixed form) */
     int fit_wide;        /* lanes with a fit at or below which a fit wavefront
                             evaluates them together (L-BFGS-B fits); lanes per
-                            fit (Newton fits) */
+                            fit (lane groups) */
     int fit_fpw;         /* fits a wavefront starts with (L-BFGS-B fits) */
     long fit_next0;      /* first queue entry not taken at launch */
-    int tile_rows;       /* gamma2 rows per cross-term tile (0: the form's default) */
+    int tile_rows;       /* pairs of gamma2 rows per unit (0: as many as fit) */
     int rot_gt;          /* gamma per block of the MFMA rotation (16 or 8), 0: the
                             rotation-then-transpose kernels */
 };
@@ -2482,7 +2489,8 @@ static int plan_init(fsx_plan *p, const fsx_hip_args *A, int tile_rows, int slot
     z[P_KEYS] = sizeof(int) * n;
     z[P_INFO] = sizeof(int2) * n;
     z[P_COUNTS] = sizeof(int) * 2 * p->nkeys;   /* counts, then fills */
-    z[P_OFFS] = sizeof(int) * (p->nkeys + 3);   /* then records, buckets, units */
+    /* then records, buckets, units; then those of each (beta2, z) */
+    z[P_OFFS] = sizeof(int) * (p->nkeys + 4) + sizeof(int2) * (size_t)nb * zn;
     z[P_UNITS] = sizeof(fsx_unit) * (size_t)n;
     z[P_RECS] = sizeof(int4) * n;
     z[P_ACC] = sizeof(double) * 6 * Q * (size_t)n;
@@ -2835,8 +2843,11 @@ static int plan_enqueue(fsx_plan *p, hipStream_t s, hipEvent_t *ev, int stages =
                        (int *)g[P_NEXT], (int)p->fit_next0, (unsigned long long *)g[P_TALLY]);
     hipLaunchKernelGGL(k_count, dim3(nblk(n, 256)), dim3(256), 0, s, p->dposes, n, zn, p->nb, p->na,
                        ng, p->mirror, (int *)g[P_KEYS], (int2 *)g[P_INFO], counts);
-    hipLaunchKernelGGL(k_units, dim3(nblk((long)p->nb * zn, 4)), dim3(256), 0, s, (const int *)counts,
-                       p->nb * zn, p->nb, zn, ng, p->urows, offs, (fsx_unit *)g[P_UNITS], tail);
+    int2 *grp = (int2 *)(offs + ((nkeys + 4) & ~1L));
+    hipLaunchKernelGGL(k_units<0>, dim3(nblk((long)p->nb * zn, 4)), dim3(256), 0, s, (const int *)counts,
+                       p->nb * zn, p->nb, zn, ng, p->urows, offs, (fsx_unit *)g[P_UNITS], tail, grp);
+    hipLaunchKernelGGL(k_units<1>, dim3(nblk((long)p->nb * zn, 4)), dim3(256), 0, s, (const int *)counts,
+                       p->nb * zn, p->nb, zn, ng, p->urows, offs, (fsx_unit *)g[P_UNITS], tail, grp);
     hipLaunchKernelGGL(k_scatter, dim3(nblk(n, 256)), dim3(256), 0, s, (const int *)g[P_KEYS],
                        (const int2 *)g[P_INFO], n, ng, (const int *)offs, counts + nkeys,
                        (int4 *)g[P_RECS]);
@@ -3068,7 +3079,8 @@ static size_t g_gkey_len = 0;
 
 /* the launch parameters a captured graph depends on, per complex */
 struct fsx_gkey {
-    int L, nb, na, ng, Q, zn, n, flags, half, npk, C, urows, mirror, tile_rows, aq_lds;
+    int L, nb, na, ng, Q, zn, n, flags, half, npk, C, urows, mirror, tile_rows, aq_lds,
+        fit_wide, fit_fpw;
     long lanes;
     double mult, peak, c1_lo, c1_hi, c2_lo, c2_hi;
     void *d[P_NBUF];
@@ -3123,8 +3135,8 @@ static int get_bat(int i, size_t bytes, void *ctx, void **out)
 
 /* ---- tile-shape tuner ----
  * Per expansion-order bucket (L <= 10, 15, 20, 25, 30, 40) and form, the
- * gamma2 rows per cross-term tile with the shortest cross-term stage on the
- * first complex of that bucket; FSX_TUNE_FILE names a text file the table is
+ * pairs of gamma2 rows per unit with the shortest cross-term stage on the first
+ * complex of that bucket; FSX_TUNE_FILE names a text file the table is
  * read from and appended to ("bucket mixed rows slots ms" lines, slots 0:
  * the form's default pairing-slot cap). */
 #define FSX_TUNE_BUCKETS 6
@@ -3195,7 +3207,7 @@ static void tune_save(int b, int m, int r, int c, double ms)
 static int tune_one(const fsx_hip_args *A)
 {
     const int mixed = (A->flags & FSX_MIXED_FP32) != 0, b = tune_bucket(A->L);
-    /* gamma2 rows per tile; the pairing-slot cap stays the form's default,
+    /* pairs of gamma2 rows per unit; the pairing-slot cap stays the form's default,
      * since it sets the m-chunks and with them the order of the FP32 sums
      * (rows change no arithmetic: a tuned batch scores every pose exactly as
      * a single call does) */
@@ -3465,6 +3477,7 @@ static int run_batch_locked(int nprob, const fsx_hip_args *args, fsx_stats *st)
         ky->n = p->n; ky->flags = (int)A->flags; ky->half = p->half; ky->npk = p->npk; ky->C = p->C;
         ky->urows = p->urows; ky->mirror = p->mirror;
         ky->tile_rows = p->tile_rows; ky->aq_lds = p->aq_lds; ky->lanes = p->lanes;
+        ky->fit_wide = p->fit_wide; ky->fit_fpw = p->fit_fpw;
         ky->mult = A->mult; ky->peak = A->peak; ky->c1_lo = A->c1_lo; ky->c1_hi = A->c1_hi;
         ky->c2_lo = A->c2_lo; ky->c2_hi = A->c2_hi;
         memcpy(ky->d, p->d, sizeof(ky->d));
