@@ -2,7 +2,7 @@
  * fsx_cross.h -- the per-pose cross terms (device code, included by
  * fsx_kernels.hip).
  *
- * Work unit of one block: one q and one fsx_unit, a run of poses with the same
+ * Work item of one block: one q and one fsx_unit, a run of poses with the same
  * (z, beta2) on at most FSX_UROWS different gamma2 (the poses are sorted by
  * (beta2, z, gamma2), so a unit is a range of the sorted records).  The block
  *   1. translates the unit's ligand rows on the matrix cores,
@@ -30,7 +30,8 @@
 #define FSX_CROSS_H
 
 #define FSX_UROWS 8           /* most gamma2 rows of a unit */
-#define FSX_UPOSES 64         /* most poses of a unit */
+#define FSX_UPOSES 256        /* most poses of a unit: one per thread */
+#define FSX_UBATCH 64         /* poses paired between two writes of their sums */
 #define FSX_CROSS_BLOCK 256
 
 /* poses p0 .. p0 + n - 1 of the sorted records; row r (gamma2 g2[r]) holds the
@@ -42,6 +43,7 @@ struct fsx_unit {
     int nrow, pad;
 };
 static_assert(sizeof(fsx_unit) == 64, "one unit per 64-byte line");
+static_assert(FSX_UPOSES == FSX_CROSS_BLOCK && FSX_UBATCH == 64, "a wavefront holds a batch's records");
 
 /* One tile of the translation: up to FSX_CROSS_TILE l of one m.  Its operands are nks
  * steps from value bo of a ligand row and from value to of a translation block;
@@ -94,8 +96,8 @@ __host__ __device__ __forceinline__ int cross_us(int ns)
 template <typename F>
 __host__ __device__ __forceinline__ size_t cross_lds(int ns, int urows)
 {
-    return sizeof(F) * (2 * 3 * (size_t)urows * cross_us<F>(ns) + 6 * FSX_UPOSES) +
-           sizeof(int2) * FSX_UPOSES;
+    return sizeof(F) * (2 * 3 * (size_t)urows * cross_us<F>(ns) + 6 * FSX_UBATCH) +
+           sizeof(int2) * FSX_UBATCH;
 }
 
 /* l per translation tile: FP32 one 16x16x4 product, FP64 four 4x4x4 */
@@ -392,7 +394,7 @@ __device__ __forceinline__ void cross_body(const fsx_cross_job &A)
     const int us = cross_us<F>(ns);
     E *sU = reinterpret_cast<E *>(smem_raw);             /* [urows][3][us] */
     int2 *sP = reinterpret_cast<int2 *>(sU + 3 * A.urows * us);
-    F *sO = reinterpret_cast<F *>(sP + FSX_UPOSES);
+    F *sO = reinterpret_cast<F *>(sP + FSX_UBATCH);
     const int tid = threadIdx.x, lane = tid & (FSX_WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / FSX_WAVE);
     const int nwave = FSX_CROSS_BLOCK / FSX_WAVE;
@@ -447,7 +449,7 @@ __device__ __forceinline__ void cross_body(const fsx_cross_job &A)
      * translation */
     const FSX_CONST fsx_unit *u = fsx_const(A.units) + uidx;
     int4 rpf = make_int4(0, 0, 0, 0);
-    if (tid < FSX_UPOSES) rpf = A.recs[u->p0 + min(tid, u->n - 1)];
+    if (tid < u->n) rpf = A.recs[u->p0 + tid];
     typename std::conditional<sizeof(F) == 4, cross_u32, cross_u64>::type U;
     /* translation tiles, dealt to the wavefronts in turn */
     int ti = 0;
@@ -469,15 +471,13 @@ __device__ __forceinline__ void cross_body(const fsx_cross_job &A)
     item_begin();
     for (;;) {
         const int p0 = u->p0, n = u->n;
-        /* records: (receptor row, 8 alpha2 + row of the unit); past the last
-         * pose it is repeated, so the pose loop reads them without a clamp */
-        if (tid < FSX_UPOSES) {
-            const int jj = min(tid, n - 1), nrow = u->nrow;
-            int r = 0;
+        /* the record of pose tid: (receptor row, 8 alpha2 + row of the unit) */
+        const int nrow = u->nrow;
+        int r = 0;
 #pragma unroll
-            for (int k = 1; k < FSX_UROWS; k++) r += k < nrow && jj >= (int)(u->cum[k / 4] >> k % 4 * 8 & 255);
-            sP[tid] = make_int2(rpf.y, (rpf.z << 3) | r);
-        }
+        for (int k = 1; k < FSX_UROWS; k++) r += k < nrow && tid >= (int)(u->cum[k / 4] >> k % 4 * 8 & 255);
+        const int2 mine = make_int2(rpf.y, (rpf.z << 3) | r);
+        if (tid < FSX_UBATCH) sP[tid] = mine;
         /* ---- translation ---- */
         while (ti < A.ntiles) {
             const fsx_tile ct = tl;
@@ -495,12 +495,14 @@ __device__ __forceinline__ void cross_body(const fsx_cross_job &A)
         if (more) {
             for (uidx += nw; uidx >= (int)nunits; uidx -= (int)nunits) q++;
             u = fsx_const(A.units) + uidx;
-            if (tid < FSX_UPOSES) rpf = A.recs[u->p0 + min(tid, u->n - 1)];
+            if (tid < u->n) rpf = A.recs[u->p0 + tid];
             item_begin();
         }
         /* ---- pairing ---- */
         const char *RqB = reinterpret_cast<const char *>(A.R) + (size_t)qc * A.nrows * rstride;
-        for (int p = wave; p < n; p += nwave) {
+        for (int pb = 0;;) {
+        const int nb = min(n - pb, FSX_UBATCH);
+        for (int p = wave; p < nb; p += nwave) {
             const int2 rec = sP[p];
             const int prow = rec.y & 7;
             E rr[3][J];
@@ -582,16 +584,23 @@ __device__ __forceinline__ void cross_body(const fsx_cross_job &A)
             v[0] += dpp_mov<FSX_DPP_XOR2>(v[0]);
             if (writer) sO[p * 6 + slot] = v[0];
         }
-        /* the unit's sums to acc (pose-major [pose][q][6]), added to those of
-         * the earlier m-chunks; no barrier after it: sO is written again only
-         * after the next item's barrier */
+        /* the batch's sums to acc (pose-major [pose][q][6]), added to those of
+         * the earlier m-chunks (one launch after another: the atomic add, which no
+         * other block makes to the same value, spares the wait for the old one);
+         * no barrier after the last batch: sO is written again only after the
+         * next item's barrier */
         lds_barrier();
-        for (int i = tid; i < n * 6; i += FSX_CROSS_BLOCK) {
+        for (int i = tid; i < nb * 6; i += FSX_CROSS_BLOCK) {
             const int ip = i / 6;
-            double *d = A.acc + ((size_t)(p0 + ip) * Q + qc) * 6 + (i - ip * 6);
+            double *d = A.acc + ((size_t)(p0 + pb + ip) * Q + qc) * 6 + (i - ip * 6);
             const double x = 2.0 * (double)sO[i];
             if (A.first) __builtin_nontemporal_store(x, d);
             else unsafeAtomicAdd(d, x);
+        }
+        pb += FSX_UBATCH;
+        if (pb >= n) break;
+        if (tid / FSX_UBATCH == pb / FSX_UBATCH) sP[tid % FSX_UBATCH] = mine;
+        lds_barrier();
         }
         if (!more) return;
     }

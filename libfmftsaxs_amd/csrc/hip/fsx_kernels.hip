@@ -589,7 +589,7 @@ __global__ void k_count(const long long *poses, int n, int znum, int nbeta, int 
 
 /* First record of every bucket and the cross-term units, one wavefront per
  * (beta2, z).  Units are cut greedily along gamma2: up to urows rows and
- * FSX_UPOSES poses; a bucket of more poses takes several.  PASS 0 counts every
+ * cap poses; a bucket of more poses takes several.  PASS 0 counts every
  * group's records and units (grp), PASS 1 adds those of the groups before and
  * writes; tail: records, non-empty buckets, units.  The units are in the order of
  * the groups: with ranges reserved by atomics, in the order the wavefronts came,
@@ -600,12 +600,12 @@ __global__ void k_count(const long long *poses, int n, int znum, int nbeta, int 
  * at 478,000). */
 template <int PASS>
 __global__ void __launch_bounds__(256)
-k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int *offs, fsx_unit *units,
-        int *tail, int2 *grp)
+k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int cap, int *offs,
+        fsx_unit *units, int *tail, int2 *grp)
 {
     const int zb = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (zb >= nzb) return;
-    const int *c = counts + (size_t)zb * ng, cap = FSX_UPOSES;
+    const int *c = counts + (size_t)zb * ng;
     int total = 0, first = 0;
     if (PASS) {
         for (int k = lane; k < zb; k += 64) {
@@ -2844,10 +2844,18 @@ static int plan_enqueue(fsx_plan *p, hipStream_t s, hipEvent_t *ev, int stages =
     hipLaunchKernelGGL(k_count, dim3(nblk(n, 256)), dim3(256), 0, s, p->dposes, n, zn, p->nb, p->na,
                        ng, p->mirror, (int *)g[P_KEYS], (int2 *)g[P_INFO], counts);
     int2 *grp = (int2 *)(offs + ((nkeys + 4) & ~1L));
+    /* most poses of a unit: where the buckets are crowded, 64 leave most of a unit's
+     * rows unused (1,000,000 poses FP64 L = 15: cross terms 34.6 against 30.4 ms); fewer
+     * only where the units would not fill the device four times */
+    const long items = 4L * 5 * g_ncu;
+    const int cap = (int)((long)n * Q / items > FSX_UPOSES ? FSX_UPOSES
+                          : (long)n * Q / items < 64 ? 64 : (long)n * Q / items);
     hipLaunchKernelGGL(k_units<0>, dim3(nblk((long)p->nb * zn, 4)), dim3(256), 0, s, (const int *)counts,
-                       p->nb * zn, p->nb, zn, ng, p->urows, offs, (fsx_unit *)g[P_UNITS], tail, grp);
+                       p->nb * zn, p->nb, zn, ng, p->urows, cap, offs, (fsx_unit *)g[P_UNITS], tail,
+                       grp);
     hipLaunchKernelGGL(k_units<1>, dim3(nblk((long)p->nb * zn, 4)), dim3(256), 0, s, (const int *)counts,
-                       p->nb * zn, p->nb, zn, ng, p->urows, offs, (fsx_unit *)g[P_UNITS], tail, grp);
+                       p->nb * zn, p->nb, zn, ng, p->urows, cap, offs, (fsx_unit *)g[P_UNITS], tail,
+                       grp);
     hipLaunchKernelGGL(k_scatter, dim3(nblk(n, 256)), dim3(256), 0, s, (const int *)g[P_KEYS],
                        (const int2 *)g[P_INFO], n, ng, (const int *)offs, counts + nkeys,
                        (int4 *)g[P_RECS]);
