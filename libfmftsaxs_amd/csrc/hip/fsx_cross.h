@@ -17,14 +17,14 @@
  * Only rows that some pose asks for are translated.  What bounds it depends on
  * the poses per unit: with many (210,000 poses at L = 15: 38 to a unit) the
  * receptor rows, 6 KB (FP64) or 3 KB per pose and q, most of which an XCD's 4 MB
- * L2 does not hold in FP64 (73 GB from behind it in 9.7 ms); with few (200,000 to
- * 300,000 on a 37 x 128 grid of 0.5 A steps at L = 25: about 10) the loads and
- * waits of an item's chain, unit, operands, products, rows.
- * The form before it, tiles of adjacent gamma2 with all z inside and the
- * translation on the vector units, translated every row of a tile for every z
- * in use and read 100 bytes of LDS per lane for 24 multiply-adds: L = 25, 81 q,
- * 300,000 poses FP32 224 ms against 65.6 now, 200,000 poses FP64 219 against 156;
- * L = 15, 51 q, 210,000 poses FP32 4.7 against 4.4, FP64 9.7 and 9.7.
+ * L2 does not hold in FP64; with few (200,000 to 300,000 on a 37 x 128 grid of 0.5 A
+ * steps at L = 25: about 10) the loads and waits of an item's chain, unit, operands,
+ * products, rows.  The form before it, tiles of adjacent gamma2 with all z inside
+ * and the translation on the vector units, translated every row of a tile for every
+ * z in use and read 100 bytes of LDS per lane for 24 multiply-adds: L = 25, 81 q,
+ * 300,000 poses FP32 224 ms against 63 now, 200,000 poses FP64 219 against 145;
+ * L = 15, 51 q, 210,000 poses FP32 4.7 against 4.5, FP64 9.65 against 9.3; crowded
+ * buckets (1,000,000 poses) FP64 28.6 against 30.4.
  */
 #ifndef FSX_CROSS_H
 #define FSX_CROSS_H
