@@ -1,0 +1,23 @@
+/*
+ * fsx_rules.h -- rules by which a call's sizes choose among kernel forms,
+ * shared by the HIP side and host C (so that they can be exercised on the CPU).
+ */
+#ifndef FSX_RULES_H
+#define FSX_RULES_H
+
+/* Poses a wavefront of the cross-term pairing takes at a time, for chunks of ns
+ * pairing slots.  Two poses of 32 lanes share the lane sums' instructions and
+ * leave fewer lanes without a slot; one pose of 64 lanes has half the loads and
+ * registers per lane.  Cross terms with 41 q, z 30 to 49 A, one against two poses:
+ *   FP32  140,000 poses: L = 6 (25 slots) 0.90 and 0.51 ms, 7 (32) 0.88 and 0.49,
+ *         10 (61) 0.96 and 0.91, 12 (85) 1.97 and 1.52, 13 (98) 1.95 and 1.96;
+ *         20,000: 6 0.18 and 0.11, 12 0.36 and 0.32, 13 0.40 and 0.43, 15 (128) 0.47
+ *         and 0.50, 16 (two chunks of about 72) 0.79 and 0.74, 20 (112) 1.18 and 1.28;
+ *   FP64  140,000: 6 1.41 and 0.78, 10 1.64 and 1.37, 12 2.86 and 2.20, 15 3.16 and
+ *         2.95; 20,000: 6 0.29 and 0.18, 15 1.09 and 1.06, 20 (118) 3.89 and 3.87. */
+static inline int fsx_cross_pw(int mixed, int ns)
+{
+    return ns <= (mixed ? 96 : 128) ? 2 : 1;
+}
+
+#endif

@@ -383,8 +383,8 @@ struct cross_u64 {
     }
 };
 
-/* J: slots per lane */
-template <int J, typename E>
+/* J: slots per lane; PW: poses per wavefront */
+template <int J, typename E, int PW>
 __device__ __forceinline__ void cross_body(const fsx_cross_job &A)
 {
 #pragma clang fp contract(fast)
@@ -398,16 +398,14 @@ __device__ __forceinline__ void cross_body(const fsx_cross_job &A)
     const int tid = threadIdx.x, lane = tid & (FSX_WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / FSX_WAVE);
     const int nwave = FSX_CROSS_BLOCK / FSX_WAVE;
-    /* pairing: one pose per wavefront, its lane i taking slots i, i + 64, ... (J per
-     * lane).  With npk > 0 (conjugate-symmetric coefficients, the chunk of m = 0)
-     * the m = 0 entries l = 2i and 2i + 1 share slot i, both real after the turns
-     * by i^l and i^-l: the real part of the slot is the first, the imaginary part
-     * the second (negated in U, so that Re(R U) of the slot adds the two
-     * products); their twiddle is 1.  (FP32 tables, two poses per wavefront of 32
-     * lanes each share the lane sums' instructions but hold twice the loads per
-     * lane: 86 against 75 ms at L = 25 with 300,000 poses, the same at L = 15.) */
-    constexpr int LP = FSX_WAVE;
-    const int sl = lane;
+    /* pairing: PW poses per wavefront of LP lanes each, lane sl of a pose taking
+     * slots sl, sl + LP, ... (J per lane).  With npk > 0 (conjugate-symmetric
+     * coefficients, the chunk of m = 0) the m = 0 entries l = 2i and 2i + 1 share
+     * slot i, both real after the turns by i^l and i^-l: the real part of the slot
+     * is the first, the imaginary part the second (negated in U, so that Re(R U) of
+     * the slot adds the two products); their twiddle is 1. */
+    constexpr int LP = FSX_WAVE / PW;
+    const int sl = lane % LP, half = lane / LP;
     const unsigned rstride = 3u * (unsigned)ns * (unsigned)sizeof(E);
     const unsigned ustride = 3u * (unsigned)us * (unsigned)sizeof(E);
     const unsigned soff = (unsigned)(sl * sizeof(E));
@@ -429,9 +427,12 @@ __device__ __forceinline__ void cross_body(const fsx_cross_job &A)
         const int odd = A.mirror && ec >= npk && ec < ns ? (A.el[e] + m) & 1 : 0;
         emo[j] = (unsigned)((m + L) * twk + odd) * (unsigned)sizeof(E);
     }
-    /* after the lane reduction lanes 0, 8, .., 40 hold the six sums */
-    const int slot = lane >> 3;
-    const bool writer = (lane & 7) == 0 && slot < 6;
+    /* after the lane reduction: one pose: lanes 0, 8, .., 40 hold the six sums;
+     * two poses: lanes 0, 8, 4, 16, 24, 20 of each half (bits 4, 3, 2 of the
+     * lane select sum 3 b4 + (b2 ? 2 : b3)) */
+    const bool b4 = lane & 16, b3 = lane & 8, b2 = lane & 4;
+    const int slot = PW == 1 ? lane >> 3 : (b4 ? 3 : 0) + (b2 ? 2 : b3);
+    const bool writer = PW == 1 ? (lane & 7) == 0 && slot < 6 : (lane & 3) == 0 && !(b2 && b3);
     const E *tw2 = reinterpret_cast<const E *>(A.tw2);
     /* items (q, unit) in nx contiguous ranges, one per XCD (blocks go to the
      * XCDs round-robin), each walked by that XCD's blocks together: at any
@@ -502,7 +503,10 @@ __device__ __forceinline__ void cross_body(const fsx_cross_job &A)
         const char *RqB = reinterpret_cast<const char *>(A.R) + (size_t)qc * A.nrows * rstride;
         for (int pb = 0;;) {
         const int nb = min(n - pb, FSX_UBATCH);
-        for (int p = wave; p < nb; p += nwave) {
+        /* PW poses per step; one past the batch's last repeats some earlier
+         * record of sP (in bounds), and nothing reads its sums */
+        for (int pp = wave; PW * pp < nb; pp += nwave) {
+            const int p = PW * pp + half;
             const int2 rec = sP[p];
             const int prow = rec.y & 7;
             E rr[3][J];
@@ -536,8 +540,15 @@ __device__ __forceinline__ void cross_body(const fsx_cross_job &A)
                                                        __umul24((unsigned)prow, ustride));
             /* Re of each product, accumulated term by term (one fused
              * multiply-add per term), the products of the imaginary parts
-             * apart (FP32 tables): their sign is the pose's */
-            F va[6] = {0, 0, 0, 0, 0, 0}, vb[6] = {0, 0, 0, 0, 0, 0};
+             * apart (FP32 tables): their sign is the pose's.  With two poses per
+             * wavefront the even and the odd j are summed apart: those of lanes
+             * i and i + 32 of the form with one pose, so that a pose's sums
+             * have the same bits in both. */
+            F sa[PW][6], sb[PW][6];
+#pragma unroll
+            for (int h = 0; h < PW; h++)
+#pragma unroll
+                for (int k = 0; k < 6; k++) sa[h][k] = sb[h][k] = 0;
 #pragma unroll
             for (int j = 0; j < J; j++) {
                 const bool ok = j < J - 1 || sl + LP * j < ns;
@@ -549,7 +560,7 @@ __device__ __forceinline__ void cross_body(const fsx_cross_job &A)
                 const F vr = w_r * rv.re - w_i * rv.im, vi = w_r * rv.im + w_i * rv.re;
                 const F dr = w_r * rd.re - w_i * rd.im, di = w_r * rd.im + w_i * rd.re;
                 const F xr = w_r * rw.re - w_i * rw.im, xi = w_r * rw.im + w_i * rw.re;
-                F *vc = sizeof(E) == 8 ? vb : va;
+                F *va = sa[j % PW], *vc = sizeof(E) == 8 ? sb[j % PW] : va;
                 const F sg = sizeof(E) == 8 ? (F)1 : (F)-1;
                 va[0] += vr * uv.re; vc[0] += sg * (vi * uv.im);
                 va[1] += vr * ud.re; vc[1] += sg * (vi * ud.im);
@@ -564,22 +575,43 @@ __device__ __forceinline__ void cross_body(const fsx_cross_job &A)
             if (sizeof(E) == 8) {
                 const F sg = A.mirror && ((unsigned)rec.y >> 3 & 1) ? (F)1 : (F)-1;
 #pragma unroll
-                for (int k = 0; k < 6; k++) va[k] += sg * vb[k];
+                for (int h = 0; h < PW; h++)
+#pragma unroll
+                    for (int k = 0; k < 6; k++) sa[h][k] += sg * sb[h][k];
             }
             /* the cross-lane sums run in the contraction's type */
-            F v[8] = {va[0], va[1], va[2], va[3], va[4], va[5], 0, 0};
-            /* transpose-reduce over the 64 lanes: after the three halving steps
-             * lane bits 5,4,3 select the slot, then a sum over the 8 lanes of bits
-             * 2,1,0; lanes 0, 8, .., 40 hold slots 0..5 */
+            F v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-            for (int i = 0; i < 4; i++) v[i] = tr_swap32(v[i], v[i + 4]);
+            for (int k = 0; k < 6; k++) v[k] = PW == 2 && J > 1 ? sa[0][k] + sa[PW - 1][k] : sa[0][k];
+            if (PW == 1) {
+                /* transpose-reduce over the 64 lanes: after the three halving
+                 * steps lane bits 5,4,3 select the slot, then a sum over the 8
+                 * lanes of bits 2,1,0; lanes 0, 8, .., 40 hold slots 0..5 */
 #pragma unroll
-            for (int i = 0; i < 2; i++) v[i] = tr_swap16(v[i], v[i + 2]);
-            const bool hi = (lane & 8) != 0;
-            const F send = hi ? v[0] : v[1];
-            const F keep = hi ? v[1] : v[0];
-            v[0] = keep + dpp_mov<FSX_DPP_ROR8>(send);
-            v[0] += dpp_mov<FSX_DPP_HMIRROR>(v[0]);
+                for (int i = 0; i < 4; i++) v[i] = tr_swap32(v[i], v[i + 4]);
+#pragma unroll
+                for (int i = 0; i < 2; i++) v[i] = tr_swap16(v[i], v[i + 2]);
+                const F send = b3 ? v[0] : v[1];
+                const F keep = b3 ? v[1] : v[0];
+                v[0] = keep + dpp_mov<FSX_DPP_ROR8>(send);
+                v[0] += dpp_mov<FSX_DPP_HMIRROR>(v[0]);
+            } else {
+                /* the same within each 32-lane half, on the six sums: bit 4
+                 * pairs sums i and i + 3; bit 3 the first two of those, the
+                 * third across itself; bit 2 the two results: the same pairs
+                 * as above */
+#pragma unroll
+                for (int i = 0; i < 3; i++) v[i] = tr_swap16(v[i], v[i + 3]);
+                {
+                    const F send = b3 ? v[0] : v[1];
+                    const F keep = b3 ? v[1] : v[0];
+                    v[0] = keep + dpp_mov<FSX_DPP_ROR8>(send);
+                    v[1] = v[2] + dpp_mov<FSX_DPP_ROR8>(v[2]);
+                }
+                const F send = b2 ? v[0] : v[1];
+                const F keep = b2 ? v[1] : v[0];
+                v[0] = keep + dpp_mov<FSX_DPP_HMIRROR>(send);
+            }
             v[0] += dpp_mov<FSX_DPP_XOR1>(v[0]);
             v[0] += dpp_mov<FSX_DPP_XOR2>(v[0]);
             if (writer) sO[p * 6 + slot] = v[0];
@@ -610,11 +642,11 @@ __device__ __forceinline__ void cross_body(const fsx_cross_job &A)
 template <typename E>
 __host__ __device__ constexpr int cross_waves() { return sizeof(E) == 8 ? 4 : 3; }
 
-template <int J, typename E>
+template <int J, typename E, int PW>
 __global__ void __launch_bounds__(FSX_CROSS_BLOCK, (cross_waves<E>()))
 k_cross(const fsx_cross_job job)
 {
-    cross_body<J, E>(job);
+    cross_body<J, E, PW>(job);
 }
 
 /* The launches of several complexes in one (the batched form): every block
@@ -622,13 +654,13 @@ k_cross(const fsx_cross_job job)
  * launch drains between complexes.  The jobs of one launch share the template
  * parameters; a complex appears once per launch (its m-chunks are launched in
  * order, one launch per chunk index). */
-template <int J, typename E>
+template <int J, typename E, int PW>
 __global__ void __launch_bounds__(FSX_CROSS_BLOCK, (cross_waves<E>()))
 k_cross_jobs(const fsx_cross_job *jobs, int njobs)
 {
     for (int k = 0; k < njobs; k++) {
         const fsx_cross_job jb = jobs[k];
-        cross_body<J, E>(jb);
+        cross_body<J, E, PW>(jb);
         /* the next job lays out the LDS for its own chunk size */
         __syncthreads();
     }

@@ -30,6 +30,7 @@
 
 #include "../fsx_internal.h"
 #include "../fsx_pose.h"
+#include "../fsx_rules.h"
 /* the fit kernels keep the L-BFGS-B blocks K11, K12, K22 and WN1 in LDS, one
  * column of 256 lanes (a fit block) per value */
 #define FSX_LB_KSHARED
@@ -2024,21 +2025,27 @@ static inline unsigned nblk(long n, int t) { return (unsigned)((n + t - 1) / t);
         if (r_ != FSX_OK) return r_;   \
     } while (0)
 
-/* kernel of a cross-term launch for chunks of ns slots */
-template <typename E>
+/* kernel of a cross-term launch with jn slots per lane and pw poses per wavefront */
+template <typename E, int PW>
 static const void *cross_kernel(int jn, int jobs)
 {
     if (jobs)
-        return jn <= 1 ? (const void *)k_cross_jobs<1, E> : jn <= 2 ? (const void *)k_cross_jobs<2, E>
-             : jn <= 3 ? (const void *)k_cross_jobs<3, E> : (const void *)k_cross_jobs<4, E>;
-    return jn <= 1 ? (const void *)k_cross<1, E> : jn <= 2 ? (const void *)k_cross<2, E>
-         : jn <= 3 ? (const void *)k_cross<3, E> : (const void *)k_cross<4, E>;
+        return jn <= 1 ? (const void *)k_cross_jobs<1, E, PW> : jn <= 2 ? (const void *)k_cross_jobs<2, E, PW>
+             : jn <= 3 ? (const void *)k_cross_jobs<3, E, PW> : (const void *)k_cross_jobs<4, E, PW>;
+    return jn <= 1 ? (const void *)k_cross<1, E, PW> : jn <= 2 ? (const void *)k_cross<2, E, PW>
+         : jn <= 3 ? (const void *)k_cross<3, E, PW> : (const void *)k_cross<4, E, PW>;
 }
-static const void *cross_kernel_of(int mixed, int jn, int jobs)
+static const void *cross_kernel_of(int mixed, int jn, int pw, int jobs)
 {
-    return mixed ? cross_kernel<cplx32>(jn, jobs) : cross_kernel<cplx>(jn, jobs);
+    return pw == 2 ? (mixed ? cross_kernel<cplx32, 2>(jn, jobs) : cross_kernel<cplx, 2>(jn, jobs))
+                   : (mixed ? cross_kernel<cplx32, 1>(jn, jobs) : cross_kernel<cplx, 1>(jn, jobs));
 }
-static int cross_jn(int ns) { return ns <= FSX_WAVE ? 1 : (ns + FSX_WAVE - 1) / FSX_WAVE; }
+/* poses per wavefront (FSX_CROSS_PW overrides where two fit, four slots per lane) */
+static int cross_pw(int mixed, int ns)
+{
+    return ns <= 4 * (FSX_WAVE / 2) && env_int("FSX_CROSS_PW", fsx_cross_pw(mixed, ns), 1, 2) == 2 ? 2 : 1;
+}
+static int cross_jn(int ns, int pw) { return (pw * ns + FSX_WAVE - 1) / FSX_WAVE; }
 static size_t cross_lds_of(int mixed, int ns, int urows)
 {
     return mixed ? cross_lds<float>(ns, urows) : cross_lds<double>(ns, urows);
@@ -2069,7 +2076,7 @@ static int cross_nx(long grid)
  * complex's m-chunks become jobs, grouped into launches of k_cross_jobs by
  * chunk index and kernel shape. */
 struct fsx_cross_group {
-    int mixed, jn, chunk;       /* the kernel and the m-chunk index */
+    int mixed, jn, pw, chunk;   /* the kernel and the m-chunk index */
     size_t lds;                 /* the largest job's LDS */
     int njobs, cap;
     long grid;                  /* blocks of the launch */
@@ -2866,7 +2873,8 @@ static int plan_enqueue(fsx_plan *p, hipStream_t s, hipEvent_t *ev, int stages =
     if (stages & FSX_ST_CROSS) {
     for (int c = 0; c < p->C; c++) {
         const int ns = p->ent[FSX_E_RSR(p) + c] / 6;
-        const void *kern = cross_kernel_of(p->mixed, cross_jn(ns), 0);
+        const int pw = cross_pw(p->mixed, ns);
+        const void *kern = cross_kernel_of(p->mixed, cross_jn(ns, pw), pw, 0);
         const size_t lds = cross_lds_of(p->mixed, ns, p->urows);
         /* no more blocks than (q, unit) items can be */
         long grid = cross_grid(kern, lds);
@@ -3280,11 +3288,11 @@ static int plan_cross_collect(const fsx_plan *p, fsx_cross_group **gr, int *ngr)
     for (int c = 0; c < p->C; c++) {
         const int ns = p->ent[FSX_E_RSR(p) + c] / 6;
         const size_t lds = cross_lds_of(p->mixed, ns, p->urows);
-        const int jn = cross_jn(ns);
+        const int pw = cross_pw(p->mixed, ns), jn = cross_jn(ns, pw);
         fsx_cross_group *t = NULL;
         for (int i = 0; i < *ngr; i++) {
             fsx_cross_group *u = &(*gr)[i];
-            if (u->mixed == p->mixed && u->jn == jn && u->chunk == c) t = u;
+            if (u->mixed == p->mixed && u->jn == jn && u->pw == pw && u->chunk == c) t = u;
         }
         if (!t) {
             fsx_cross_group *ng2 = (fsx_cross_group *)realloc(*gr, sizeof(fsx_cross_group) * (*ngr + 1));
@@ -3292,7 +3300,7 @@ static int plan_cross_collect(const fsx_plan *p, fsx_cross_group **gr, int *ngr)
             *gr = ng2;
             t = &(*gr)[(*ngr)++];
             memset(t, 0, sizeof(*t));
-            t->mixed = p->mixed; t->jn = jn; t->chunk = c;
+            t->mixed = p->mixed; t->jn = jn; t->pw = pw; t->chunk = c;
         }
         if (t->njobs == t->cap) {
             const int cap = t->cap ? 2 * t->cap : 8;
@@ -3420,7 +3428,7 @@ static int run_batch_locked(int nprob, const fsx_hip_args *args, fsx_stats *st)
         size_t ntot = 0;
         for (int i = 0; i < ncg; i++) ntot += cg[i].njobs;
         for (int i = 0; rc == FSX_OK && i < ncg; i++) {
-            cg[i].grid = cross_grid(cross_kernel_of(cg[i].mixed, cg[i].jn, 1), cg[i].lds);
+            cg[i].grid = cross_grid(cross_kernel_of(cg[i].mixed, cg[i].jn, cg[i].pw, 1), cg[i].lds);
             for (int j = 0; j < cg[i].njobs; j++) cg[i].jobs[j].nx = cross_nx(cg[i].grid);
         }
         if (rc == FSX_OK) rc = grow_dev((void **)&g_cjob_dev, &g_cjob_cap,
@@ -3537,7 +3545,7 @@ static int run_batch_locked(int nprob, const fsx_hip_args *args, fsx_stats *st)
                     const fsx_cross_job *jobs = g_cjob_dev + o;
                     int nj = cg[i].njobs;
                     void *kargs[2] = {(void *)&jobs, (void *)&nj};
-                    if (hipLaunchKernel(cross_kernel_of(cg[i].mixed, cg[i].jn, 1),
+                    if (hipLaunchKernel(cross_kernel_of(cg[i].mixed, cg[i].jn, cg[i].pw, 1),
                                         dim3((unsigned)cg[i].grid), dim3(FSX_CROSS_BLOCK), kargs,
                                         cg[i].lds, g_stream) !=
                         hipSuccess)

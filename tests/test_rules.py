@@ -1,0 +1,35 @@
+"""The size rules of csrc/fsx_rules.h, compiled for the host with gcc."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SRC = r"""
+#include "fsx_rules.h"
+int cross_pw(int mixed, int ns) { return fsx_cross_pw(mixed, ns); }
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    src, so = d / "rules.c", d / "librules.so"
+    src.write_text(SRC)
+    subprocess.run(["gcc", "-std=c11", "-O2", "-Wall", "-Werror", "-shared", "-fPIC",
+                    "-I" + os.path.join(ROOT, "libfmftsaxs_amd", "csrc"), str(src), "-o",
+                    str(so)], check=True)
+    return C.CDLL(str(so))
+
+
+def test_two_poses_per_wavefront_at_small_orders(rules):
+    """Slots of one chunk at order L: (L + 1)(L + 2) / 2 less the packed m = 0
+    pairs.  Orders 6 to 12 leave lanes of a one-pose wavefront without a slot or
+    its last slots half empty."""
+    for L in range(6, 13):
+        ns = (L + 1) * (L + 2) // 2 - (L + 1) // 2
+        assert rules.cross_pw(1, ns) == 2 and rules.cross_pw(0, ns) == 2, L
+    assert rules.cross_pw(1, 128) == 1 and rules.cross_pw(0, 128) == 2
+    assert rules.cross_pw(1, 176) == 1 and rules.cross_pw(0, 176) == 1
