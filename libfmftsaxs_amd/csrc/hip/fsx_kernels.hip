@@ -9,7 +9,7 @@
  *                 ligand    B^Y_lm(b2,g2,q) = sum_m2 e^{-i m2 g2} d^l_{m m2}(b2) conj(B^Y_{l m2})
  *                 (the beta/gamma factors of compute_sum1/compute_sum2 and of the
  *                 3-D DFT, fftsaxs.c:251-333, 416-524, 680, folded per pose axis)
- *   k_count/k_units/k_scatter  bucket poses by (beta2, z, gamma2), units of buckets
+ *   k_count/k_units/k_scatter  bucket poses by (z, beta2, gamma2), units of buckets
  *   k_cross       per unit and q (fsx_cross.h): U^Y_lm = sum_l1 conj(T_{|m| l l1}) B^Y_{l1 m} in LDS,
  *                 then per pose 2 Re sum_lm e^{-i m a2} (R^X U^Y [+ R^Y U^X]) for the six
  *                 cross terms VV,VD,VW,DD,DW,WW (fill_var, fftsaxs.c:87-108)
@@ -566,7 +566,7 @@ __device__ __forceinline__ void fsx_mirror(int nbeta, int na, int ng, int *b1, i
     *alpha = 2 * *alpha + m1;
 }
 
-/* bucket (beta2, z, gamma2) of each pose, its receptor row and twiddle
+/* bucket (z, beta2, gamma2) of each pose, its receptor row and twiddle
  * row */
 __global__ void k_count(const long long *poses, int n, int znum, int nbeta, int na, int ng,
                         int mirror, int *keys, int2 *info, int *counts)
@@ -576,12 +576,9 @@ __global__ void k_count(const long long *poses, int n, int znum, int nbeta, int 
     int row, alpha;
     int key = fsx_pose_key(poses[i], znum, nbeta, na, ng, &row, &alpha);
     if (key >= 0) {
-        const int zb = key / ng, z = zb / nbeta;
-        const int b2 = zb - z * nbeta, g2 = key - zb * ng;
         int b1 = row / ng, g1 = row - b1 * ng;
         if (mirror) fsx_mirror(nbeta, na, ng, &b1, &g1, &alpha);
         row = b1 * ng + g1;
-        key = (b2 * znum + z) * ng + g2;
         atomicAdd(&counts[key], 1);
     }
     keys[i] = key;
@@ -589,14 +586,19 @@ __global__ void k_count(const long long *poses, int n, int znum, int nbeta, int 
 }
 
 /* First record of every bucket and the cross-term units, one wavefront per
- * (beta2, z).  Units are cut greedily along gamma2: up to urows rows and
+ * (z, beta2).  Units are cut greedily along gamma2: up to urows rows and
  * cap poses; a bucket of more poses takes several.  PASS 0 counts every
  * group's records and units (grp), PASS 1 adds those of the groups before and
- * writes; tail: records, non-empty buckets, units.  The units are in the order of
- * the groups: with ranges reserved by atomics, in the order the wavefronts came,
- * an XCD's blocks worked on all beta2 at a time and its L2 lost the ligand rows (cross
- * terms FP64 L = 15, 210,000 poses 9.76 against 9.27 ms; L = 25, 200,000 poses 156
- * against 146, FP32 300,000 poses 65.5 against 61.7).
+ * writes; tail: records, non-empty buckets, units.
+ * The records, and with them the fits, are in the order of (z, beta2): the poses of
+ * one z take about the same number of evaluations, and the long ones don't come
+ * last (in the order of (beta2, z) the fits of 210,000 poses, L = 10, 41 q took 1.05
+ * against 0.67 ms in the mixed form and 1.53 against 1.27 in FP64, L = 12 1.13
+ * against 0.73 and 1.69 against 1.35; 20,000 poses within 0.1 ms either way).
+ * The units are in the order of (beta2, z): in the order of the records, or with ranges
+ * reserved by atomics, an XCD's blocks work on all beta2 at a time and its L2 loses
+ * the ligand rows (cross terms FP64 L = 15, 210,000 poses 9.76 against 9.27 ms; L =
+ * 25, 200,000 poses 156 against 146, FP32 300,000 poses 65.5 against 61.7).
  * Against a scan by a single block, whose time grew with the number of buckets (828 us
  * at 478,000). */
 template <int PASS>
@@ -607,12 +609,13 @@ k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int cap, 
     const int zb = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (zb >= nzb) return;
     const int *c = counts + (size_t)zb * ng;
+    const int z = zb / nb, b2 = zb - z * nb;
     int total = 0, first = 0;
     if (PASS) {
-        for (int k = lane; k < zb; k += 64) {
-            total += grp[k].x;
-            first += grp[k].y;
-        }
+        /* records by (z, beta2), units by (beta2, z) */
+        const int ub = b2 * zn + z;
+        for (int k = lane; k < zb; k += 64) total += grp[k].x;
+        for (int k = lane; k < ub; k += 64) first += grp[k].y;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
             total += __shfl_xor(total, o);
@@ -623,8 +626,8 @@ k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int cap, 
     }
     int p = 0, nz = 0, un = 0, ur = 0, uc = 0;   /* records so far, buckets; open unit's poses and rows; units */
     fsx_unit u;
-    u.b2 = zb / zn % nb;
-    u.z = zb % zn;
+    u.b2 = b2;
+    u.z = z;
     u.pad = 0;
     for (int g0 = 0; g0 < ng; g0 += 64) {
         const int v = g0 + lane < ng ? c[g0 + lane] : 0;
@@ -684,7 +687,8 @@ k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int cap, 
         uc++;
     }
     if (!PASS && lane == 0) {
-        grp[zb] = make_int2(p, uc);
+        grp[zb].x = p;
+        grp[b2 * zn + z].y = uc;
         if (p > 0) {
             atomicAdd(&tail[0], p);
             atomicAdd(&tail[1], nz);
@@ -2496,7 +2500,7 @@ static int plan_init(fsx_plan *p, const fsx_hip_args *A, int tile_rows, int slot
     z[P_KEYS] = sizeof(int) * n;
     z[P_INFO] = sizeof(int2) * n;
     z[P_COUNTS] = sizeof(int) * 2 * p->nkeys;   /* counts, then fills */
-    /* then records, buckets, units; then those of each (beta2, z) */
+    /* then records, buckets, units; then those of each (z, beta2), (beta2, z) */
     z[P_OFFS] = sizeof(int) * (p->nkeys + 4) + sizeof(int2) * (size_t)nb * zn;
     z[P_UNITS] = sizeof(fsx_unit) * (size_t)n;
     z[P_RECS] = sizeof(int4) * n;
@@ -2845,7 +2849,7 @@ static int plan_enqueue(fsx_plan *p, hipStream_t s, hipEvent_t *ev, int stages =
     }
     HIPR(hipGetLastError());
     if (ev) HIPR(hipEventRecord(ev[2], s));
-    /* poses sorted by (beta2, z, gamma2), and the cross-term units */
+    /* poses sorted by (z, beta2, gamma2), and the cross-term units */
     hipLaunchKernelGGL(k_init, dim3(nblk(2 * nkeys, 256)), dim3(256), 0, s, counts, 2 * nkeys, tail,
                        (int *)g[P_NEXT], (int)p->fit_next0, (unsigned long long *)g[P_TALLY]);
     hipLaunchKernelGGL(k_count, dim3(nblk(n, 256)), dim3(256), 0, s, p->dposes, n, zn, p->nb, p->na,
