@@ -599,12 +599,12 @@ __global__ void k_count(const long long *poses, int n, int znum, int nbeta, int 
  * reserved by atomics, an XCD's blocks work on all beta2 at a time and its L2 loses
  * the ligand rows (cross terms FP64 L = 15, 210,000 poses 9.76 against 9.27 ms; L =
  * 25, 200,000 poses 156 against 146, FP32 300,000 poses 65.5 against 61.7).
- * Against a scan by a single block, whose time grew with the number of buckets (828 us
- * at 478,000). */
+ * scanned: grp holds the sums already (k_unit_scan), for many groups; summing them in
+ * every wavefront costs the square of their number. */
 template <int PASS>
 __global__ void __launch_bounds__(256)
 k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int cap, int *offs,
-        fsx_unit *units, int *tail, int2 *grp)
+        fsx_unit *units, int *tail, int2 *grp, int scanned)
 {
     const int zb = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (zb >= nzb) return;
@@ -614,12 +614,17 @@ k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int cap, 
     if (PASS) {
         /* records by (z, beta2), units by (beta2, z) */
         const int ub = b2 * zn + z;
-        for (int k = lane; k < zb; k += 64) total += grp[k].x;
-        for (int k = lane; k < ub; k += 64) first += grp[k].y;
+        if (scanned) {
+            total = grp[zb].x;
+            first = grp[ub].y;
+        } else {
+            for (int k = lane; k < zb; k += 64) total += grp[k].x;
+            for (int k = lane; k < ub; k += 64) first += grp[k].y;
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            total += __shfl_xor(total, o);
-            first += __shfl_xor(first, o);
+            for (int o = 1; o < 64; o <<= 1) {
+                total += __shfl_xor(total, o);
+                first += __shfl_xor(first, o);
+            }
         }
         total = __builtin_amdgcn_readfirstlane(total);
         first = __builtin_amdgcn_readfirstlane(first);
@@ -694,6 +699,53 @@ k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int cap, 
             atomicAdd(&tail[1], nz);
             atomicAdd(&tail[2], uc);
         }
+    }
+}
+
+/* The groups' counts (grp of k_units<0>) to the sums of those before, in place, by
+ * one block, four groups per thread and step. */
+__global__ void __launch_bounds__(1024)
+k_unit_scan(int2 *grp, int nzb)
+{
+    __shared__ int2 part[16];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int2 base = make_int2(0, 0);
+    for (long g0 = 0; g0 < nzb; g0 += 4096) {
+        const long i0 = g0 + 4 * threadIdx.x;
+        int2 v[4], s = make_int2(0, 0);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int2 c = i0 + k < nzb ? grp[i0 + k] : make_int2(0, 0);
+            v[k] = s;
+            s.x += c.x;
+            s.y += c.y;
+        }
+        /* over the wavefront, then over the wavefronts */
+        int2 x = s;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int a = __shfl_up(x.x, o), b = __shfl_up(x.y, o);
+            if (lane >= o) {
+                x.x += a;
+                x.y += b;
+            }
+        }
+        if (lane == 63) part[w] = x;
+        __syncthreads();
+        int2 all = base;
+        for (int k = 0; k < 16; k++) {
+            if (k == w) {
+                x.x += all.x - s.x;
+                x.y += all.y - s.y;
+            }
+            all.x += part[k].x;
+            all.y += part[k].y;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (i0 + k < nzb) grp[i0 + k] = make_int2(x.x + v[k].x, x.y + v[k].y);
+        base = all;
+        __syncthreads();
     }
 }
 
@@ -2861,12 +2913,12 @@ static int plan_enqueue(fsx_plan *p, hipStream_t s, hipEvent_t *ev, int stages =
     const long items = 4L * 5 * g_ncu;
     const int cap = (int)((long)n * Q / items > FSX_UPOSES ? FSX_UPOSES
                           : (long)n * Q / items < 64 ? 64 : (long)n * Q / items);
-    hipLaunchKernelGGL(k_units<0>, dim3(nblk((long)p->nb * zn, 4)), dim3(256), 0, s, (const int *)counts,
-                       p->nb * zn, p->nb, zn, ng, p->urows, cap, offs, (fsx_unit *)g[P_UNITS], tail,
-                       grp);
-    hipLaunchKernelGGL(k_units<1>, dim3(nblk((long)p->nb * zn, 4)), dim3(256), 0, s, (const int *)counts,
-                       p->nb * zn, p->nb, zn, ng, p->urows, cap, offs, (fsx_unit *)g[P_UNITS], tail,
-                       grp);
+    const int nzb = p->nb * zn, scan = fsx_unit_scan(nzb);
+    hipLaunchKernelGGL(k_units<0>, dim3(nblk(nzb, 4)), dim3(256), 0, s, (const int *)counts, nzb, p->nb, zn, ng,
+                       p->urows, cap, offs, (fsx_unit *)g[P_UNITS], tail, grp, 0);
+    if (scan) hipLaunchKernelGGL(k_unit_scan, dim3(1), dim3(1024), 0, s, grp, nzb);
+    hipLaunchKernelGGL(k_units<1>, dim3(nblk(nzb, 4)), dim3(256), 0, s, (const int *)counts, nzb, p->nb, zn, ng,
+                       p->urows, cap, offs, (fsx_unit *)g[P_UNITS], tail, grp, scan);
     hipLaunchKernelGGL(k_scatter, dim3(nblk(n, 256)), dim3(256), 0, s, (const int *)g[P_KEYS],
                        (const int2 *)g[P_INFO], n, ng, (const int *)offs, counts + nkeys,
                        (int4 *)g[P_RECS]);

@@ -10,6 +10,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SRC = r"""
 #include "fsx_rules.h"
 int cross_pw(int mixed, int ns) { return fsx_cross_pw(mixed, ns); }
+int unit_scan(long groups) { return fsx_unit_scan(groups); }
 """
 
 
@@ -33,3 +34,10 @@ def test_two_poses_per_wavefront_at_small_orders(rules):
         assert rules.cross_pw(1, ns) == 2 and rules.cross_pw(0, ns) == 2, L
     assert rules.cross_pw(1, 128) == 1 and rules.cross_pw(0, 128) == 2
     assert rules.cross_pw(1, 176) == 1 and rules.cross_pw(0, 176) == 1
+
+
+def test_group_sums_of_their_own_for_many_groups(rules):
+    """Summed by every wavefront they cost the square of the number of groups."""
+    rules.unit_scan.argtypes = [C.c_long]
+    assert not rules.unit_scan(1) and not rules.unit_scan(684)
+    assert rules.unit_scan(3737) and rules.unit_scan(2 ** 30)
