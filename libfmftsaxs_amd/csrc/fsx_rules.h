@@ -20,6 +20,19 @@ static inline int fsx_cross_pw(int mixed, int ns)
     return ns <= (mixed ? 96 : 128) ? 2 : 1;
 }
 
+/* Lanes per fit of the mixed form's lane-group fit: about 16 q per lane, at least
+ * four lanes.  They set the order of the sums over q, so they depend on nothing else.
+ * Fit stage, averages of four problems: 31 q, 2,000 fits 0.17 ms with two lanes, 0.12
+ * with four; 40,000 0.29 and 0.23, 210,000 0.54 and 0.47 (21 q 0.37 and 0.42); 41 q,
+ * 2,000 fits 0.13 with four, 0.10 with eight, 40,000 0.25 and 0.29, 210,000 0.55 and
+ * 0.65. */
+static inline int fsx_fit_lanes(int Q)
+{
+    int fpl = 4;
+    while (fpl < 64 && fpl * 16 < Q) fpl *= 2;
+    return fpl;
+}
+
 /* Whether the (z, beta2) groups' counts are summed by a launch of their own, between
  * the two passes of the bucketing, instead of by every wavefront of the second pass.
  * Bucketing stage without and with it: 341 groups 33 and 34 us, 684 45 and 45, 3,737

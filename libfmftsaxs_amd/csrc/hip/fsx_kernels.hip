@@ -1307,7 +1307,7 @@ k_fit(const double *acc, const int4 *recs, const int *nvalid_p, int Q, const dou
  * loop over q): four wavefronts per SIMD, against one for the
  * compact form's state (on the 210,000-pose L = 15 workload 1.50 ms,
  * against 1.60 ms at three wavefronts in 168 registers without spills).
- * With four lanes per fit (many fits, Q up to 64) a wavefront runs 16 fits, so the
+ * With four lanes per fit (Q up to 64) a wavefront runs 16 fits, so the
  * solver's divergent code is shared by many fits while the evaluation of
  * each is split four ways (at three wavefronts per SIMD: 1.64 ms, against
  * 1.83 ms with two lanes and 1.87 ms with eight).  The moments, q and the
@@ -1315,7 +1315,6 @@ k_fit(const double *acc, const int4 *recs, const int *nvalid_p, int Q, const dou
  * ii * fpl + j for q = j qpl + ii, so the lanes of a group read consecutive
  * doubles.  Groups take poses from a queue (next) until none is left. */
 #define FSX_FG_ARR 8     /* LDS arrays: a0..a5, q, 1 / (q_i - q_{i-1}) */
-#define FSX_FG_QLANE 16  /* q per lane the default lanes per fit aim at */
 #ifndef FSX_FG_WAVES
 #define FSX_FG_WAVES 4   /* wavefronts per SIMD (the register budget of the launch bounds) */
 #endif
@@ -2582,15 +2581,11 @@ static int plan_init(fsx_plan *p, const fsx_hip_args *A, int tile_rows, int slot
      * groups (k_fitg), or with FSX_FIT_COMPACT (or a q grid whose arrays do
      * not fit the block's LDS) the compact-form L-BFGS-B lane per fit, both
      * evaluated in one pass over q; the FP64 form: the reference's
-     * L-BFGS-B, lane per fit.  Lanes per fit of the group fit: about
-     * FSX_FG_QLANE q per lane, at least two, twice that where the lanes
-     * resident at once still take all fits (2,000 fits of 31 q 0.37 ms with 4
-     * lanes, 0.21 with 8, 0.26 with 16; 20,000 of 51 q 0.27, 0.23, 0.28;
-     * 210,000 0.60, 0.68, 0.94) (FSX_FIT_GROUP_LANES overrides), doubled until
-     * the block's LDS fits */
-    int fpl = 2;
-    while (fpl < FSX_WAVE && fpl * FSX_FG_QLANE < Q) fpl *= 2;
-    if (fpl < FSX_WAVE && 2L * fpl * n <= 256L * FSX_FG_WAVES * g_ncu) fpl *= 2;
+     * L-BFGS-B, lane per fit.  Lanes per fit of the group fit from the number
+     * of q alone (fsx_fit_lanes; FSX_FIT_GROUP_LANES overrides), doubled until
+     * the block's LDS fits: they set the order of the sums over q, and a pose's
+     * result must not depend on the length of its list */
+    int fpl = fsx_fit_lanes(Q);
     fpl = env_int("FSX_FIT_GROUP_LANES", fpl, 1, FSX_WAVE);
     while (fpl & (fpl - 1)) fpl &= fpl - 1;   /* a power of two */
     while (fpl < FSX_WAVE && fitg_lds(Q, fpl) > FSX_FIT_LDS) fpl *= 2;

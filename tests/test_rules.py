@@ -10,6 +10,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SRC = r"""
 #include "fsx_rules.h"
 int cross_pw(int mixed, int ns) { return fsx_cross_pw(mixed, ns); }
+int fit_lanes(int Q) { return fsx_fit_lanes(Q); }
 int unit_scan(long groups) { return fsx_unit_scan(groups); }
 """
 
@@ -41,3 +42,8 @@ def test_group_sums_of_their_own_for_many_groups(rules):
     rules.unit_scan.argtypes = [C.c_long]
     assert not rules.unit_scan(1) and not rules.unit_scan(684)
     assert rules.unit_scan(3737) and rules.unit_scan(2 ** 30)
+
+
+def test_lanes_per_fit(rules):
+    got = [rules.fit_lanes(Q) for Q in (2, 32, 33, 51, 64, 65, 81, 128, 129, 512, 513, 1024, 4000)]
+    assert got == [4, 4, 4, 4, 4, 8, 8, 8, 16, 32, 64, 64, 64]
