@@ -586,8 +586,12 @@ __global__ void k_count(const long long *poses, int n, int znum, int nbeta, int 
 }
 
 /* First record of every bucket and the cross-term units, one wavefront per
- * (z, beta2).  Units are cut greedily along gamma2: up to urows rows and
- * cap poses; a bucket of more poses takes several.  PASS 0 counts every
+ * (z, beta2).  Units are cut greedily along gamma2: up to urows rows, in even
+ * shares, and cap poses; a bucket of more poses takes several.  Blocks take units
+ * at a fixed stride, so that one small unit per group (the last of 25 rows cut by
+ * eights) left every fourth block with small ones only: cross terms FP32, L = 12,
+ * 25-point grids, 70,000 poses 0.86 against 0.80 ms, L = 20, 41-point grids, 400,000
+ * poses 6.10 against 5.67.  PASS 0 counts every
  * group's records and units (grp), PASS 1 adds those of the groups before and
  * writes; tail: records, non-empty buckets, units.
  * The records, and with them the fits, are in the order of (z, beta2): the poses of
@@ -634,8 +638,13 @@ k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int cap, 
     u.b2 = b2;
     u.z = z;
     u.pad = 0;
+    /* non-empty buckets left, and rows of the open unit at most: the same number of
+     * units in even shares (25 rows as 7, 6, 6, 6, not 8, 8, 8, 1) */
+    const int v0 = lane < ng ? c[lane] : 0;
+    int rem = __popcll(__ballot(v0 > 0)), lim = 0;
+    for (int g0 = 64; g0 < ng; g0 += 64) rem += __popcll(__ballot(g0 + lane < ng && c[g0 + lane] > 0));
     for (int g0 = 0; g0 < ng; g0 += 64) {
-        const int v = g0 + lane < ng ? c[g0 + lane] : 0;
+        const int v = g0 == 0 ? v0 : g0 + lane < ng ? c[g0 + lane] : 0;
         if (PASS) {
             /* exclusive scan over the 64 buckets */
             int x = v;
@@ -654,7 +663,7 @@ k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int cap, 
             int left = __builtin_amdgcn_readlane(v, b);
             while (left > 0) {
                 /* close the open unit where the row does not fit in it */
-                if (un > 0 && (ur == urows || un + left > cap)) {
+                if (un > 0 && (ur == lim || un + left > cap)) {
                     if (PASS && lane == 0) {
                         u.n = un;
                         u.nrow = ur;
@@ -663,6 +672,7 @@ k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int cap, 
                     uc++;
                     un = ur = 0;
                 }
+                if (un == 0) lim = (int)ceilf((float)rem / ceilf((float)rem / (float)urows));
                 const int k = left < cap - un ? left : cap - un;
                 if (PASS) {
                     if (un == 0) u.p0 = total + p;
@@ -681,6 +691,7 @@ k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int cap, 
                 p += k;
                 left -= k;
             }
+            rem--;
         }
     }
     if (un > 0) {
