@@ -20,6 +20,32 @@ static inline int fsx_cross_pw(int mixed, int ns)
     return ns <= (mixed ? 96 : 128) ? 2 : 1;
 }
 
+/* Most cross-term blocks per CU; rows3: gamma2 rows per unit that the LDS leaves with
+ * three; ns, pw: slots of the largest chunk and poses per wavefront; nrows: receptor
+ * rows of a q; per_bucket: poses per (z, beta2, gamma2).
+ * FP32: five; more only take each other's cache lines (300,000 poses at L = 25 98,
+ * 76, 66.2, 65.6 and 73.7 ms with 2 to 6 blocks; 210,000 at L = 15 5.63, 4.64, 4.40,
+ * 4.46 and 4.64).
+ * FP64: as many as fit, three or four, but the receptor rows in flight (four
+ * wavefronts of pw rows per block) take up the XCD's 4 MB of L2 themselves: 4.7 MB
+ * with three blocks at L = 15, two poses per wavefront.  Two blocks
+ *  - where three leave four rows per unit (from 172 slots on): two leave six or
+ *    eight.  Cross terms, against three blocks: L = 18 (181 slots) 0.88 times with
+ *    0.4 poses per bucket, 0.85 with 2, 0.86 with 6, 0.90 with 15; L = 20 (221) 1.02,
+ *    0.99, 0.95, 0.92; L = 28 (217) 1.03, 1.00, 0.98, 0.95;
+ *  - where the receptor rows of a q are 6 MB or more and the buckets so full that the
+ *    pairing outweighs the translation.  64 x 19 grid, 6, 9 and 15 poses per bucket: L
+ *    = 14 1.03, 0.96 and 0.90 times, L = 15 1.03, 0.94, 0.89 (two poses per
+ *    wavefront), L = 17 0.97, 0.97, 0.95, L = 25 0.98, 1.00, 0.95 (one); 128 x 37 grid,
+ *    L = 25, 5.2 per bucket 0.93, 2.5 1.06.  Tables of 4 MB (L = 15, 36 x 19) 1.12, 1.05,
+ *    0.98. */
+static inline int fsx_cross_blocks(int mixed, int rows3, int ns, int pw, long nrows, double per_bucket)
+{
+    if (mixed) return 5;
+    if (rows3 <= 4) return per_bucket >= (ns <= 200 ? 0 : 4) ? 2 : 5;
+    return 48.0 * ns * (double)nrows >= 6e6 && per_bucket >= (pw == 2 ? 8 : 5) ? 2 : 5;
+}
+
 /* Lanes per fit of the mixed form's lane-group fit: about 16 q per lane, at least
  * four lanes.  They set the order of the sums over q, so they depend on nothing else.
  * Fit stage, averages of four problems: 31 q, 2,000 fits 0.17 ms with two lanes, 0.12

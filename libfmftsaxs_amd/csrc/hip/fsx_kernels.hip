@@ -2116,18 +2116,16 @@ static size_t cross_lds_of(int mixed, int ns, int urows)
 {
     return mixed ? cross_lds<float>(ns, urows) : cross_lds<double>(ns, urows);
 }
-/* blocks of a cross-term launch: those resident at once, up to five per CU
- * (FSX_CROSS_BLOCKS_PER_CU overrides the per-CU count).  More only take each
- * other's cache lines: FP32 tables, 300,000 poses at L = 25, 98, 76, 66.2, 65.6 and
- * 73.7 ms with 2 to 6 blocks; 210,000 at L = 15 5.63, 4.64, 4.40, 4.46 and 4.64. */
-static long cross_grid(const void *kern, size_t lds)
+/* blocks of a cross-term launch: those resident at once, up to most per CU
+ * (fsx_cross_blocks; FSX_CROSS_BLOCKS_PER_CU overrides the per-CU count) */
+static long cross_grid(const void *kern, size_t lds, int most)
 {
     int per = env_int("FSX_CROSS_BLOCKS_PER_CU", 0, 0, 16);
     if (per == 0) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, FSX_CROSS_BLOCK, lds) != hipSuccess ||
             per < 1)
             per = 1;
-        per = per > 5 ? 5 : per;
+        per = per > most ? most : per;
     }
     return (long)g_ncu * per;
 }
@@ -2145,6 +2143,7 @@ struct fsx_cross_group {
     int mixed, jn, pw, chunk;   /* the kernel and the m-chunk index */
     size_t lds;                 /* the largest job's LDS */
     int njobs, cap;
+    int most;                   /* most blocks per CU any job takes */
     long grid;                  /* blocks of the launch */
     fsx_cross_job *jobs;
 };
@@ -2239,6 +2238,7 @@ struct fsx_plan {
     fsx_hip_args A;
     int L, K, K2, N, Q, n, nb, na, ng, zn, nrows, mixed, half, mlo, npk, C, Tn, ne, dev_out;
     int urows;           /* gamma2 rows per cross-term unit */
+    int xblocks;         /* most cross-term blocks per CU */
     int mirror, nbr;     /* tables of beta <= pi / 2 only (fsx_mirror); their betas */
     long nkeys;
     size_t dsz, spf, es, nent;
@@ -2493,25 +2493,24 @@ static int plan_init(fsx_plan *p, const fsx_hip_args *A, int tile_rows, int slot
         plan_free_host(p);
         return FSX_ERR_ARG;
     }
+    const long rows_all = p->nrows;
     p->nrows = p->nbr * ng;
     p->C = C;
     p->ne = ne;
     plan_entries(p, chunk);
     free(chunk);
+    /* rows per unit: as many as the LDS leaves room for with three blocks to a CU,
+     * or two where more are not wanted: a unit's fixed cost is shared by more poses,
+     * but a CU needs its blocks to cover the receptor rows' latency */
+    auto rows_of = [&](int blocks) {
+        int r = FSX_UROWS;
+        while (r > 2 && blocks * ((cross_lds_of(p->mixed, nsmax, r) + 2047) / 2048) > 80) r -= 2;
+        return r;
+    };
+    p->xblocks = fsx_cross_blocks(p->mixed, rows_of(3), nsmax, cross_pw(p->mixed, nsmax), rows_all,
+                                  (double)n / (double)p->nkeys);
     p->urows = 2 * (tile_rows > 0 ? tile_rows : env_int("FSX_CROSS_ROWS", 0, 0, 4));
-    if (p->urows == 0) {
-        /* as many rows as three blocks' LDS leaves room for: a unit's fixed cost
-         * is shared by more poses, but a CU needs three blocks to cover the
-         * receptor rows' latency (FP64, L = 15, 210,000 poses: 9.5 ms with 6
-         * rows, 12.6 ms with 8 and two blocks, 12.6 ms with 4) */
-        int nsm = 0;
-        for (int c = 0; c < C; c++) {
-            const int ns = p->ent[FSX_E_RSR(p) + c] / 6;
-            if (ns > nsm) nsm = ns;
-        }
-        p->urows = FSX_UROWS;
-        while (p->urows > 2 && 3 * ((cross_lds_of(p->mixed, nsm, p->urows) + 2047) / 2048) > 80) p->urows -= 2;
-    }
+    if (p->urows == 0) p->urows = rows_of(p->xblocks < 3 ? p->xblocks : 3);
     /* twiddle e^{-i m a2 2pi/na} per (a2, m): the same table entries the
      * reference's exact transform uses, gathered by (m a2) mod na */
     for (int a2 = 0; a2 < na; a2++)
@@ -2939,7 +2938,7 @@ static int plan_enqueue(fsx_plan *p, hipStream_t s, hipEvent_t *ev, int stages =
         const void *kern = cross_kernel_of(p->mixed, cross_jn(ns, pw), pw, 0);
         const size_t lds = cross_lds_of(p->mixed, ns, p->urows);
         /* no more blocks than (q, unit) items can be */
-        long grid = cross_grid(kern, lds);
+        long grid = cross_grid(kern, lds, p->xblocks);
         if (grid > (long)n * Q) grid = ((long)n * Q + g_nxcd - 1) / g_nxcd * g_nxcd;
         fsx_cross_job jb = cross_job(p, c, grid);
         void *args[1] = {&jb};
@@ -3372,6 +3371,7 @@ static int plan_cross_collect(const fsx_plan *p, fsx_cross_group **gr, int *ngr)
             t->cap = cap;
         }
         if (lds > t->lds) t->lds = lds;
+        if (p->xblocks > t->most) t->most = p->xblocks;
         t->jobs[t->njobs++] = cross_job(p, c, 1);
     }
     return FSX_OK;
@@ -3490,7 +3490,7 @@ static int run_batch_locked(int nprob, const fsx_hip_args *args, fsx_stats *st)
         size_t ntot = 0;
         for (int i = 0; i < ncg; i++) ntot += cg[i].njobs;
         for (int i = 0; rc == FSX_OK && i < ncg; i++) {
-            cg[i].grid = cross_grid(cross_kernel_of(cg[i].mixed, cg[i].jn, cg[i].pw, 1), cg[i].lds);
+            cg[i].grid = cross_grid(cross_kernel_of(cg[i].mixed, cg[i].jn, cg[i].pw, 1), cg[i].lds, cg[i].most);
             for (int j = 0; j < cg[i].njobs; j++) cg[i].jobs[j].nx = cross_nx(cg[i].grid);
         }
         if (rc == FSX_OK) rc = grow_dev((void **)&g_cjob_dev, &g_cjob_cap,
