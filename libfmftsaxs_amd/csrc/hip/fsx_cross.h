@@ -3,8 +3,8 @@
  * fsx_kernels.hip).
  *
  * Work item of one block: one q and one fsx_unit, a run of poses with the same
- * (z, beta2) on at most FSX_UROWS different gamma2 (the poses are sorted by
- * (z, beta2, gamma2), so a unit is a range of the sorted records).  The block
+ * (z, beta2) on at most FSX_UROWS different gamma2 (the poses are sorted by z, beta2
+ * and gamma2, so a unit is a range of the sorted records).  The block
  *   1. translates the unit's ligand rows on the matrix cores,
  *        U^Y_lm(row) = sum_{l1 >= |m|} tau^{|m|}_{l l1}(q z) B^Y_{l1 m}(row),
  *      per m one matrix product with 16 rows (ligand row, re/im) for each of Y

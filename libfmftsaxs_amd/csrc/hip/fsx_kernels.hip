@@ -9,7 +9,7 @@
  *                 ligand    B^Y_lm(b2,g2,q) = sum_m2 e^{-i m2 g2} d^l_{m m2}(b2) conj(B^Y_{l m2})
  *                 (the beta/gamma factors of compute_sum1/compute_sum2 and of the
  *                 3-D DFT, fftsaxs.c:251-333, 416-524, 680, folded per pose axis)
- *   k_count/k_units/k_scatter  bucket poses by (z, beta2, gamma2), units of buckets
+ *   k_count/k_units/k_scatter  bucket poses by z, beta2 and gamma2, units of buckets
  *   k_cross       per unit and q (fsx_cross.h): U^Y_lm = sum_l1 conj(T_{|m| l l1}) B^Y_{l1 m} in LDS,
  *                 then per pose 2 Re sum_lm e^{-i m a2} (R^X U^Y [+ R^Y U^X]) for the six
  *                 cross terms VV,VD,VW,DD,DW,WW (fill_var, fftsaxs.c:87-108)
@@ -566,16 +566,20 @@ __device__ __forceinline__ void fsx_mirror(int nbeta, int na, int ng, int *b1, i
     *alpha = 2 * *alpha + m1;
 }
 
-/* bucket (z, beta2, gamma2) of each pose, its receptor row and twiddle
- * row */
+/* bucket of each pose, (z, beta2, gamma2) or, zmajor 0, (beta2, z, gamma2), its
+ * receptor row and twiddle row */
 __global__ void k_count(const long long *poses, int n, int znum, int nbeta, int na, int ng,
-                        int mirror, int *keys, int2 *info, int *counts)
+                        int mirror, int zmajor, int *keys, int2 *info, int *counts)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     int row, alpha;
     int key = fsx_pose_key(poses[i], znum, nbeta, na, ng, &row, &alpha);
     if (key >= 0) {
+        if (!zmajor) {
+            const int zb = key / ng, z = zb / nbeta;
+            key += ((zb - z * nbeta) * znum + z - zb) * ng;
+        }
         int b1 = row / ng, g1 = row - b1 * ng;
         if (mirror) fsx_mirror(nbeta, na, ng, &b1, &g1, &alpha);
         row = b1 * ng + g1;
@@ -594,12 +598,14 @@ __global__ void k_count(const long long *poses, int n, int znum, int nbeta, int 
  * poses 6.10 against 5.67.  PASS 0 counts every
  * group's records and units (grp), PASS 1 adds those of the groups before and
  * writes; tail: records, non-empty buckets, units.
- * The records, and with them the fits, are in the order of (z, beta2): the poses of
- * one z take about the same number of evaluations, and the long ones don't come
- * last (in the order of (beta2, z) the fits of 210,000 poses, L = 10, 41 q took 1.05
- * against 0.67 ms in the mixed form and 1.53 against 1.27 in FP64, L = 12 1.13
- * against 0.73 and 1.69 against 1.35; 20,000 poses within 0.1 ms either way).
- * The units are in the order of (beta2, z): in the order of the records, or with ranges
+ * The records, and with them the fits, are in the order of the groups.  Lists of more
+ * fits than start at once have them by (z, beta2) (zmajor): the poses of one z take
+ * about the same number of evaluations, and the long ones don't come last (by (beta2,
+ * z) the fits of 210,000 poses, L = 10, 41 q took 1.05 against 0.67 ms in the mixed form
+ * and 1.53 against 1.27 in FP64, L = 12 1.13 against 0.73 and 1.69 against 1.35).
+ * Shorter ones by (beta2, z), which spreads the long fits over the wavefronts (2,000
+ * poses, L = 10, 31 q 0.35 against 0.38 ms mixed, 0.31 against 0.32 FP64).
+ * The units are in the order of (beta2, z): by (z, beta2), or with ranges
  * reserved by atomics, an XCD's blocks work on all beta2 at a time and its L2 loses
  * the ligand rows (cross terms FP64 L = 15, 210,000 poses 9.76 against 9.27 ms; L =
  * 25, 200,000 poses 156 against 146, FP32 300,000 poses 65.5 against 61.7).
@@ -608,15 +614,15 @@ __global__ void k_count(const long long *poses, int n, int znum, int nbeta, int 
 template <int PASS>
 __global__ void __launch_bounds__(256)
 k_units(const int *counts, int nzb, int nb, int zn, int ng, int urows, int cap, int *offs,
-        fsx_unit *units, int *tail, int2 *grp, int scanned)
+        fsx_unit *units, int *tail, int2 *grp, int scanned, int zmajor)
 {
     const int zb = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (zb >= nzb) return;
     const int *c = counts + (size_t)zb * ng;
-    const int z = zb / nb, b2 = zb - z * nb;
+    const int z = zmajor ? zb / nb : zb % zn, b2 = zmajor ? zb % nb : zb / zn;
     int total = 0, first = 0;
     if (PASS) {
-        /* records by (z, beta2), units by (beta2, z) */
+        /* records in the order of the buckets, units by (beta2, z) */
         const int ub = b2 * zn + z;
         if (scanned) {
             total = grp[zb].x;
@@ -2239,6 +2245,8 @@ struct fsx_plan {
     int L, K, K2, N, Q, n, nb, na, ng, zn, nrows, mixed, half, mlo, npk, C, Tn, ne, dev_out;
     int urows;           /* gamma2 rows per cross-term unit */
     int xblocks;         /* most cross-term blocks per CU */
+    int zmajor;          /* more fits than start at once: records sorted by (z, beta2),
+                            else by (beta2, z) (k_units) */
     int mirror, nbr;     /* tables of beta <= pi / 2 only (fsx_mirror); their betas */
     long nkeys;
     size_t dsz, spf, es, nent;
@@ -2561,7 +2569,7 @@ static int plan_init(fsx_plan *p, const fsx_hip_args *A, int tile_rows, int slot
     z[P_KEYS] = sizeof(int) * n;
     z[P_INFO] = sizeof(int2) * n;
     z[P_COUNTS] = sizeof(int) * 2 * p->nkeys;   /* counts, then fills */
-    /* then records, buckets, units; then those of each (z, beta2), (beta2, z) */
+    /* then records, buckets, units; then records and units per (z, beta2) group */
     z[P_OFFS] = sizeof(int) * (p->nkeys + 4) + sizeof(int2) * (size_t)nb * zn;
     z[P_UNITS] = sizeof(fsx_unit) * (size_t)n;
     z[P_RECS] = sizeof(int4) * n;
@@ -2616,6 +2624,7 @@ static int plan_init(fsx_plan *p, const fsx_hip_args *A, int tile_rows, int slot
         p->lanes = (long)g_ncu * 256 * bpc;
         if (p->lanes > (long)n * fpl) p->lanes = ((long)n * fpl + 255) / 256 * 256;
         p->fit_next0 = p->lanes / fpl;
+        p->zmajor = n > p->fit_next0;
         return FSX_OK;
     }
     int fit_bpc = env_int("FSX_FIT_BLOCKS_PER_CU", 0, 0, 16);
@@ -2634,6 +2643,7 @@ static int plan_init(fsx_plan *p, const fsx_hip_args *A, int tile_rows, int slot
     if (p->fit_fpw < 1) p->fit_fpw = 1;
     if (p->lanes > n) p->lanes = ((long)(n + p->fit_fpw - 1) / p->fit_fpw * FSX_WAVE + 255) / 256 * 256;
     p->fit_next0 = p->lanes / FSX_WAVE * p->fit_fpw;
+    p->zmajor = n > p->fit_next0;
     return FSX_OK;
 }
 
@@ -2906,11 +2916,11 @@ static int plan_enqueue(fsx_plan *p, hipStream_t s, hipEvent_t *ev, int stages =
     }
     HIPR(hipGetLastError());
     if (ev) HIPR(hipEventRecord(ev[2], s));
-    /* poses sorted by (z, beta2, gamma2), and the cross-term units */
+    /* poses sorted by z, beta2 and gamma2, and the cross-term units */
     hipLaunchKernelGGL(k_init, dim3(nblk(2 * nkeys, 256)), dim3(256), 0, s, counts, 2 * nkeys, tail,
                        (int *)g[P_NEXT], (int)p->fit_next0, (unsigned long long *)g[P_TALLY]);
     hipLaunchKernelGGL(k_count, dim3(nblk(n, 256)), dim3(256), 0, s, p->dposes, n, zn, p->nb, p->na,
-                       ng, p->mirror, (int *)g[P_KEYS], (int2 *)g[P_INFO], counts);
+                       ng, p->mirror, p->zmajor, (int *)g[P_KEYS], (int2 *)g[P_INFO], counts);
     int2 *grp = (int2 *)(offs + ((nkeys + 4) & ~1L));
     /* most poses of a unit: where the buckets are crowded, 64 leave most of a unit's
      * rows unused (1,000,000 poses FP64 L = 15: cross terms 34.6 against 30.4 ms); fewer
@@ -2920,10 +2930,10 @@ static int plan_enqueue(fsx_plan *p, hipStream_t s, hipEvent_t *ev, int stages =
                           : (long)n * Q / items < 64 ? 64 : (long)n * Q / items);
     const int nzb = p->nb * zn, scan = fsx_unit_scan(nzb);
     hipLaunchKernelGGL(k_units<0>, dim3(nblk(nzb, 4)), dim3(256), 0, s, (const int *)counts, nzb, p->nb, zn, ng,
-                       p->urows, cap, offs, (fsx_unit *)g[P_UNITS], tail, grp, 0);
+                       p->urows, cap, offs, (fsx_unit *)g[P_UNITS], tail, grp, 0, p->zmajor);
     if (scan) hipLaunchKernelGGL(k_unit_scan, dim3(1), dim3(1024), 0, s, grp, nzb);
     hipLaunchKernelGGL(k_units<1>, dim3(nblk(nzb, 4)), dim3(256), 0, s, (const int *)counts, nzb, p->nb, zn, ng,
-                       p->urows, cap, offs, (fsx_unit *)g[P_UNITS], tail, grp, scan);
+                       p->urows, cap, offs, (fsx_unit *)g[P_UNITS], tail, grp, scan, p->zmajor);
     hipLaunchKernelGGL(k_scatter, dim3(nblk(n, 256)), dim3(256), 0, s, (const int *)g[P_KEYS],
                        (const int2 *)g[P_INFO], n, ng, (const int *)offs, counts + nkeys,
                        (int4 *)g[P_RECS]);

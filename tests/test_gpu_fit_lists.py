@@ -37,3 +37,22 @@ def test_long_list_equals_short_lists(F, Q, n, mixed):
         s = F.score(gp, idx[k0:k0 + m], mixed=mixed)
         for k in ("score", "c1", "c2"):
             assert np.array_equal(r[k][k0:k0 + m], s[k], equal_nan=True), (k, k0, m)
+
+
+def test_both_orders_of_the_records(F):
+    """One pose more than start at once: the records are then sorted by (z, beta2)
+    instead of (beta2, z).  A list on either side, poses of all z and beta2."""
+    nb, na, ng, Q = 4, 9, 8, 12
+    pb = build_problem(200, 150, 4, 0.4, Q, np.linspace(21.0, 33.0, 70), 20, seed=179, nbeta=nb,
+                       na=na, ng=ng)
+    rng = np.random.default_rng(180)
+    gp = _gpu_problem(F, pb)
+    total = 70 * nb * nb * na * ng * ng
+    idx = rng.choice(total, size=min(total, 120000), replace=False).astype(np.int64)
+    print(f"{idx.size} poses", flush=True)
+    for mixed in (False, True):
+        r = F.score(gp, idx, mixed=mixed)
+        s = F.score(gp, idx[:30000], want_cross=True, mixed=mixed)
+        assert not np.isnan(s["cross"]).any()
+        for k in ("score", "c1", "c2"):
+            assert np.array_equal(r[k][:30000], s[k], equal_nan=True), k
