@@ -3224,8 +3224,10 @@ static int get_bat(int i, size_t bytes, void *ctx, void **out)
  * Per expansion-order bucket (L <= 10, 15, 20, 25, 30, 40) and form, the
  * pairs of gamma2 rows per unit with the shortest cross-term stage on the first
  * complex of that bucket; FSX_TUNE_FILE names a text file the table is
- * read from and appended to ("bucket mixed rows slots ms" lines, slots 0:
- * the form's default pairing-slot cap). */
+ * read from and appended to ("bucket mixed rows slots ms pairs" lines, slots 0:
+ * the form's default pairing-slot cap).  Lines without the last word are of
+ * versions whose rows meant single rows of another kernel: they are passed over,
+ * and their buckets tuned again. */
 #define FSX_TUNE_BUCKETS 6
 static int g_tune[FSX_TUNE_BUCKETS][2][2];   /* rows, slots; 0: not tuned */
 static int g_tune_loaded = 0;
@@ -3270,8 +3272,10 @@ static void tune_load(void)
     if (!f) return;
     int b, m, r, c;
     double ms;
-    while (fscanf(f, "%d %d %d %d %lf", &b, &m, &r, &c, &ms) == 5)
-        if (b >= 0 && b < FSX_TUNE_BUCKETS && m >= 0 && m <= 1 && r >= 1 && r <= 4 &&
+    char line[128], tag[8];
+    while (fgets(line, sizeof(line), f))
+        if (sscanf(line, "%d %d %d %d %lf %7s", &b, &m, &r, &c, &ms, tag) == 6 &&
+            strcmp(tag, "pairs") == 0 && b >= 0 && b < FSX_TUNE_BUCKETS && m >= 0 && m <= 1 && r >= 1 && r <= 4 &&
             (c == 0 || (c >= 64 && c <= 4 * FSX_WAVE))) {
             g_tune[b][m][0] = r;
             g_tune[b][m][1] = c;
@@ -3285,7 +3289,7 @@ static void tune_save(int b, int m, int r, int c, double ms)
     if (!path || !*path) return;
     FILE *f = fopen(path, "a");
     if (!f) return;
-    fprintf(f, "%d %d %d %d %.4f\n", b, m, r, c, ms);
+    fprintf(f, "%d %d %d %d %.4f pairs\n", b, m, r, c, ms);
     fclose(f);
 }
 
