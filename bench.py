@@ -254,8 +254,28 @@ def w_alg(poses, L, Q, nb, ng):
     return 24.0 * Q * C1 * zb2 + 72.0 * Q * C2 * slabs
 
 
+def cross_roofline(flops, nbytes, ms, traffic, mixed):
+    """Roofline entry of k_cross: vector (VALU) arithmetic on operands held in LDS and
+    registers, against the VALU peak of its type, 78.6 TFLOP/s for FP64 and for FP32
+    as built here (packed FP32 is disabled, so FP32 issues at the FP64 rate).  traffic:
+    the measured bytes behind the L2 per launch (None: not measured).  They are given
+    as a rate and never as a share of the HBM peak: the Infinity Cache serves most of
+    them, and they rise when the L2 is used worse."""
+    peak = 78.6
+    achieved = flops / (ms * 1e-3) / 1e12
+    r = {"kernel": "k_cross", "bound": "valu", "achieved": achieved, "peak": peak,
+         "peak_basis": "VALU FMA rate, FP64 and non-packed FP32", "unit": "TFLOP/s",
+         "frac": achieved / peak, "traffic": traffic, "ms_per_launch": ms,
+         "algorithmic_flops": flops, "algorithmic_bytes": nbytes,
+         "arith": "f32" if mixed else "f64"}
+    if traffic:
+        r["traffic_gbs"] = traffic / (ms * 1e-3) / 1e9
+        r["traffic_note"] = "bytes behind L2, most of them served by the Infinity Cache"
+    return r
+
+
 def load_traffic(workload):
-    """HBM bytes per launch of the main kernels on this workload, from the
+    """Bytes behind the L2 per launch of the main kernels on this workload, from the
     committed rocprofv3 --pmc summary of the same workload (FETCH_SIZE and
     WRITE_SIZE scaled by what they read for a plain copy of known size); {}
     when no summary of this workload is committed."""
@@ -373,36 +393,10 @@ def main():
         cf = float(np.mean([s["cross_flops"] for s in stats]))
         # Roofline of the two main kernels; the stage times come from HIP
         # events the library records on the stream its kernels run on.  The
-        # cross-term kernel is vector (VALU) arithmetic on operands held in
-        # LDS and registers: its roof is the VALU peak of its type, 78.6
-        # TFLOP/s for FP64 and for FP32 as built here (packed FP32 is
-        # disabled, so FP32 issues at the FP64 rate).  The fit stream is
-        # priced against HBM (its profile read once, three results written).
-        peak = 78.6
-        achieved = cf / (avg["ms_cross"] * 1e-3) / 1e12
-        tr = traffic.get("k_cross_" + ("f32" if mixed else "f64"))
-        roof_cross = {"kernel": "k_cross", "bound": "valu", "achieved": achieved, "peak": peak,
-                      "peak_basis": "VALU FMA rate, FP64 and non-packed FP32",
-                      "unit": "TFLOP/s", "frac": achieved / peak, "traffic": tr,
-                      "ms_per_launch": avg["ms_cross"], "algorithmic_flops": cf,
-                      "algorithmic_bytes": cb, "arith": "f32" if mixed else "f64"}
-        if tr:
-            # the measured HBM bytes per launch as a rate.  The algorithmic
-            # bytes (one receptor row per pose and q) overstate what must come
-            # from HBM wherever L2 serves repeated rows (L = 15: 40.6 GB asked,
-            # 15.7 GB fetched), so HBM is taken as the binding roof only when
-            # the measured rate is clearly nearer its peak than the flops are
-            # to theirs (receptor rows that no longer fit L2, e.g. L = 25), and
-            # then priced with the smaller of the two byte counts: bytes the
-            # caches served never count as HBM throughput
-            rate = tr / (avg["ms_cross"] * 1e-3) / 1e9
-            roof_cross["traffic_gbs"] = rate
-            roof_cross["traffic_frac"] = rate / 8000.0
-            if rate / 8000.0 > 1.25 * roof_cross["frac"]:
-                ab = min(cb, tr) / (avg["ms_cross"] * 1e-3) / 1e9
-                roof_cross.update({"bound": "hbm", "achieved": ab, "peak": 8000.0,
-                                   "peak_basis": "HBM3E", "unit": "GB/s", "frac": ab / 8000.0,
-                                   "valu_tflops": achieved, "valu_frac": achieved / peak})
+        # fit stream is priced against HBM (its profile read once, three
+        # results written).
+        roof_cross = cross_roofline(cf, cb, avg["ms_cross"],
+                                    traffic.get("k_cross_" + ("f32" if mixed else "f64")), mixed)
         # each pose's six rescaled profile terms read once (FP32 in the mixed
         # form's lane-group fit, FP64 otherwise) and score, c1, c2 written
         fb = n * (6 * pb.qnum * (4 if mixed else 8) + 24)
