@@ -46,16 +46,17 @@ static inline int fsx_cross_blocks(int mixed, int rows3, int ns, int pw, long nr
     return 48.0 * ns * (double)nrows >= 6e6 && per_bucket >= (pw == 2 ? 8 : 5) ? 2 : 5;
 }
 
-/* Lanes per fit of the mixed form's lane-group fit: about 16 q per lane, at least
- * four lanes.  They set the order of the sums over q, so they depend on nothing else.
- * Fit stage, averages of four problems: 31 q, 2,000 fits 0.17 ms with two lanes, 0.12
- * with four; 40,000 0.29 and 0.23, 210,000 0.54 and 0.47 (21 q 0.37 and 0.42); 41 q,
- * 2,000 fits 0.13 with four, 0.10 with eight, 40,000 0.25 and 0.29, 210,000 0.55 and
- * 0.65. */
+/* Lanes per fit of the mixed form's lane-group fit: up to 8 q per lane, at least four
+ * lanes.  They set the order of the sums over q, so they depend on nothing else.
+ * The longest fit, a chain of dependent evaluations, sets the time of all but the
+ * longest lists.  Fit stage, averages over L = 8, 10, 12, 15, with half as many lanes
+ * and with these: 31 q (4 lanes) 2,000 fits 0.17 and 0.12 ms, 210,000 0.54 and 0.47;
+ * 51 q (8) 60,000 0.57 and 0.48, 150,000 0.80 and 0.76, but 210,000 of one box 0.57 and
+ * 0.67; 81 q (16) 2,000 0.24 and 0.20, 20,000 0.47 and 0.38, 150,000 0.96 and 1.14. */
 static inline int fsx_fit_lanes(int Q)
 {
     int fpl = 4;
-    while (fpl < 64 && fpl * 16 < Q) fpl *= 2;
+    while (fpl < 64 && fpl * 8 < Q) fpl *= 2;
     return fpl;
 }
 

@@ -1324,11 +1324,10 @@ k_fit(const double *acc, const int4 *recs, const int *nvalid_p, int Q, const dou
  * loop over q): four wavefronts per SIMD, against one for the
  * compact form's state (on the 210,000-pose L = 15 workload 1.50 ms,
  * against 1.60 ms at three wavefronts in 168 registers without spills).
- * With four lanes per fit (Q up to 64) a wavefront runs 16 fits, so the
- * solver's divergent code is shared by many fits while the evaluation of
- * each is split four ways (at three wavefronts per SIMD: 1.64 ms, against
- * 1.83 ms with two lanes and 1.87 ms with eight).  The moments, q and the
- * step reciprocals sit in LDS, slot
+ * With eight lanes per fit (33 to 64 q, fsx_fit_lanes) a wavefront runs 8 fits, so
+ * the solver's divergent code is shared by several fits while the evaluation of
+ * each, whose chain bounds all but the longest lists, is split eight ways.  The
+ * moments, q and the step reciprocals sit in LDS, slot
  * ii * fpl + j for q = j qpl + ii, so the lanes of a group read consecutive
  * doubles.  Groups take poses from a queue (next) until none is left. */
 #define FSX_FG_ARR 8     /* LDS arrays: a0..a5, q, 1 / (q_i - q_{i-1}) */

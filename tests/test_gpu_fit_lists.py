@@ -1,7 +1,7 @@
 """A pose's result does not depend on the length of its list: score, c1 and c2 of a
 long list (more fits than the device runs at once) are bit for bit those of its
-poses scored in lists of 1, 700 and 5,000, in both forms, with few q (four lanes per
-fit in the mixed form), and with 70 q (eight)."""
+poses scored in lists of 1, 700 and 5,000, in both forms, with 2, 25, 41 and 70 q (four,
+eight and sixteen lanes per fit in the mixed form; more lanes than q among them)."""
 import numpy as np
 import pytest
 

@@ -50,7 +50,7 @@ def test_group_sums_of_their_own_for_many_groups(rules):
 
 def test_lanes_per_fit(rules):
     got = [rules.fit_lanes(Q) for Q in (2, 32, 33, 51, 64, 65, 81, 128, 129, 512, 513, 1024, 4000)]
-    assert got == [4, 4, 4, 4, 4, 8, 8, 8, 16, 32, 64, 64, 64]
+    assert got == [4, 4, 8, 8, 8, 16, 16, 16, 32, 64, 64, 64, 64]
 
 
 def test_blocks_of_crowded_fp64_lists(rules):
