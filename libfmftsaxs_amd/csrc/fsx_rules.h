@@ -30,9 +30,10 @@ static inline int fsx_cross_pw(int mixed, int ns)
  * wavefronts of pw rows per block) take up the XCD's 4 MB of L2 themselves: 4.7 MB
  * with three blocks at L = 15, two poses per wavefront.  Two blocks
  *  - where three leave four rows per unit (from 172 slots on): two leave six or
- *    eight.  Cross terms, against three blocks: L = 18 (181 slots) 0.88 times with
- *    0.4 poses per bucket, 0.85 with 2, 0.86 with 6, 0.90 with 15; L = 20 (221) 1.02,
- *    0.99, 0.95, 0.92; L = 28 (217) 1.03, 1.00, 0.98, 0.95;
+ *    eight.  Cross terms, against three blocks: L = 18 (181 slots) 1.41 times with
+ *    0.01 poses per bucket, 1.20 with 0.1, 0.95 with 0.2, 0.88 with 0.4, 0.85 with 2,
+ *    0.86 with 6, 0.90 with 15; L = 20 (221) 1.02 with 0.4, 0.99 with 2, 0.95 with 6,
+ *    0.92 with 15; L = 28 (217) 1.03, 1.00, 0.98, 0.95;
  *  - where the receptor rows of a q are 6 MB or more and the buckets so full that the
  *    pairing outweighs the translation.  64 x 19 grid, 6, 9 and 15 poses per bucket: L
  *    = 14 1.03, 0.96 and 0.90 times, L = 15 1.03, 0.94, 0.89 (two poses per
@@ -42,7 +43,7 @@ static inline int fsx_cross_pw(int mixed, int ns)
 static inline int fsx_cross_blocks(int mixed, int rows3, int ns, int pw, long nrows, double per_bucket)
 {
     if (mixed) return 5;
-    if (rows3 <= 4) return per_bucket >= (ns <= 200 ? 0 : 4) ? 2 : 5;
+    if (rows3 <= 4) return per_bucket >= (ns <= 200 ? 0.2 : 4) ? 2 : 5;
     return 48.0 * ns * (double)nrows >= 6e6 && per_bucket >= (pw == 2 ? 8 : 5) ? 2 : 5;
 }
 

@@ -62,6 +62,7 @@ def test_blocks_of_crowded_fp64_lists(rules):
     assert f(0, 6, 171, 1, 4736, 5.23) == 2 and f(0, 6, 171, 1, 4736, 0.42) == 5
     # few rows per unit with three blocks
     assert f(0, 4, 181, 1, 703, 0.4) == 2 and f(0, 4, 221, 1, 861, 0.4) == 5
+    assert f(0, 4, 181, 1, 468, 0.009) == 5   # 95 poses: too few units for two blocks
     assert f(0, 4, 221, 1, 861, 35.0) == 2
     # small tables, FP32 tables
     assert f(0, 8, 61, 2, 231, 88.0) == 5 and f(1, 8, 128, 1, 1216, 22.8) == 5
