@@ -3122,8 +3122,14 @@ extern "C" int fsx_hip_run(const fsx_hip_args *A, fsx_stats *st)
  * HIP graph and replayed by one graph launch on later calls whose launch
  * parameters (sizes, tile shapes, scalars, buffer addresses) are all the same.
  * The cross-term tile shape per expansion-order bucket and form comes from a
- * tuner that times the candidates once on the first complex of the bucket. */
-#define FSX_BSTREAMS 4
+ * tuner that times the candidates once on the first complex of the bucket.
+ * Two streams: one complex's tables and fits run beside another's cross terms.  With
+ * four, several persistent cross-term grids share the CUs and their rows drive each
+ * other out of the L2: FP64, 64 complexes of 215,000 poses on average 1,312 ms with
+ * four streams, 1,221 with three, 1,188 with two, 1,103 with one; 7 of 14,000 to 71,000
+ * 30.8, 30.0, 26.3 and 24.8, 8 of 4,000 to 21,000 14.7, 13.9, 13.7 and 14.1; FP32 508,
+ * 498, 496 and 520 for the 64. */
+#define FSX_BSTREAMS 2
 struct fsx_bset {
     void *d[P_NBUF];
     size_t cap[P_NBUF];
@@ -3414,12 +3420,11 @@ static int run_batch_locked(int nprob, const fsx_hip_args *args, fsx_stats *st)
     /* FSX_BATCH_PERSIST=1: the persistent form, one cross-term launch per
      * (m-chunk index, kernel shape) and one fit launch over all complexes,
      * after every complex's table stages.  Default: each complex's whole
-     * pipeline on one of four streams, which on the 64-complex bench batch
-     * is faster (674 against 873 ms per mixed step): the streams overlap one
-     * complex's tables, another's cross terms and a third's fit, where the
-     * persistent form runs those stages one after another (96 ms of tables,
-     * 601 ms of cross terms, 189 ms of fits, the last with a block-level
-     * tail per complex) */
+     * pipeline on one of two streams, which on the 64-complex bench batch
+     * is faster (496 against 706 ms per mixed step, 1,200 against 1,325 in
+     * FP64): the streams overlap one complex's tables and fits with
+     * another's cross terms, where the persistent form runs those stages one
+     * after another, the fits with a block-level tail per complex */
     const int persist = env_int("FSX_BATCH_PERSIST", 0, 0, 1);
     /* the tuner first (it runs in the process-wide buffers) */
     for (int i = 0; tune && i < nprob; i++) {
