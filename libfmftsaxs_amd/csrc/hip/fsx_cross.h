@@ -3,28 +3,30 @@
  * fsx_kernels.hip).
  *
  * Work item of one block: one q and one fsx_unit, a run of poses with the same
- * (z, beta2) on at most FSX_UROWS different gamma2 (the poses are sorted by z, beta2
- * and gamma2, so a unit is a range of the sorted records).  The block
+ * (z, beta2) on at most FSX_UROWS different gamma2 (the poses are sorted by z and
+ * beta2, either of them first, and gamma2, so a unit is a range of the sorted
+ * records).  The block
  *   1. translates the unit's ligand rows on the matrix cores,
  *        U^Y_lm(row) = sum_{l1 >= |m|} tau^{|m|}_{l l1}(q z) B^Y_{l1 m}(row),
  *      per m one matrix product with 16 rows (ligand row, re/im) for each of Y
  *      = V, D, W and l in the columns, the m values dealt to the wavefronts,
  *      and puts U into LDS;
- *   2. pairs U with the receptor row of each pose (a pose per wavefront, the
- *      coefficient slots across the lanes),
+ *   2. pairs U with the receptor row of each pose (one or two poses per wavefront,
+ *      the coefficient slots across its lanes),
  *        2 Re sum_e e^{-i m a2} (R^X_e U^Y_e [+ R^Y_e U^X_e]),
  *      and writes the six sums, or adds them to those of earlier m-chunks.
- * Only rows that some pose asks for are translated.  What bounds it depends on
- * the poses per unit: with many (210,000 poses at L = 15: 38 to a unit) the
- * receptor rows, 6 KB (FP64) or 3 KB per pose and q, most of which an XCD's 4 MB
- * L2 does not hold in FP64; with few (200,000 to 300,000 on a 37 x 128 grid of 0.5 A
- * steps at L = 25: about 10) the loads and waits of an item's chain, unit, operands,
- * products, rows.  The form before it, tiles of adjacent gamma2 with all z inside
- * and the translation on the vector units, translated every row of a tile for every
- * z in use and read 100 bytes of LDS per lane for 24 multiply-adds: L = 25, 81 q,
- * 300,000 poses FP32 224 ms against 63 now, 200,000 poses FP64 219 against 145;
- * L = 15, 51 q, 210,000 poses FP32 4.7 against 4.5, FP64 9.65 against 9.3; crowded
- * buckets (1,000,000 poses) FP64 28.6 against 30.4.
+ * The products take 16 rows whether the unit has them or not (rows past nrow repeat
+ * row 0).  What bounds it depends on the poses per unit: with many (210,000 poses at
+ * L = 15: 38 to a unit) the receptor rows, 6 KB (FP64) or 3 KB per pose and q, most
+ * of which an XCD's 4 MB L2 does not hold in FP64; with few (200,000 to 300,000 on a
+ * 37 x 128 grid of 0.5 A steps at L = 25: about 10) the loads and waits of an item's
+ * chain, unit, operands, products, rows.  The form before it, tiles of adjacent
+ * gamma2 with all z inside and the translation on the vector units, translated every
+ * row of a tile for every z in use and read 100 bytes of LDS per lane for 24
+ * multiply-adds.  Cross terms of that form and of this one: L = 25, 81 q, 300,000
+ * poses FP32 224 and 64 ms, 200,000 poses FP64 219 and 143; L = 15, 51 q, 210,000
+ * poses FP32 4.7 and 4.4, FP64 9.65 and 9.15; crowded buckets FP64, 1,000,000 poses
+ * at L = 15 28.7 and 28.7, 2,500,000 at L = 25 645 and 657.
  */
 #ifndef FSX_CROSS_H
 #define FSX_CROSS_H
